@@ -28,11 +28,10 @@
 //
 // Nearest neighbours: the reference's shuffle scheme yields, for cluster i,
 // the first minimum of union areas (compared as uint32 bits) in the order
-// i+1, i-1, i+2, i-2, ..., i+R, i-R. Here every lane writes its box to LDS,
-// computes the R forward areas a(i, i+r) and stores them in LDS; lane i then
-// reads its backward areas a(i-r, i) from lane i-r's row and scans the
-// candidates in that order. Unions use IEEE minimum/maximum, so
-// a(i-r, i) == a(i, i-r) bit for bit.
+// i+1, i-1, i+2, i-2, ..., i+R, i-R. Here every lane writes its box to LDS and
+// computes the R forward areas a(i, i+r); the backward ones a(i-r, i) come from
+// lane i-r through lane shifts (nearest()). Unions use IEEE minimum/maximum,
+// so a(i-r, i) == a(i, i-r) bit for bit.
 //
 // Batched builds (many independent meshes in one launch): the sorted keys
 // are 64-bit (mesh << 30 | 30-bit Morton code) and each mesh's positions
@@ -87,7 +86,6 @@ struct HplocLds {
     uint32_t cid[64];
     uint32_t rep[64];
     uint32_t sz[64];                  // primitives in the cluster
-    uint32_t nn[64];
     // in-wave hand-over of the parent exchange
     uint32_t mlane[64];               // slot & 63 -> a lane that posted it
     uint32_t mslot[64];               // lane -> slot it exchanges at rightwards this step, or kInvalid
@@ -120,63 +118,64 @@ __device__ __forceinline__ Box lds_get_box(const HplocLds& s, uint32_t i) {
     return b;
 }
 
-// FindNearestNeighbor (BinaryBuilder.cu:127-163) without branching on
-// lanes: the same candidates in the same order as the reference (forward
-// a(i, i+r) then backward a(i-r, i), r = 1..R, first minimum wins). Every
-// forward area is computed (candidates past the group's clusters read spare
-// or stale slots); those that are not clusters of the group, or lie beyond
-// the lane's own radius R (the task's, uniform over its group), become
-// kInvalid. The loop runs to Rw, the largest radius of the wave's groups,
-// on scalar control.
-__device__ __forceinline__ uint32_t nearest_uniform(const HplocLds& s, const Box& own, uint32_t slot, uint32_t gl,
-                                                    uint32_t num, uint32_t Rw, uint32_t R) {
-    // candidates r < lim are the lane's; the winner is kept as the signed
-    // offset r or -r (0: none), so the loop does no per-lane index arithmetic.
-    // A backward candidate needs no radius test: lane i-r of the same group
-    // masked its forward area at distance r by the same radius.
-    const int lim = min((int)num - (int)gl, (int)R + 1);
-    const uint32_t lane4 = lane_id() * 4u;
-    uint32_t best = kInvalid;
-    int off = 0;
-#pragma unroll 2
-    for (uint32_t r = 1; r <= Rw; ++r) {
-        const uint32_t a = __float_as_uint(box_area(box_union(own, lds_get_box(s, slot + r))));
-        const uint32_t af = (int)r < lim ? a : kInvalid;
-        // lane - r (wrapping for lanes below r, whose value is not used)
-        uint32_t ab = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(lane4 - 4u * r), (int)af);
-        ab = gl >= r ? ab : kInvalid;
-        if (af < best) off = (int)r;
-        best = min(best, af);
-        if (ab < best) off = -(int)r;
-        best = min(best, ab);
-    }
-    return off ? (uint32_t)((int)gl + off) : kInvalid;
+// The value of the lane below (wave shift by one); lane 0 takes `first`.
+__device__ __forceinline__ uint32_t from_lane_below(uint32_t v, uint32_t first) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)v, 0x138, 0xF, 0xF, false);
 }
 
-// The same search unrolled for a radius known at compile time: constant LDS
-// and lane-shift offsets, no loop control. A scheduling barrier after each
-// candidate keeps the candidates' loads from being hoisted together (which
-// would raise the kernel's register count and cost occupancy).
+// FindNearestNeighbor (BinaryBuilder.cu:127-163) without branching on lanes:
+// the reference's choice is the first minimum of the areas in the order
+// forward a(i, i+1), backward a(i-1, i), a(i, i+2), a(i-2, i), ... Distances
+// are taken from the largest to 1. Every forward area is computed (candidates
+// past the group's clusters read spare or stale slots); those that are not
+// clusters of the group, or lie beyond the lane's own radius R (the task's,
+// uniform over its group), become kInvalid. Lane i + r receives a(i, i + r) as
+// its backward area by r shifts of one lane: the running minimum `bb` moves up
+// a lane before distance r is taken in, so a value taken in at distance r ends
+// r lanes up after the shift that follows distance 1. A valid area's target is
+// a cluster of the same group, so nothing valid crosses into the other group.
+// Taking an equal area at a smaller distance leaves each side's first minimum;
+// between the sides an equal area goes to the smaller distance, then forward.
+// The shifts are VALU moves (DPP): with each backward area fetched through LDS
+// (ds_bpermute) and scanned in the reference's order, a radius-8 search waited
+// on eight LDS round trips and took 78 registers instead of 70. With the
+// neighbour's neighbour taken from its lane as well and the stores' wait moved
+// (k_hploc), H-PLOC went 100 -> 84 us at 2,003 primitives, 612 -> 555 us at
+// 2.9M (64-lane schedule), 3250 -> 3175 us at 28.1M, and the 2,048-mesh batch
+// 2006 -> 1885 us.
+template <uint32_t UNROLL>
+__device__ __forceinline__ uint32_t nearest(const HplocLds& s, const Box& own, uint32_t slot, uint32_t gl, int lim,
+                                            uint32_t top) {
+    uint32_t bf = kInvalid, bb = kInvalid, rf = 0, rb = 0;
+#pragma unroll UNROLL
+    for (uint32_t r = top; r >= 1; --r) {
+        const uint32_t a = __float_as_uint(box_area(box_union(own, lds_get_box(s, slot + r))));
+        const uint32_t af = (int)r < lim ? a : kInvalid;
+        bb = min(from_lane_below(bb, kInvalid), af);
+        rb = from_lane_below(rb, 0u);
+        rb = bb == af ? r : rb;
+        bf = min(bf, af);
+        rf = bf == af ? r : rf;
+    }
+    bb = from_lane_below(bb, kInvalid);
+    rb = from_lane_below(rb, 0u);
+    const bool fwd = bf < bb || (bf == bb && rf <= rb);
+    const uint32_t other = fwd ? gl + rf : gl - rb;
+    return min(bf, bb) == kInvalid ? kInvalid : other;
+}
+
+// Radius known at compile time: constant LDS offsets, no loop control.
 template <uint32_t R>
 __device__ __forceinline__ uint32_t nearest_fixed(const HplocLds& s, const Box& own, uint32_t slot, uint32_t gl,
                                                   uint32_t num) {
-    const int lim = (int)num - (int)gl;
-    const uint32_t lane4 = lane_id() * 4u;
-    uint32_t best = kInvalid;
-    int off = 0;
-#pragma unroll
-    for (uint32_t r = 1; r <= R; ++r) {
-        const uint32_t a = __float_as_uint(box_area(box_union(own, lds_get_box(s, slot + r))));
-        const uint32_t af = (int)r < lim ? a : kInvalid;
-        uint32_t ab = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(lane4 - 4u * r), (int)af);
-        ab = gl >= r ? ab : kInvalid;
-        if (af < best) off = (int)r;
-        best = min(best, af);
-        if (ab < best) off = -(int)r;
-        best = min(best, ab);
-        __builtin_amdgcn_sched_barrier(0);
-    }
-    return off ? (uint32_t)((int)gl + off) : kInvalid;
+    return nearest<R>(s, own, slot, gl, (int)num - (int)gl, R);
+}
+
+// The loop runs to Rw, the largest radius of the wave's groups, on scalar
+// control; R is the lane's own radius.
+__device__ __forceinline__ uint32_t nearest_uniform(const HplocLds& s, const Box& own, uint32_t slot, uint32_t gl,
+                                                    uint32_t num, uint32_t Rw, uint32_t R) {
+    return nearest<2>(s, own, slot, gl, min((int)num - (int)gl, (int)R + 1), Rw);
 }
 
 struct NodeStore {
@@ -509,17 +508,15 @@ __device__ __forceinline__ void ploc_merge(HplocLds& s, bool has_task, uint32_t 
     // clusters here and after every compaction below.
     while (num > threshold) {
         // ---- FindNearestNeighbor (BinaryBuilder.cu:127-163) ----
-        // lane i computes the forward areas a(i, i+r); a(i-r, i) is lane
-        // i-r's forward area at distance r, fetched with a lane shuffle
         uint32_t nn = kInvalid;
         if (fixed_r == 8) nn = nearest_fixed<8>(s, own, slot, gl, num);
         else nn = nearest_uniform(s, own, slot, gl, num, r_wave, R);
         if (gl >= num) nn = kInvalid;
 
         // ---- MergeClustersCreateBVH2Node (BinaryBuilder.cu:72-124) ----
-        s.nn[slot] = nn;
-        wave_lds_sync();
-        uint32_t nnnn = nn < (uint32_t)GW ? s.nn[gbase + nn] : kInvalid;
+        // the neighbour's neighbour, from its lane
+        const uint32_t theirs = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((gbase + nn) * 4u), (int)nn);
+        const uint32_t nnnn = nn < (uint32_t)GW ? theirs : kInvalid;
         bool mutual = gl < num && nnnn == gl;
         bool merge = mutual && gl < nn;
         uint64_t mm = ballot(merge) & gmask;
@@ -608,6 +605,7 @@ __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6
 
     uint32_t left = 0, right = 0, split = 0;
     bool active = false;
+    bool pending = false;        // a merge's stores may be in flight (wave-uniform)
     MeshCtx mc{0u, n, 0u, 0u};  // this lane's mesh (the whole array for a single build)
     uint32_t hi = n - 1;
 
@@ -714,10 +712,14 @@ __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6
         // left-going lane hands its range end over and stops. Each slot has
         // one candidate per side, so a lane found through the slot hash is
         // the partner iff it posted the same slot; every other lane takes
-        // the exchange. The wave's stores are complete (end of the previous
-        // step), so the continuing lane reads the partner's clusters as it
+        // the exchange. The wave's stores are complete (the wait just below),
+        // so the continuing lane reads the partner's clusters as it
         // would after an exchange. Skipped (wave-uniform) unless the wave
         // has lanes going both ways, as on the serial climb near the root.
+        if (pending) {
+            pending = false;
+            wait_memory_ops();
+        }
         if (ballot(active && to_right) != 0 && ballot(active && !to_right) != 0) {
             const uint32_t slot = to_right ? right : left - 1;
             s.mslot[lane] = (active && to_right) ? slot : kInvalid;
@@ -801,8 +803,9 @@ __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6
             ploc_merge<GW, !BATCH>(s, has, tl, ts, tr + 1, tf, gl, gbase, gmask, cluster, recs, csizes, ns, tm, rp, flags);
         }
         // Merge outputs are agent-scope atomic stores; they must be complete
-        // before this wave's next parent exchange hands the subtree over.
-        wait_memory_ops();
+        // before this wave's next parent exchange hands the subtree over. The
+        // wait stands after the next step's key loads, whose latency it covers.
+        pending = true;
     }
 }
 
