@@ -305,10 +305,10 @@ nxb_status prep_bvh2(uint32_t n, const nxb_build_config& cfg, const Carved& w, h
     const uint32_t bits = morton_bits_of(cfg);
     uint32_t b, e;
     morton_sort_window(bits, b, e);
-    const SortPlan pl = plan_sort(n, bits, b, e, digit_bits_of(cfg, bits, n));
+    const SortPlan pl = plan_sort(n, bits, b, e, digit_bits_of(cfg, bits, n), cfg.sort_digit_bits == 0);
     // header, parent table and the sort's digit histograms in one launch
     NXB_HIP(launch_build_prep(w.hdr(), kHdrHplocChunks + kHplocCounterWords, w.parent(), n, w.hist(),
-                              pl.passes << pl.bits, s));
+                              pl.merge ? 0u : pl.passes << pl.bits, s));
     return NXB_SUCCESS;
 }
 
@@ -324,9 +324,13 @@ nxb_status run_bvh2(const void* prims, nxb_prim_type type, uint32_t n, const nxb
     BoundsScratch bs{w.partials(), w.done(), kMaxBoundsBlocks};
     NXB_HIP(launch_scene_bounds(prims, type, n, nodes, w.scene(), w.flags(), bs, s, indices, vertex_count));
     ev.record(1, s);
-    // Morton codes with the sort's digit histograms (zeroed in prep_bvh2).
-    SortPlan pl = plan_sort(n, bits, b, e, digit_bits_of(cfg, bits, n));
-    NXB_HIP(launch_morton_hist(nodes, n, w.scene(), w.keys_a(), pl, w.hist(), s));
+    // Morton codes with the sort's digit histograms (zeroed in prep_bvh2); a
+    // merged sort needs none
+    SortPlan pl = plan_sort(n, bits, b, e, digit_bits_of(cfg, bits, n), cfg.sort_digit_bits == 0);
+    if (pl.merge)
+        NXB_HIP(launch_morton(nodes, n, w.scene(), bits, w.keys_a(), nullptr, s));
+    else
+        NXB_HIP(launch_morton_hist(nodes, n, w.scene(), w.keys_a(), pl, w.hist(), s));
     ev.record(2, s);
     NXB_HIP(launch_sort_passes(w.keys_a(), nullptr, w.keys_b(), w.vals_b(), w.keys_tmp(), w.vals_tmp(), n, pl,
                                w.sort(), s));
@@ -920,8 +924,7 @@ nxb_status nxb_radix_sort_pairs(const void* d_keys_in, const uint32_t* d_values_
                                 nxb_stream_t stream) {
     if (key_bits != 32 && key_bits != 64) return NXB_ERROR_INVALID_VALUE;
     if (begin_bit > end_bit || end_bit > key_bits) return NXB_ERROR_INVALID_VALUE;
-    if (digit_bits == 0) digit_bits = default_digit_bits(n, key_bits);
-    if (digit_bits < 6 || digit_bits > 9) return NXB_ERROR_INVALID_VALUE;
+    if (digit_bits != 0 && (digit_bits < 6 || digit_bits > 9)) return NXB_ERROR_INVALID_VALUE;
     if (n > NXB_MAX_PRIMS) return NXB_ERROR_TOO_LARGE;
     if (n == 0) return NXB_SUCCESS;
     if (!d_keys_in || !d_keys_out || !d_values_out) return NXB_ERROR_INVALID_VALUE;

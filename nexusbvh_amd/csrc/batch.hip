@@ -395,7 +395,7 @@ nxb_status enqueue_batch(nxb_batch_plan& p, hipStream_t s, bool events) {
     // flags, then the H-PLOC chunk counters from word kBatchHplocChunks
     NXB_HIPB(launch_fill_u32(p.flags, 0u, kBatchHplocChunks + kHplocCounterWords, s));
     // the sort's digit histograms, counted by the Morton kernel
-    const SortPlan pl = plan_sort(n, 64, 2, p.key_end, p.digit_bits);
+    const SortPlan pl = plan_sort(n, 64, 2, p.key_end, p.digit_bits, p.cfg.sort_digit_bits == 0);
     if (pl.passes > kBatchHistMaxPasses) return NXB_ERROR_INVALID_VALUE;
     SortScratch ss{p.hist, p.counts, p.counts_words};
     NXB_HIPB(launch_sort_prepare(pl, ss, s));

@@ -93,19 +93,23 @@ hipError_t launch_build_prep(uint32_t* hdr, uint32_t hdr_words, uint32_t* parent
 struct SortPlan {
     uint32_t key_bits, begin, end, bits, passes, tiles;
     uint32_t wide;  // 1: wide tile shape (large inputs)
+    uint32_t merge;  // 1: runs sorted in LDS and merged (small inputs): no digit histograms, no count table
 };
-SortPlan plan_sort(uint32_t n, uint32_t key_bits, uint32_t begin_bit, uint32_t end_bit, uint32_t digit_bits);
+// merge_ok: the caller left the digit width open, so small inputs may be merged.
+SortPlan plan_sort(uint32_t n, uint32_t key_bits, uint32_t begin_bit, uint32_t end_bit, uint32_t digit_bits,
+                   bool merge_ok);
 // Digit width used when the caller leaves it open: 7 for 32-bit keys; 8 for
 // 64-bit keys, 9 once the input takes the wide tile shape.
 uint32_t default_digit_bits(uint32_t n, uint32_t key_bits);
 size_t sort_scratch_bytes(uint32_t n, uint32_t key_bits, uint32_t digit_bits);
-// Zeroes the digit histograms of a plan.
+// Zeroes the digit histograms of a plan (none for a merged one).
 hipError_t launch_sort_prepare(const SortPlan& pl, SortScratch sc, hipStream_t s);
 // Digit histograms of every pass (also produced by the Morton kernel).
 hipError_t launch_sort_histogram(const void* keys, uint32_t n, const SortPlan& pl, SortScratch sc, hipStream_t s);
 hipError_t launch_sort_passes(const void* keys_in, const uint32_t* values_in, void* keys_out, uint32_t* values_out,
                               void* keys_tmp, uint32_t* values_tmp, uint32_t n, const SortPlan& pl, SortScratch sc,
                               hipStream_t s);
+// digit_bits 0: the library's choice.
 hipError_t launch_radix_sort(const void* keys_in, const uint32_t* values_in, void* keys_out,
                              uint32_t* values_out, void* keys_tmp, uint32_t* values_tmp, uint32_t n,
                              uint32_t key_bits, uint32_t begin_bit, uint32_t end_bit, uint32_t digit_bits,

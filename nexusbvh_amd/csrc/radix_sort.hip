@@ -20,6 +20,9 @@
 //  * keys and values are read with the nontemporal hint (each pass streams
 //    them once; measured 7% faster at 28.1M keys); stores stay normal, since
 //    the scattered runs of a pass are combined in L2;
+//  * small inputs are sorted in runs of 2,048 keys in LDS and the runs merged
+//    by rank (k_sort_runs, k_sort_merge): one to three launches in all, where
+//    the passes above take three each, 4 to 9 us a launch however few the keys;
 //  * block b works on tile (b % 8) * per + b / 8: blocks are dispatched to
 //    the 8 XCDs round-robin, so each XCD gets a contiguous range of tiles
 //    and the table lines its blocks write and read stay in its own L2.
@@ -446,6 +449,184 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) 
     }
 }
 
+// ---- small inputs: runs sorted in LDS, then merged -------------------------
+//
+// Sorts every run of kRunKeys keys (block b: run b) on bits [begin_bit,
+// end_bit): the keys stay in registers from pass to pass and go through LDS
+// for the reordering. Ranking as in k_sort_downsweep (row k of wave w holds 64
+// consecutive elements). Elements past n carry the all-ones key and stay last.
+// Bound by the latency of a pass's five barriers (2.5 us a pass; 256 threads
+// 26 us a run of 64-bit Morton keys, 512 and 1024 threads 21 us; runs of 4,096
+// keys 31 us, of 8,192 keys 52 us).
+constexpr int kRunThreads = 512;
+constexpr uint32_t kRunKeys = 2048;
+constexpr int kRunItems = kRunKeys / kRunThreads;
+
+template <typename K>
+__global__ __launch_bounds__(kRunThreads) void k_sort_runs(const K* __restrict__ keys_in,
+                                                           const uint32_t* __restrict__ vals_in,
+                                                           K* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
+                                                           uint32_t n, uint32_t begin_bit, uint32_t end_bit) {
+    constexpr int BITS = 8, RADIX = 1 << BITS, WAVES = kRunThreads / 64, ITEMS = kRunItems;
+    __shared__ K skeys[kRunKeys];
+    __shared__ uint32_t svals[kRunKeys];
+    __shared__ uint32_t wave_off[WAVES / 2][RADIX];  // as in k_sort_downsweep
+    __shared__ uint32_t scan_tmp[WAVES];
+    const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+    const uint32_t wrow = w >> 1, wsh = (w & 1) * 16;
+    const uint32_t local = w * ITEMS * 64 + lane, first = blockIdx.x * kRunKeys + local;
+    K key[ITEMS];
+    uint32_t val[ITEMS];
+    load_rows<K, ITEMS>(keys_in, vals_in, n, first, key, val);
+    fix_rows<K, ITEMS>(n, first, key, val);
+    for (uint32_t shift = begin_bit; shift < end_bit; shift += BITS) {
+        const uint32_t width = min((uint32_t)BITS, end_bit - shift);
+        auto digit = [&](K k) {
+            if constexpr (sizeof(K) == 8)
+                return shift >= 32 ? pass_digit<K, true>(k, shift, width) : pass_digit<K, false>(k, shift, width);
+            else
+                return pass_digit<K, false>(k, shift, width);
+        };
+        for (uint32_t i = tid; i < (uint32_t)(WAVES / 2 * RADIX); i += kRunThreads) (&wave_off[0][0])[i] = 0;
+        __syncthreads();
+        uint32_t rl[ITEMS], lbase[ITEMS];  // rl = rank among peers | leader lane << 8
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const uint32_t d = digit(key[k]);
+            const uint64_t peers = match_digit<BITS>(d);
+            const uint32_t rr = mask_rank(peers);
+            rl[k] = rr | ((uint32_t)__builtin_ctzll(peers) << 8);
+            uint32_t got = 0;
+            if (rr == 0)
+                got = __hip_atomic_fetch_add(&wave_off[wrow][d], (uint32_t)__popcll(peers) << wsh, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP) >> wsh;
+            lbase[k] = got;
+        }
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) rl[k] = (rl[k] & 0xFFu) + (__shfl(lbase[k], (int)(rl[k] >> 8)) & 0xFFFFu);
+        __syncthreads();
+        // thread d: the slot of each wave's first key of digit d
+        uint32_t tsum = 0;
+        if (tid < (uint32_t)RADIX) {
+#pragma unroll
+            for (int ww = 0; ww < WAVES / 2; ++ww) {
+                const uint32_t pair = wave_off[ww][tid];
+                tsum += (pair & 0xFFFFu) + (pair >> 16);
+            }
+        }
+        uint32_t slot = block_exclusive_scan<WAVES>(tsum, scan_tmp, nullptr);
+        if (tid < (uint32_t)RADIX) {
+#pragma unroll
+            for (int ww = 0; ww < WAVES / 2; ++ww) {
+                const uint32_t pair = wave_off[ww][tid];
+                const uint32_t s0 = slot;
+                slot += pair & 0xFFFFu;
+                wave_off[ww][tid] = s0 | (slot << 16);
+                slot += pair >> 16;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            const uint32_t pos = ((wave_off[wrow][digit(key[k])] >> wsh) & 0xFFFFu) + rl[k];
+            skeys[pos] = key[k];
+            svals[pos] = val[k];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < ITEMS; ++k) {
+            key[k] = skeys[local + k * 64];
+            val[k] = svals[local + k * 64];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < ITEMS; ++k) {
+        if (first + k * 64 < n) {
+            keys_out[first + k * 64] = key[k];
+            vals_out[first + k * 64] = val[k];
+        }
+    }
+}
+
+// Merges every group of up to kMergeRuns sorted runs of `run` keys (a multiple
+// of kMergeThreads * kMergeSamples) into one, by rank: an element's place is
+// its index in its own run plus, for every other run of the group, the number
+// of elements before it there (equal ones count as before in earlier runs, as
+// after in later ones, so the merge is stable). Each run is searched first
+// among kMergeSamples samples in LDS, then among the run / kMergeSamples
+// elements between two samples, kMergeUnroll runs at a time so that their
+// loads overlap. mask: the key bits compared. Bound by latency up to ~100K keys
+// (~6 us a level), then by the searches' instructions (15 runs of 12 to 16
+// steps for every key: 35 us a level at 300K keys).
+constexpr int kMergeThreads = 256;
+constexpr uint32_t kMergeRuns = 16, kMergeSamples = 128, kMergeUnroll = 4;
+static_assert(kMergeRuns % kMergeUnroll == 0 && kRunKeys % kMergeThreads == 0 && kRunKeys % kMergeSamples == 0, "runs");
+
+template <typename K>
+__global__ __launch_bounds__(kMergeThreads) void k_sort_merge(const K* __restrict__ keys,
+                                                              const uint32_t* __restrict__ vals,
+                                                              K* __restrict__ keys_out,
+                                                              uint32_t* __restrict__ vals_out, uint32_t n,
+                                                              uint32_t run, K mask) {
+    __shared__ K sample[kMergeRuns][kMergeSamples];
+    const uint32_t tid = threadIdx.x, i0 = blockIdx.x * kMergeThreads, i = i0 + tid;
+    const uint32_t g0 = i0 - i0 % (run * kMergeRuns);        // the group's first element
+    const uint32_t own = (i0 - g0) / run;                    // the block's run in the group
+    const uint32_t runs = min(kMergeRuns, (n - g0 + run - 1) / run);
+    const uint32_t gap = run / kMergeSamples;
+    // sample k of a run: the last of its (k+1)-th `gap` elements; past n: larger than any masked key or equal to it
+    for (uint32_t k = tid; k < runs * kMergeSamples; k += kMergeThreads) {
+        const uint32_t at = g0 + (k + 1) * gap - 1;
+        (&sample[0][0])[k] = at < n ? keys[at] & mask : ~(K)0;
+    }
+    const K key = keys[min(i, n - 1)];
+    const uint32_t val = vals[min(i, n - 1)];
+    const K x = key & mask;
+    __syncthreads();
+    uint32_t rank = g0 + (i - g0) % run;
+    for (uint32_t r0 = 0; r0 < runs; r0 += kMergeUnroll) {
+        uint32_t q[kMergeUnroll];
+#pragma unroll
+        for (uint32_t u = 0; u < kMergeUnroll; ++u) q[u] = 0;
+#pragma unroll
+        for (uint32_t step = kMergeSamples / 2;; step >>= 1) {
+            // the last round (step 0) tests the one sample left
+#pragma unroll
+            for (uint32_t u = 0; u < kMergeUnroll; ++u) {
+                const K k = sample[min(r0 + u, runs - 1)][q[u] + (step ? step - 1 : 0)];
+                const bool before = r0 + u < own ? !(x < k) : k < x;
+                q[u] += before ? max(step, 1u) : 0u;
+            }
+            if (step == 0) break;
+        }
+        uint32_t base[kMergeUnroll];
+#pragma unroll
+        for (uint32_t u = 0; u < kMergeUnroll; ++u) {
+            base[u] = g0 + (r0 + u) * run;
+            q[u] *= gap;
+        }
+        for (uint32_t step = gap / 2; step; step >>= 1) {
+            K k[kMergeUnroll];
+#pragma unroll
+            for (uint32_t u = 0; u < kMergeUnroll; ++u) k[u] = keys[min(base[u] + q[u] + step - 1, n - 1)];
+#pragma unroll
+            for (uint32_t u = 0; u < kMergeUnroll; ++u) {
+                const uint32_t at = q[u] + step - 1;
+                const K m = k[u] & mask;
+                const bool before = (r0 + u < own ? !(x < m) : m < x) && at < run && base[u] + at < n;
+                q[u] += before ? step : 0u;
+            }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kMergeUnroll; ++u)
+            if (r0 + u < runs && r0 + u != own) rank += q[u];
+    }
+    if (i < n && rank < n) {  // rank < n always holds
+        keys_out[rank] = key;
+        vals_out[rank] = val;
+    }
+}
+
 template <typename K>
 __global__ void k_copy_pairs(const K* __restrict__ ki, const uint32_t* __restrict__ vi, K* __restrict__ ko,
                              uint32_t* __restrict__ vo, uint32_t n) {
@@ -476,6 +657,17 @@ struct TileShape {
 };
 
 constexpr uint32_t kWideMinKeys = 1u << 23;
+// Keys up to which runs are sorted and merged, by the passes that the LSD sort
+// would take (measured on Morton keys, us, merged / LSD):
+//   8 passes (64-bit keys): 21 / 123 at 2,003, 33 / 141 at 16,411, 50 / 146 at
+//     100K, 90 / 153 at 300K, 130 / 158 at 2^19, the most that two levels hold;
+//   4 passes (32-bit keys): 11 / 64, 22 / 73, 36 / 75, 67 / 76, 104 / 77, equal
+//     between 300K and 400K.
+// Fewer passes: only up to one level, a launch or two against three per pass.
+constexpr uint32_t merge_sort_max(uint32_t passes) {
+    return passes >= 8 ? 1u << 19 : passes >= 4 ? 5u << 16 : kRunKeys * kMergeRuns;
+}
+static_assert(merge_sort_max(8) <= kRunKeys * kMergeRuns * kMergeRuns, "two levels of merging");
 
 constexpr uint32_t tile_keys(uint32_t key_bytes, uint32_t bits, bool wide) {
     return wide ? (key_bytes == 8 ? TileShape<8, 8, true>::tile : TileShape<4, 8, true>::tile)
@@ -537,6 +729,29 @@ hipError_t run_histogram(const K* keys, uint32_t n, const SortPlan& pl, SortScra
     return hipGetLastError();
 }
 
+// Levels of merging that n keys take: 0 (one run), 1 or 2.
+template <typename K>
+hipError_t run_merge_sort(const K* ki, const uint32_t* vi, K* ko, uint32_t* vo, K* kt, uint32_t* vt, uint32_t n,
+                          const SortPlan& pl, hipStream_t s) {
+    const uint32_t levels = n <= kRunKeys ? 0u : n <= kRunKeys * kMergeRuns ? 1u : 2u;
+    const K mask = (K)(~(K)0 >> (8 * sizeof(K) - (pl.end - pl.begin))) << pl.begin;
+    // the runs start where the last merge ends in the outputs
+    K* dk = levels == 1 ? kt : ko;
+    uint32_t* dv = levels == 1 ? vt : vo;
+    hipLaunchKernelGGL(k_sort_runs<K>, dim3((n + kRunKeys - 1) / kRunKeys), dim3(kRunThreads), 0, s, ki, vi, dk, dv, n,
+                       pl.begin, pl.end);
+    uint32_t run = kRunKeys;
+    for (uint32_t l = 0; l < levels; ++l, run *= kMergeRuns) {
+        K* nk = dk == ko ? kt : ko;
+        uint32_t* nv = dv == vo ? vt : vo;
+        hipLaunchKernelGGL(k_sort_merge<K>, dim3((n + kMergeThreads - 1) / kMergeThreads), dim3(kMergeThreads), 0, s,
+                           dk, dv, nk, nv, n, run, mask);
+        dk = nk;
+        dv = nv;
+    }
+    return hipGetLastError();
+}
+
 template <typename K>
 hipError_t dispatch(bool hist_only, const void* ki, const uint32_t* vi, void* ko, uint32_t* vo, void* kt,
                     uint32_t* vt, uint32_t n, const SortPlan& pl, SortScratch sc, hipStream_t s) {
@@ -554,7 +769,8 @@ hipError_t dispatch(bool hist_only, const void* ki, const uint32_t* vi, void* ko
 
 }  // namespace
 
-SortPlan plan_sort(uint32_t n, uint32_t key_bits, uint32_t begin_bit, uint32_t end_bit, uint32_t digit_bits) {
+SortPlan plan_sort(uint32_t n, uint32_t key_bits, uint32_t begin_bit, uint32_t end_bit, uint32_t digit_bits,
+                   bool merge_ok) {
     SortPlan pl;
     pl.key_bits = key_bits;
     pl.begin = begin_bit;
@@ -564,6 +780,7 @@ SortPlan plan_sort(uint32_t n, uint32_t key_bits, uint32_t begin_bit, uint32_t e
     pl.wide = n >= kWideMinKeys ? 1u : 0u;
     const uint32_t tile = tile_keys(key_bits / 8, digit_bits, pl.wide != 0);
     pl.tiles = (n + tile - 1) / tile;
+    pl.merge = merge_ok && pl.passes && n <= merge_sort_max(pl.passes) ? 1u : 0u;
     return pl;
 }
 
@@ -587,13 +804,13 @@ size_t sort_scratch_bytes(uint32_t n, uint32_t key_bits, uint32_t digit_bits) {
 
 hipError_t launch_sort_prepare(const SortPlan& pl, SortScratch sc, hipStream_t s) {
     if (pl.passes > (uint32_t)kMaxPasses || (pl.passes << pl.bits) > kHistCopyWords) return hipErrorInvalidValue;
-    if (pl.passes == 0) return hipSuccess;
+    if (pl.passes == 0 || pl.merge) return hipSuccess;
     hipLaunchKernelGGL(k_sort_init, dim3(kHistCopies), dim3(256), 0, s, sc.hist, pl.passes << pl.bits);
     return hipGetLastError();
 }
 
 hipError_t launch_sort_histogram(const void* keys, uint32_t n, const SortPlan& pl, SortScratch sc, hipStream_t s) {
-    if (pl.passes == 0 || n <= 1) return hipSuccess;
+    if (pl.passes == 0 || pl.merge || n <= 1) return hipSuccess;
     if (pl.key_bits == 32) return dispatch<uint32_t>(true, keys, nullptr, nullptr, nullptr, nullptr, nullptr, n, pl, sc, s);
     return dispatch<uint64_t>(true, keys, nullptr, nullptr, nullptr, nullptr, nullptr, n, pl, sc, s);
 }
@@ -614,6 +831,13 @@ hipError_t launch_sort_passes(const void* keys_in, const uint32_t* values_in, vo
                                values_out, n);
         return hipGetLastError();
     }
+    if (pl.merge) {
+        if (pl.key_bits == 32)
+            return run_merge_sort(static_cast<const uint32_t*>(keys_in), values_in, static_cast<uint32_t*>(keys_out),
+                                  values_out, static_cast<uint32_t*>(keys_tmp), values_tmp, n, pl, s);
+        return run_merge_sort(static_cast<const uint64_t*>(keys_in), values_in, static_cast<uint64_t*>(keys_out),
+                              values_out, static_cast<uint64_t*>(keys_tmp), values_tmp, n, pl, s);
+    }
     if (((size_t)pl.tiles << pl.bits) > sc.counts_words || pl.passes > (uint32_t)kMaxPasses ||
         (pl.passes << pl.bits) > kHistCopyWords)
         return hipErrorInvalidValue;
@@ -627,8 +851,10 @@ hipError_t launch_radix_sort(const void* keys_in, const uint32_t* values_in, voi
                              uint32_t key_bits, uint32_t begin_bit, uint32_t end_bit, uint32_t digit_bits,
                              SortScratch sc, hipStream_t s) {
     if (end_bit < begin_bit || end_bit > key_bits || (key_bits != 32 && key_bits != 64)) return hipErrorInvalidValue;
+    const bool any = digit_bits == 0;
+    if (any) digit_bits = default_digit_bits(n, key_bits);
     if (digit_bits < 6 || digit_bits > 9) return hipErrorInvalidValue;
-    SortPlan pl = plan_sort(n, key_bits, begin_bit, end_bit, digit_bits);
+    SortPlan pl = plan_sort(n, key_bits, begin_bit, end_bit, digit_bits, any);
     hipError_t e = launch_sort_prepare(pl, sc, s);
     if (e != hipSuccess) return e;
     e = launch_sort_histogram(keys_in, n, pl, sc, s);
