@@ -57,21 +57,23 @@ bool fail_alloc_injected() {
     return v && v[0] == '1';
 }
 
-// BVH8 levels enqueued before the first counter readback. NXB_BVH8_FIRST_LEVELS
-// (1..96) fixes the count; tests use it to reach the path that adds levels
-// after the readback. Otherwise: one more than the depth of the device's last
-// tree when that had within 1/8 as many primitives (rebuilds of one scene),
-// else kBvh8FirstLevels. A level launch past the end of the tree costs ~4.5 us
-// on the GPU, one too few a readback round trip.
-uint32_t bvh8_first_levels(uint32_t n, uint32_t last_n, uint32_t last_depth) {
+// Collapse launches enqueued before the first counter readback.
+// NXB_BVH8_FIRST_LEVELS (1..96) fixes the count; tests use it to reach the path
+// that adds launches after the readback. Otherwise, for rebuilds of one scene
+// (within 1/8 as many primitives as the device's last tree): as many as that
+// tree took, and one more where a launch is a level; else 8, or 24 levels. A
+// launch past the end of the tree costs ~4.5 us on the GPU, one too few a
+// readback round trip.
+uint32_t bvh8_first_launches(uint32_t n, uint32_t last_n, uint32_t last_launches) {
+    const uint32_t unknown = bvh8_small(n) ? 8u : 24u;
     if (const char* v = std::getenv("NXB_BVH8_FIRST_LEVELS")) {
         const long x = std::strtol(v, nullptr, 10);
-        return x >= 1 && x < (long)kBvh8LevelWords ? (uint32_t)x : kBvh8FirstLevels;
+        return x >= 1 && x < (long)kBvh8LevelWords ? (uint32_t)x : unknown;
     }
     const uint32_t tol = n / 8;
-    if (last_depth && last_n + tol >= n && last_n <= n + tol)
-        return last_depth + 1 < kBvh8LevelWords ? last_depth + 1 : kBvh8LevelWords - 1;
-    return kBvh8FirstLevels;
+    if (last_launches && last_n + tol >= n && last_n <= n + tol && bvh8_small(last_n) == bvh8_small(n))
+        return min(last_launches + (bvh8_small(n) ? 0u : 1u), kBvh8LevelWords - 1);
+    return unknown;
 }
 
 // Scratch carved from one device buffer. Sizes depend on (n, key bytes).
@@ -90,16 +92,17 @@ constexpr uint32_t kMaxBoundsBlocks = 2048;
 //   [16..22) scene box (6 floats)
 //   [32..36) two FP64 SAH accumulators   [48..56) H-PLOC spare node slot
 //   [64..80) H-PLOC spare wide record (BVH8 builds; 64-byte aligned)
-//   [128..130) BVH8 node counter (finished << 32 | allocated), own cache line
+//   [128..130) BVH8 node counter (own cache line): nodes below the root of a
+//              build; (finished << 32 | allocated) of the stage entry point
 //   [160] BVH8 work grab counter, own cache line
 //   [256..512) H-PLOC chunk counters
-//   [512..609) BVH8 level counters (level-synchronous collapse)
+//   [512..609) BVH8 queue counters, one per collapse launch
 constexpr size_t kHdrDone = 0, kHdrFlags = 1, kHdrMovedParent = 2, kHdrMovedSize = 3, kHdrFallbacks = 4,
                  kHdrScene = 16, kHdrHplocChunks = 256,
                  kHdrSah = 32, kHdrMoved = 48, kHdrMovedRec = 64, kHdrBvh8Ctr = 128, kHdrBvh8Grab = 160,
                  kHdrBvh8Levels = 512;
 constexpr size_t kHeaderBytes = 4096;
-// header words read back after a build: flags, scene box, BVH8 level counters
+// header words read back after a build: flags, scene box, BVH8 counters
 constexpr size_t kReadbackWords = kHdrBvh8Levels + kBvh8LevelWords;
 static_assert(kHdrHplocChunks + kHplocCounterWords <= kHdrBvh8Levels, "header words overlap");
 
@@ -179,7 +182,7 @@ struct DeviceState {
     uint8_t* ws = nullptr;
     size_t ws_bytes = 0;
     uint32_t* host = nullptr;  // pinned readback buffer (kReadbackWords words)
-    uint32_t last_n = 0, last_depth = 0;  // primitives and BVH8 levels of the last build
+    uint32_t last_n = 0, last_launches = 0;  // primitives and collapse launches of the last BVH8 build
     hipEvent_t ev[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};  // stage timing (builds hold g_mutex)
     // Stage entry points that return before their kernels finish
     // (nxb_compute_scene_bounds, nxb_radix_sort_pairs without a workspace of
@@ -307,7 +310,7 @@ nxb_status prep_bvh2(uint32_t n, const nxb_build_config& cfg, const Carved& w, h
     morton_sort_window(bits, b, e);
     const SortPlan pl = plan_sort(n, bits, b, e, digit_bits_of(cfg, bits, n), cfg.sort_digit_bits == 0);
     // header, parent table and the sort's digit histograms in one launch
-    NXB_HIP(launch_build_prep(w.hdr(), kHdrHplocChunks + kHplocCounterWords, w.parent(), n, w.hist(),
+    NXB_HIP(launch_build_prep(w.hdr(), kReadbackWords, w.parent(), n, w.hist(),
                               pl.merge ? 0u : pl.passes << pl.bits, s));
     return NXB_SUCCESS;
 }
@@ -518,36 +521,37 @@ nxb_status build_common(const void* prims, nxb_prim_type type, uint32_t n, const
         if (!st) st = alloc_out((void**)&ob.prim_idx, (size_t)n * sizeof(uint32_t), s);
     }
     if (!st) st = run_bvh2(prims, type, n, cfg, ob.nodes, w, ev, s, indices, vertex_count);
-    // level-synchronous BVH8: the first levels here; their counters come back
-    // with the header below, and deeper trees get more levels there
-    uint32_t* level_cnt = w.hdr() + kHdrBvh8Levels;
-    uint32_t launched = 0, node8 = 0;
+    // BVH8: the first collapse launches here; their counters come back with
+    // the header below, and trees that need more get them there
+    uint32_t* cnt = w.hdr() + kHdrBvh8Levels;
+    uint32_t* nodes_below = w.hdr() + kHdrBvh8Ctr;
+    uint32_t launched = 0, launches = 0, node8 = 0;
     if (!st && out8) {
-        launched = max(bvh8_first_levels(n, d.last_n, d.last_depth), kBvh8TopLevels);
-        st = from_hip(launch_bvh8_levels(ob.nodes, n, ob.n8, ob.prim_idx, cap, bs, level_cnt, 0, launched, s));
+        launched = bvh8_first_launches(n, d.last_n, d.last_launches);
+        if (!bvh8_small(n)) launched = max(launched, kBvh8TopLevels);
+        st = from_hip(launch_bvh8_collapse(ob.nodes, n, ob.n8, ob.prim_idx, cap, bs, cnt, nodes_below, 0, launched, s));
     }
     if (st) return st;
     ev.record(5, s);
-    // Read back flags, scene box and BVH8 level counters in one copy.
+    // Read back flags, scene box and BVH8 counters in one copy.
     NXB_HIP(hipMemcpyAsync(d.host, w.hdr(), kReadbackWords * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     NXB_HIP(hipStreamSynchronize(s));
     d.ws_pending = false;  // s waited for the pending stage work and has drained
-    while (out8 && !bvh8_levels_done(n, d.host + kHdrBvh8Levels, launched, &node8)) {
+    while (out8 && !(launches = bvh8_launches(n, d.host + kHdrBvh8Levels, d.host[kHdrBvh8Ctr], launched, &node8))) {
         if (launched >= kBvh8LevelWords - 1) {
-            d.host[kHdrFlags] |= kFlagBadIndex;  // deeper than the level counters reach
+            d.host[kHdrFlags] |= kFlagBadIndex;  // more launches than the counters reach
             break;
         }
-        NXB_HIP(launch_bvh8_levels(ob.nodes, n, ob.n8, ob.prim_idx, cap, bs, level_cnt, launched, 16, s));
-        launched += 16;
+        const uint32_t more = min(bvh8_small(n) ? 4u : 16u, kBvh8LevelWords - 1 - launched);
+        NXB_HIP(launch_bvh8_collapse(ob.nodes, n, ob.n8, ob.prim_idx, cap, bs, cnt, nodes_below, launched, more, s));
+        launched += more;
         ev.record(5, s);
         NXB_HIP(hipMemcpyAsync(d.host, w.hdr(), kReadbackWords * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
         NXB_HIP(hipStreamSynchronize(s));
     }
-    if (out8 && node8) {
-        uint32_t depth = 0;
-        while (depth < kBvh8LevelWords && d.host[kHdrBvh8Levels + depth] != 0) ++depth;
+    if (out8 && launches) {
         d.last_n = n;
-        d.last_depth = depth;
+        d.last_launches = launches;
     }
     uint32_t flags = d.host[kHdrFlags];
     nxb_aabb scene;

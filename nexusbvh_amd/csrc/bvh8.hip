@@ -405,8 +405,7 @@ template <bool KEEP = true>
 __device__ __forceinline__ void emit_node(const ChildBoxes& cbx, uint32_t tid, const Collapsed& c, uint32_t k,
                                           uint32_t child_base, uint32_t prim_base, uint32_t leaf_count,
                                           const uint32_t sz[8], nxb_bvh8_node* out, uint32_t* prim_idx,
-                                          uint32_t n, uint32_t node_count, uint32_t capacity, uint64_t* work,
-                                          uint64_t* work2, uint32_t* flags,
+                                          uint32_t n, uint32_t capacity, uint64_t* work, uint32_t* flags,
                                           uint32_t& keep_slot, uint32_t& keep_x, uint32_t& keep_base) {
     keep_slot = kNoSlot;
     keep_x = kInvalid;
@@ -416,10 +415,10 @@ __device__ __forceinline__ void emit_node(const ChildBoxes& cbx, uint32_t tid, c
     for (uint32_t s = 0; s < 8; ++s) {
         uint32_t a = nib(c.assign, s);
         if (a == 0xFu) continue;
-        uint32_t ch = 0, pl = 0, pr = 0;
+        uint32_t ch = 0, pr = 0;
 #pragma unroll
         for (uint32_t t = 0; t < 8; ++t)
-            if (t == a) { ch = c.child[t]; pl = c.cleft[t]; pr = c.cright[t]; }
+            if (t == a) { ch = c.child[t]; pr = c.cright[t]; }
         if (c.im & (1u << s)) {
             uint32_t slot = child_base + bits_below(c.im, s);
             const uint32_t size = sz[s];
@@ -428,7 +427,6 @@ __device__ __forceinline__ void emit_node(const ChildBoxes& cbx, uint32_t tid, c
             } else if (!KEEP) {
                 // read by the next level's kernel
                 work[slot] = ((uint64_t)next_base << 32) | ch;
-                if (work2) work2[slot] = ((uint64_t)pr << 32) | pl;
             } else if (keep_slot == kNoSlot) {
                 keep_slot = slot;
                 keep_x = ch;
@@ -561,8 +559,8 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8(const nxb_bvh2_node* __re
                 uint32_t child_base = ic ? node_base + (excl >> 16) : 0u;
                 uint32_t sz[8];
                 load_child_sizes(c, nsize, n, node_count, sz);
-                emit_node(cbx, tid, c, slot, child_base, pbase, c.count - ic, sz, out, prim_idx, n, node_count,
-                          capacity, work, nullptr, flags, ks, kx, kb);
+                emit_node(cbx, tid, c, slot, child_base, pbase, c.count - ic, sz, out, prim_idx, n, capacity, work,
+                          flags, ks, kx, kb);
             }
             slot = ks;
             x = kx;
@@ -612,15 +610,11 @@ __device__ __forceinline__ uint32_t block_scan_256(uint32_t v, uint32_t* tmp, ui
 // nodes) one after another, the children's ids taken from a running count
 // instead of a global atomic. Saves the launches and counter round trips of
 // the levels whose time is all latency.
-// REC: collapse from the wide records (rec) instead of the BVH2 nodes; no
-// nsize, no work2.
-template <uint32_t SLOT, bool REC>
-__global__ __launch_bounds__(kBvh8Threads) void k_bvh8_top(const nxb_bvh2_node* __restrict__ b2, uint32_t n,
+template <uint32_t SLOT>
+__global__ __launch_bounds__(kBvh8Threads) void k_bvh8_top(const uint4* __restrict__ rec, uint32_t n,
                                                            uint32_t node_count, nxb_bvh8_node* __restrict__ out,
                                                            uint32_t* prim_idx, uint32_t capacity, uint64_t* work,
-                                                           uint64_t* work2, uint32_t* cnt,
-                                                           const uint32_t* __restrict__ nsize, uint32_t* flags,
-                                                           const uint4* __restrict__ rec) {
+                                                           uint32_t* cnt, uint32_t* flags) {
     __shared__ ChildBoxes cbx;
     __shared__ uint32_t scan_tmp[kBvh8Threads / 64];
     const uint32_t tid = threadIdx.x;
@@ -636,34 +630,25 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_top(const nxb_bvh2_node* 
             uint32_t pbase = 0;
             if (k < hi) {
                 uint32_t x = node_count - 1;  // the root, primitive base 0
-                uint64_t lr = 0;
                 if (level > 0) {
                     // written by this block's previous level (agent-scope
                     // loads: not through the CU's L1)
                     const uint64_t v = load_agent64(&work[k]);
-                    if constexpr (!REC) lr = load_agent64(&work2[k]);
                     x = (uint32_t)v;
                     pbase = (uint32_t)(v >> 32);
                 }
-                if constexpr (REC)
-                    ok = collapse_rec(rec, n, node_count, x, c, cbx, tid, SLOT);
-                else
-                    ok = x < node_count && collapse_node(b2, node_count, x, c, cbx, tid, SLOT, level > 0,
-                                                         (uint32_t)lr, (uint32_t)(lr >> 32));
+                ok = collapse_rec(rec, n, node_count, x, c, cbx, tid, SLOT);
                 if (!ok) atomic_or_agent(flags, kFlagBadIndex);
             }
             const uint32_t ic = ok ? (uint32_t)__popc(c.im) : 0u;
             uint32_t sz[8];
-            if (ok) {
-                if constexpr (REC) rec_child_sizes(c, sz);
-                else load_child_sizes(c, nsize, n, node_count, sz);
-            }
+            if (ok) rec_child_sizes(c, sz);
             uint32_t total = 0;
             const uint32_t excl = block_scan_256(ic, scan_tmp, &total);
             if (ok) {
                 uint32_t ks, kx, kb;
                 emit_node<false>(cbx, tid, c, k, ic ? hi + next + excl : 0u, pbase, c.count - ic, sz, out, prim_idx,
-                                 n, node_count, capacity, work, REC ? nullptr : work2, flags, ks, kx, kb);
+                                 n, capacity, work, flags, ks, kx, kb);
             }
             next += total;
         }
@@ -674,13 +659,11 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_top(const nxb_bvh2_node* 
     }
 }
 
-template <uint32_t SLOT, bool REC>
-__global__ __launch_bounds__(kBvh8Threads) void k_bvh8_level(const nxb_bvh2_node* __restrict__ b2, uint32_t n,
+template <uint32_t SLOT>
+__global__ __launch_bounds__(kBvh8Threads) void k_bvh8_level(const uint4* __restrict__ rec, uint32_t n,
                                                              uint32_t node_count, nxb_bvh8_node* __restrict__ out,
                                                              uint32_t* prim_idx, uint32_t capacity, uint64_t* work,
-                                                             uint64_t* work2, uint32_t* cnt, uint32_t level,
-                                                             const uint32_t* __restrict__ nsize, uint32_t* flags,
-                                                             const uint4* __restrict__ rec) {
+                                                             uint32_t* cnt, uint32_t level, uint32_t* flags) {
     __shared__ ChildBoxes cbx;
     __shared__ uint32_t scan_tmp[kBvh8Threads / 64];
     __shared__ uint32_t sbase;
@@ -703,22 +686,12 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_level(const nxb_bvh2_node
             const uint64_t v = work[k];
             const uint32_t x = (uint32_t)v;
             pbase = (uint32_t)(v >> 32);
-            if constexpr (REC) {
-                ok = collapse_rec(rec, n, node_count, x, c, cbx, tid, SLOT);
-            } else {
-                const bool have_lr = level > 0;  // written with work[k] by the level above
-                const uint64_t lr = have_lr ? work2[k] : 0ull;
-                ok = x < node_count && collapse_node(b2, node_count, x, c, cbx, tid, SLOT, have_lr, (uint32_t)lr,
-                                                     (uint32_t)(lr >> 32));
-            }
+            ok = collapse_rec(rec, n, node_count, x, c, cbx, tid, SLOT);
             if (!ok) atomic_or_agent(flags, kFlagBadIndex);
         }
         const uint32_t ic = ok ? (uint32_t)__popc(c.im) : 0u;
         uint32_t sz[8];
-        if (ok) {
-            if constexpr (REC) rec_child_sizes(c, sz);
-            else load_child_sizes(c, nsize, n, node_count, sz);
-        }
+        if (ok) rec_child_sizes(c, sz);
         uint32_t total = 0;
         const uint32_t excl = block_scan_256(ic, scan_tmp, &total);
         if (tid == 0) sbase = total ? hi + atomic_add_agent(&cnt[level + 1], total) : 0u;
@@ -727,7 +700,440 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_level(const nxb_bvh2_node
         if (ok) {
             uint32_t ks, kx, kb;
             emit_node<false>(cbx, tid, c, k, ic ? base + excl : 0u, pbase, c.count - ic, sz, out, prim_idx, n,
-                             node_count, capacity, work, REC ? nullptr : work2, flags, ks, kx, kb);
+                             capacity, work, flags, ks, kx, kb);
+        }
+    }
+}
+
+// ---- few launches (single builds of small meshes) ---------------------------
+//
+// One lane collapses one node; a block reserves the ids of its nodes' inner
+// children with one atomic add on the node counter and passes the children on
+// to itself, through LDS, while they fit its lanes, else to the next launch
+// through a queue in global memory. Launch l takes the queue positions
+// [cnt[1] + ... + cnt[l-1], +cnt[l]), counts that earlier launches completed,
+// so no lane ever waits on another (no polling, no spin limit); launch 0 is
+// the root.
+//
+// What bounds it is latency: a node costs its lane up to seven dependent record
+// loads (~1,300 cycles each with the choice of the next), then the slots and
+// the quantization. A level took 15 to 17 us as a launch of its own (counters,
+// queue and a cold L2 first), and a mesh has log2(n) of them, since a node's
+// largest child keeps half of its primitives. Inside a block a level is ~7 us.
+// The children of the node each lane collapses, in LDS (child t of lane i at
+// [t][i]): box, id (a leaf is an id below n, its primitive index) and
+// primitive count. Indexed by slot when they are read back, which in
+// registers would take a select over all eight per field.
+struct RecChildren {
+    float4 a[8][kBvh8Threads];  // lx, ly, lz, hx
+    uint4 b[8][kBvh8Threads];   // hy, hz, id, primitives
+};
+__device__ __forceinline__ void put_rec_child(RecChildren& ch, uint32_t t, uint32_t tid, const Box& b, uint32_t id,
+                                              uint32_t prims) {
+    ch.a[t][tid] = make_float4(b.lx, b.ly, b.lz, b.hx);
+    ch.b[t][tid] = make_uint4(__float_as_uint(b.hy), __float_as_uint(b.hz), id, prims);
+}
+__device__ __forceinline__ Box get_child_box(const RecChildren& ch, uint32_t t, uint32_t tid) {
+    const float4 a = ch.a[t][tid];
+    const uint2 c = *reinterpret_cast<const uint2*>(&ch.b[t][tid]);
+    Box b;
+    b.lx = a.x; b.ly = a.y; b.lz = a.z; b.hx = a.w; b.hy = __uint_as_float(c.x); b.hz = __uint_as_float(c.y);
+    return b;
+}
+
+// Collapse of internal node x (record x - n). Same push/pop order as
+// collapse_node; the node's box is the union of its children's (as H-PLOC
+// formed it, bit for bit). False for an id out of range.
+__device__ __forceinline__ bool collapse_children(const uint4* rec, uint32_t n, uint32_t node_count, uint32_t x, Box& pb,
+                                             uint32_t& count, uint32_t& inner, RecChildren& ch, uint32_t tid) {
+    if (x < n || x >= node_count) return false;
+    inner = 0;
+    uint32_t top = 0, msb = 0, cur = x;  // top: the last slot in use
+    for (;;) {
+        Box b0, b1;
+        uint32_t i0, i1, s0, s1;
+        load_rec8(rec, cur - n, b0, b1, i0, i1, s0, s1);
+        if (max(i0, i1) >= node_count) return false;
+        // the smaller child into the popped slot, the larger on top
+        const bool first_is_1 = !(box_area(b0) < box_area(b1));
+        const uint32_t na = first_is_1 ? i1 : i0, nb = first_is_1 ? i0 : i1;
+        if (top == 0) pb = box_union(b0, b1);
+        ++top;
+        put_rec_child(ch, msb, tid, first_is_1 ? b1 : b0, na, first_is_1 ? s1 : s0);
+        put_rec_child(ch, top, tid, first_is_1 ? b0 : b1, nb, first_is_1 ? s0 : s1);
+        inner |= (na >= n ? 1u << msb : 0u) | (nb >= n ? 1u << top : 0u);
+        if (inner == 0 || top == 7) break;
+        // the highest inner slot is expanded next: the larger child just
+        // pushed, else the smaller one, else an older child
+        msb = 31u - (uint32_t)__clz(inner);
+        cur = nb >= n ? nb : na;
+        if (cur < n) cur = ch.b[msb][tid].z;
+        inner &= ~(1u << msb);
+    }
+    count = top + 1;
+    return true;
+}
+
+// GreedyAssignment (WideConverter.cu:106-153): each child in push order takes
+// the free slot of the largest cost (GetCost 25-30), the lowest on a tie; with
+// no comparable cost the first free slot. Slots s and 7 - s have opposite
+// costs, bit for bit, so four sums give all eight. Nibble s of the result is
+// the child in slot s, 0xF none.
+__device__ __forceinline__ uint32_t greedy_assign(const Box& pb, const RecChildren& ch, uint32_t tid, uint32_t count) {
+    const float lowest = -3.402823466e+38f;
+    const float pcx = pb.lx + pb.hx, pcy = pb.ly + pb.hy, pcz = pb.lz + pb.hz;
+    uint32_t assign = 0xFFFFFFFFu, free_slots = 0xFFu;
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+        const Box cb = get_child_box(ch, k, tid);
+        const float ox = pcx - (cb.hx + cb.lx), oy = pcy - (cb.hy + cb.ly), oz = pcz - (cb.hz + cb.lz);
+        const float p = ox + oy, m = ox - oy;
+        const float c[4] = {p + oz, p - oz, m + oz, m - oz};
+        // the largest cost of the free slots (a NaN is dropped), then the
+        // lowest slot that has it
+        float cost[8], most = lowest;
+#pragma unroll
+        for (uint32_t s = 0; s < 8; ++s) {
+            cost[s] = (free_slots & (1u << s)) ? (s < 4 ? c[s & 3] : -c[(7 - s) & 3]) : lowest;
+            most = fmaxf(most, cost[s]);
+        }
+        uint32_t best = 8u;
+#pragma unroll
+        for (int s = 7; s >= 0; --s) best = cost[s] == most ? (uint32_t)s : best;
+        if (!(most > lowest)) best = (uint32_t)__builtin_ctz(free_slots | 0x100u);
+        if (k < count) {
+            free_slots &= ~(1u << best);
+            assign = with_nib(assign, best, k);
+        }
+    }
+    return assign;
+}
+
+// Auction slots (auction_assign) of the same children.
+__device__ __forceinline__ uint32_t auction_slots(const Box& pb, const RecChildren& ch, uint32_t tid, uint32_t count) {
+    const float pcx = pb.lx + pb.hx, pcy = pb.ly + pb.hy, pcz = pb.lz + pb.hz;
+    float ox[8], oy[8], oz[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+        ox[k] = oy[k] = oz[k] = 0.0f;
+        if (k < count) {
+            const Box cb = get_child_box(ch, k, tid);
+            ox[k] = pcx - (cb.lx + cb.hx);
+            oy[k] = pcy - (cb.ly + cb.hy);
+            oz[k] = pcz - (cb.lz + cb.hz);
+        }
+    }
+    return auction_assign(pb, ox, oy, oz, count);
+}
+
+// What the lanes that emit a node need to know of it.
+struct RecNodes {
+    float4 a[kBvh8Threads];  // box: lx, ly, lz, hx
+    uint4 b[kBvh8Threads];   // hy, hz, children | inner-child bits << 8, first primitive
+    uint2 c[kBvh8Threads];   // BVH8 id, inner children of the block's earlier nodes
+};
+
+// Work items passed on inside a block.
+struct BlockQueue {
+    uint32_t x[kBvh8Threads], base[kBvh8Threads], id[kBvh8Threads];
+};
+
+// Where a level's children go: ids[0..] in the order of the nodes' slots, to
+// the block's queue (keep) or to the queue positions from `queue` on.
+struct ChildSink {
+    BlockQueue* bq;
+    bool keep;
+    uint32_t ids, queue, level;  // level: of the children
+    uint64_t *work, *work2;
+    uint32_t capacity, n;
+
+    __device__ __forceinline__ bool put(uint32_t at, uint32_t x, uint32_t base, uint32_t prims) const {
+        const uint32_t cid = ids + at;
+        bool good = cid < capacity && prims >= 2 && base + prims <= n;
+        const uint32_t cx = good ? x : kInvalid;  // an invalid item is flagged, not followed
+        if (keep) {
+            bq->x[at] = cx;
+            bq->base[at] = base;
+            bq->id[at] = cid;
+        } else if (queue + at < capacity) {
+            work[queue + at] = ((uint64_t)base << 32) | cx;
+            work2[queue + at] = ((uint64_t)level << 32) | cid;
+        } else {
+            good = false;
+        }
+        return good;
+    }
+};
+
+// Exponents of a node's quantization grid (CreateBVH8Node, WideConverter.cu:156-206).
+__device__ __forceinline__ uint32_t grid_exponents(const Box& pb, float& ix, float& iy, float& iz) {
+    const float qstep = 1.0f / 255.0f;
+    const uint32_t e0 = ceil_log2((pb.hx - pb.lx) * qstep) & 0xFFu;
+    const uint32_t e1 = ceil_log2((pb.hy - pb.ly) * qstep) & 0xFFu;
+    const uint32_t e2 = ceil_log2((pb.hz - pb.lz) * qstep) & 0xFFu;
+    ix = inv_pow2(e0);
+    iy = inv_pow2(e1);
+    iz = inv_pow2(e2);
+    return e0 | (e1 << 8) | (e2 << 16);
+}
+
+// Emits the node of one lane: primIdx entries of its leaves, work items of its
+// inner children, the 80 bytes. Primitive ranges are fixed top-down: a node's
+// leaves take the front of its range, then each inner child, in slot order, a
+// range of its primitive count.
+__device__ __forceinline__ bool emit_lane(const RecChildren& ch, uint32_t tid, const Box& pb, uint32_t count,
+                                          uint32_t inner, uint32_t assign, uint32_t base, uint32_t id, uint32_t excl,
+                                          const ChildSink& sink, nxb_bvh8_node* out, uint32_t* prim_idx) {
+    const uint32_t ic = (uint32_t)__popc(inner), leaf_count = count - ic;
+    float ix, iy, iz;
+    const uint32_t e = grid_exponents(pb, ix, iy, iz);
+    uint32_t next_base = base + leaf_count, leaves = 0, nth = 0, im = 0;
+    uint32_t meta[2] = {0, 0}, qlx[2] = {0, 0}, qly[2] = {0, 0}, qlz[2] = {0, 0};
+    uint32_t qhx[2] = {0, 0}, qhy[2] = {0, 0}, qhz[2] = {0, 0};
+    bool good = true;
+#pragma unroll
+    for (uint32_t s = 0; s < 8; ++s) {
+        // (an empty slot computes on child 7's words and keeps zeros)
+        const uint32_t a = nib(assign, s) & 7u;
+        const bool used = nib(assign, s) != 0xFu, in = used && ((inner >> a) & 1u);
+        const float4 ca = ch.a[a][tid];
+        const uint4 cb = ch.b[a][tid];
+        const uint32_t w = s >> 2, sh = 8 * (s & 3);
+        auto put = [&](uint32_t* q, uint32_t v) { q[w] |= used ? v << sh : 0u; };
+        put(qlx, q_floor((ca.x - pb.lx) * ix));
+        put(qly, q_floor((ca.y - pb.ly) * iy));
+        put(qlz, q_floor((ca.z - pb.lz) * iz));
+        put(qhx, q_ceil((ca.w - pb.lx) * ix));
+        put(qhy, q_ceil((__uint_as_float(cb.x) - pb.ly) * iy));
+        put(qhz, q_ceil((__uint_as_float(cb.y) - pb.lz) * iz));
+        put(meta, (1u << 5) | (in ? 24u + s : leaves));
+        if (in) {
+            im |= 1u << s;
+            good &= sink.put(excl + nth, cb.z, next_base, cb.w);
+            next_base += cb.w;
+            ++nth;
+        } else if (used) {
+            if (base + leaves < sink.n) prim_idx[base + leaves] = cb.z;
+            else good = false;
+            ++leaves;
+        }
+    }
+    uint4* o = reinterpret_cast<uint4*>(out + id);
+    o[0] = make_uint4(__float_as_uint(pb.lx), __float_as_uint(pb.ly), __float_as_uint(pb.lz), e | (im << 24));
+    o[1] = make_uint4(ic ? sink.ids + excl : 0u, leaf_count ? base : 0u, meta[0], meta[1]);
+    o[2] = make_uint4(qlx[0], qlx[1], qly[0], qly[1]);
+    o[3] = make_uint4(qlz[0], qlz[1], qhx[0], qhx[1]);
+    o[4] = make_uint4(qhy[0], qhy[1], qhz[0], qhz[1]);
+    return good;
+}
+
+// Value of another lane of the same eight: lane ^ 1, lane ^ 2, and (for values
+// alike in each four lanes) lane ^ 4.
+template <int CTRL>
+__device__ __forceinline__ float dpp_f(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141;
+// Lane K of each eight (ds_swizzle, bit-mask mode: lane & 0x18 | K).
+template <int K>
+__device__ __forceinline__ float lane_of_8(float v) {
+    return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (K << 5) | 0x18));
+}
+
+// Slot choice of child K (greedy_assign): lane s holds slot s (mine: its child,
+// 8 while free) and, as child s, the offsets ox, oy, oz.
+template <uint32_t K>
+__device__ __forceinline__ void greedy_step(float ox, float oy, float oz, uint32_t s, uint32_t count, uint64_t lower,
+                                            uint32_t& mine) {
+    const float lowest = -3.402823466e+38f;
+    const float kx = lane_of_8<K>(ox), ky = lane_of_8<K>(oy), kz = lane_of_8<K>(oz);
+    const float cost = ((s & 4u ? -kx : kx) + (s & 2u ? -ky : ky)) + (s & 1u ? -kz : kz);
+    const bool free_slot = mine == 8u;
+    float most = free_slot ? fmaxf(cost, lowest) : lowest;
+    most = fmaxf(most, dpp_f<kDppXor1>(most));
+    most = fmaxf(most, dpp_f<kDppXor2>(most));
+    most = fmaxf(most, dpp_f<kDppHalfMirror>(most));
+    const bool fits = K < count && free_slot && (cost == most || !(most > lowest));
+    if (fits && (ballot(fits) & lower) == 0) mine = K;
+    if constexpr (K < 7) greedy_step<K + 1>(ox, oy, oz, s, count, lower, mine);
+}
+
+// Emits `nodes` nodes of the block, eight lanes per node and one slot per lane
+// (greedy slots): the same results as greedy_assign and emit_lane. A wave takes
+// eight nodes at a time; their 640 bytes are put together in LDS.
+__device__ __forceinline__ bool emit_groups(const RecChildren& ch, const RecNodes& nd, uint32_t nodes,
+                                            uint8_t (*stage)[8 * sizeof(nxb_bvh8_node)], const ChildSink& sink,
+                                            nxb_bvh8_node* out, uint32_t* prim_idx) {
+    const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63u, s = lane & 7u, g = lane >> 3;
+    const uint64_t lower = ((1ull << lane) - 1ull) & (0xFFull << (lane & 56u));  // earlier lanes of the eight
+    uint8_t* st = stage[w] + g * sizeof(nxb_bvh8_node);
+    bool good = true;
+    for (uint32_t j0 = w * 8; j0 < nodes; j0 += kBvh8Threads / 8) {
+        const uint32_t j = min(j0 + g, nodes - 1);
+        const float4 na = nd.a[j];
+        const uint4 nb = nd.b[j];
+        const uint2 nc = nd.c[j];
+        const Box pb = {na.x, na.y, na.z, na.w, __uint_as_float(nb.x), __uint_as_float(nb.y)};
+        const uint32_t count = j0 + g < nodes ? nb.z & 0xFFu : 0u, inner = nb.z >> 8, base = nb.w;
+        // as child s
+        uint32_t mine = 8u;
+        {
+            const Box cb = get_child_box(ch, s, j);
+            greedy_step<0>((pb.lx + pb.hx) - (cb.hx + cb.lx), (pb.ly + pb.hy) - (cb.hy + cb.ly),
+                           (pb.lz + pb.hz) - (cb.hz + cb.lz), s, count, lower, mine);
+        }
+        // as slot s
+        const bool used = mine < 8u, in = used && ((inner >> (mine & 7u)) & 1u);
+        const float4 ca = ch.a[mine & 7u][j];
+        const uint4 cb = ch.b[mine & 7u][j];
+        const uint32_t im = (uint32_t)(ballot(in) >> (lane & 56u)) & 0xFFu;
+        const uint32_t lm = (uint32_t)(ballot(used && !in) >> (lane & 56u)) & 0xFFu;
+        const uint32_t leaf_count = (uint32_t)__popc(lm), leaf = bits_below(lm, s);
+        uint32_t before = in ? cb.w : 0u;  // primitives of the inner slots up to this one
+#pragma unroll
+        for (uint32_t off = 1; off < 8; off <<= 1) {
+            const uint32_t v = (uint32_t)__shfl_up((int)before, off);
+            before += s >= off ? v : 0u;
+        }
+        if (in) good &= sink.put(nc.y + bits_below(im, s), cb.z, base + leaf_count + before - cb.w, cb.w);
+        if (used && !in) {
+            if (base + leaf < sink.n) prim_idx[base + leaf] = cb.z;
+            else good = false;
+        }
+        float ix, iy, iz;
+        const uint32_t e = grid_exponents(pb, ix, iy, iz);
+        auto put = [&](uint32_t k, uint32_t v) { st[24 + 8 * k + s] = (uint8_t)(used ? v : 0u); };
+        put(0, (1u << 5) | (in ? 24u + s : leaf));
+        put(1, q_floor((ca.x - pb.lx) * ix));
+        put(2, q_floor((ca.y - pb.ly) * iy));
+        put(3, q_floor((ca.z - pb.lz) * iz));
+        put(4, q_ceil((ca.w - pb.lx) * ix));
+        put(5, q_ceil((__uint_as_float(cb.x) - pb.ly) * iy));
+        put(6, q_ceil((__uint_as_float(cb.y) - pb.lz) * iz));
+        if (s == 0) {
+            uint2* h = reinterpret_cast<uint2*>(st);
+            h[0] = make_uint2(__float_as_uint(pb.lx), __float_as_uint(pb.ly));
+            h[1] = make_uint2(__float_as_uint(pb.lz), e | (im << 24));
+            h[2] = make_uint2(im ? sink.ids + nc.y : 0u, leaf_count ? base : 0u);
+        }
+        wave_lds_sync();
+        const uint32_t k = lane / 5u, part = lane - 5u * k;  // 16 bytes of node j0 + k
+        if (k < 8 && j0 + k < nodes && (nd.b[j0 + k].z & 0xFFu) != 0)
+            reinterpret_cast<uint4*>(out + nd.c[j0 + k].x)[part] =
+                *reinterpret_cast<const uint4*>(stage[w] + k * sizeof(nxb_bvh8_node) + part * 16);
+        wave_lds_sync();
+    }
+    return good;
+}
+
+// Primitives up to which a build takes the kernel below; above, one launch per
+// level (three blocks of 48 KB LDS per CU where this one has two). Collapse
+// stage, us, launches that follow subtrees / a launch per level, on a surface,
+// blobs and slivers: 82/147, 65/109, 66/110 at 2,003; 119/201, 113/193, 101/169
+// at 48K; 134/207, 165/245, 140/209 at 300K; 240/254, 262/300, 244/265 at 1.1M;
+// 269/296, 318/343, 280/307 at 2M; 345/357, 415/388, 325/337 at 3M.
+constexpr uint32_t kSmallPrims = 1u << 21;
+bool bvh8_small(uint32_t n) { return n <= kSmallPrims; }
+
+// Levels that a block follows while the queue grows, by queued nodes: a node's
+// children hold about 1/2, 1/4, 1/8, ... of its primitives (the larger child is
+// expanded each time), so a block that went on alone with a large one would
+// hold up the launch (300K triangles: 181 to 230 us without the limits). 4096
+// and 16384 instead measured within 5%.
+constexpr uint32_t kThreeLevelNodes = 2048, kTwoLevelNodes = 32768;
+
+// Nodes of a block up to which eight lanes emit a node (emit_groups: ~2,000
+// cycles per 32 nodes of a block; greedy_assign and emit_lane: ~8,500 cycles
+// however few). 32 and 96 measured alike, 256 a tenth slower.
+constexpr uint32_t kGroupNodes = 96;
+
+// work[q] = (first primitive << 32 | BVH2 id), work2[q] = (level << 32 | BVH8
+// id) of queue position q. alloc counts the nodes below the root (the root is
+// node 0), zero before launch 0.
+template <uint32_t SLOT>
+__global__ __launch_bounds__(kBvh8Threads) void k_bvh8_collapse(const uint4* __restrict__ rec, uint32_t n,
+                                                                uint32_t node_count, nxb_bvh8_node* __restrict__ out,
+                                                                uint32_t* __restrict__ prim_idx, uint32_t capacity,
+                                                                uint64_t* work, uint64_t* work2, uint32_t* cnt,
+                                                                uint32_t launch, uint32_t* alloc, uint32_t* flags) {
+    __shared__ RecChildren ch;
+    __shared__ RecNodes nd;
+    __shared__ BlockQueue bq;
+    __shared__ __attribute__((aligned(16))) uint8_t stage[kBvh8Threads / 64][8 * sizeof(nxb_bvh8_node)];
+    __shared__ uint32_t scan_tmp[kBvh8Threads / 64];
+    __shared__ uint32_t sids, squeue, slevel;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t m = launch == 0 ? 1u : min(cnt[launch], capacity);
+    if (m == 0) return;
+    uint32_t lo = 0;
+    for (uint32_t j = 1; j < launch; ++j) lo += cnt[j];
+    const uint32_t hi = launch == 0 ? 0u : lo + m;
+    // one share per block where the grid holds all items (the block then
+    // follows its subtrees), else whole blocks of items, one level of each
+    const bool follow = m <= gridDim.x * kBvh8Threads;
+    // levels before the rest goes to the queue: all in the first launch and
+    // once the queue shrinks, else few enough that no block runs on alone
+    uint32_t left = kMaxLevels;
+    if (launch != 0 && (launch == 1 || m >= cnt[launch - 1])) left = m <= kThreeLevelNodes ? 3u : m <= kTwoLevelNodes ? 2u : 1u;
+    const uint32_t per = follow ? (m + gridDim.x - 1) / gridDim.x : (uint32_t)kBvh8Threads;
+    for (uint32_t i0 = blockIdx.x * per; i0 < m; i0 += gridDim.x * per) {
+        uint32_t nodes = min(per, m - i0);
+        uint32_t x = node_count - 1, base = 0, id = 0, level = 0;  // the root
+        if (launch != 0) {
+            if (tid == 0) slevel = 0;
+            __syncthreads();
+            const bool has = tid < nodes && lo + i0 + tid < capacity;
+            const uint64_t v = has ? work[lo + i0 + tid] : (uint64_t)kInvalid, v2 = has ? work2[lo + i0 + tid] : 0ull;
+            x = (uint32_t)v;
+            base = (uint32_t)(v >> 32);
+            id = (uint32_t)v2;
+            atomicMax(&slevel, (uint32_t)(v2 >> 32));
+            __syncthreads();
+            level = slevel;  // the deepest of the share: a bound for its levels
+        }
+        for (;;) {
+            const bool has = tid < nodes;
+            Box pb = {0, 0, 0, 0, 0, 0};
+            uint32_t count = 0, inner = 0;
+            const bool ok = has && level < kMaxLevels && id < capacity &&
+                            collapse_children(rec, n, node_count, x, pb, count, inner, ch, tid);
+            bool good = ok || !has;
+            // the ids of the children, reserved while their slots are chosen
+            const uint32_t ic = ok ? (uint32_t)__popc(inner) : 0u;
+            uint32_t total = 0;
+            const uint32_t excl = block_scan_256(ic, scan_tmp, &total);
+            const bool keep = follow && --left != 0 && total <= (uint32_t)kBvh8Threads;
+            const bool groups = SLOT == NXB_SLOT_GREEDY && nodes <= kGroupNodes;
+            if (tid == 0) sids = total ? 1u + atomic_add_agent(alloc, total) : 0u;
+            if (tid == 64) squeue = total && !keep ? hi + atomic_add_agent(&cnt[launch + 1], total) : 0u;
+            uint32_t assign = 0xFFFFFFFFu;
+            if (groups) {
+                if (has) {
+                    nd.a[tid] = make_float4(pb.lx, pb.ly, pb.lz, pb.hx);
+                    nd.b[tid] = make_uint4(__float_as_uint(pb.hy), __float_as_uint(pb.hz),
+                                           ok ? count | (inner << 8) : 0u, base);
+                    nd.c[tid] = make_uint2(id, excl);
+                }
+            } else if (ok) {
+                assign = SLOT == NXB_SLOT_AUCTION ? auction_slots(pb, ch, tid, count)
+                                                  : greedy_assign(pb, ch, tid, count);
+            }
+            __syncthreads();
+            const ChildSink sink{&bq, keep, sids, squeue, level + 1, work, work2, capacity, n};
+            if (groups)
+                good &= emit_groups(ch, nd, nodes, stage, sink, out, prim_idx);
+            else if (ok)
+                good &= emit_lane(ch, tid, pb, count, inner, assign, base, id, excl, sink, out, prim_idx);
+            if (!good) atomic_or_agent(flags, kFlagBadIndex);
+            __syncthreads();  // the block's queue is written, sids and squeue are read
+            if (!keep || total == 0) break;
+            nodes = total;
+            ++level;
+            if (tid < nodes) {
+                x = bq.x[tid];
+                base = bq.base[tid];
+                id = bq.id[tid];
+            }
         }
     }
 }
@@ -1052,9 +1458,9 @@ hipError_t launch_bvh8_forest(const nxb_bvh2_node* bvh2, uint32_t n, uint32_t tr
     return hipGetLastError();
 }
 
-hipError_t launch_bvh8_levels(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_node* out, uint32_t* prim_idx,
-                              uint32_t capacity, Bvh8Scratch sc, uint32_t* cnt, uint32_t from, uint32_t count,
-                              hipStream_t s) {
+hipError_t launch_bvh8_collapse(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_node* out, uint32_t* prim_idx,
+                                uint32_t capacity, Bvh8Scratch sc, uint32_t* cnt, uint32_t* alloc, uint32_t from,
+                                uint32_t count, hipStream_t s) {
     if (n == 0) return hipSuccess;
     if (n == 1) {
         if (from == 0)
@@ -1062,25 +1468,32 @@ hipError_t launch_bvh8_levels(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_no
                                prim_idx, capacity, sc.work, sc.ctr, sc.grab, sc.nsize, sc.flags, 1u);
         return hipGetLastError();
     }
-    const bool rec = sc.rec8 != nullptr;
-    if (!rec && !sc.work2) return hipErrorInvalidValue;
+    if (!sc.rec8 || !sc.work2) return hipErrorInvalidValue;
     const bool auction = sc.slot_mode == NXB_SLOT_AUCTION;
+    if (bvh8_small(n)) {
+        auto kernel = auction ? k_bvh8_collapse<NXB_SLOT_AUCTION> : k_bvh8_collapse<NXB_SLOT_GREEDY>;
+        // two blocks of 80 KB LDS per CU
+        const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 2u);
+        const uint32_t end = min(from + count, kMaxLevels);
+        for (uint32_t l = from; l < end; ++l)
+            hipLaunchKernelGGL(kernel, dim3(l == 0 ? 1u : grid), dim3(kBvh8Threads), 0, s, sc.rec8, n, 2 * n - 1, out,
+                               prim_idx, capacity, sc.work, sc.work2, cnt, l, alloc, sc.flags);
+        return hipGetLastError();
+    }
     // three 48 KB blocks per CU; a level of m nodes uses ceil(m / 256) blocks
     const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 3u);
     if (from == 0) {
-        auto top = auction ? (rec ? k_bvh8_top<NXB_SLOT_AUCTION, true> : k_bvh8_top<NXB_SLOT_AUCTION, false>)
-                           : (rec ? k_bvh8_top<NXB_SLOT_GREEDY, true> : k_bvh8_top<NXB_SLOT_GREEDY, false>);
-        hipLaunchKernelGGL(top, dim3(1), dim3(kBvh8Threads), 0, s, bvh2, n, 2 * n - 1, out, prim_idx, capacity,
-                           sc.work, sc.work2, cnt, sc.nsize, sc.flags, sc.rec8);
+        hipLaunchKernelGGL(auction ? k_bvh8_top<NXB_SLOT_AUCTION> : k_bvh8_top<NXB_SLOT_GREEDY>, dim3(1),
+                           dim3(kBvh8Threads), 0, s, sc.rec8, n, 2 * n - 1, out, prim_idx, capacity, sc.work, cnt,
+                           sc.flags);
         from = kBvh8TopLevels;
         count = count > kBvh8TopLevels ? count - kBvh8TopLevels : 0u;
     }
-    auto level = auction ? (rec ? k_bvh8_level<NXB_SLOT_AUCTION, true> : k_bvh8_level<NXB_SLOT_AUCTION, false>)
-                         : (rec ? k_bvh8_level<NXB_SLOT_GREEDY, true> : k_bvh8_level<NXB_SLOT_GREEDY, false>);
+    auto level = auction ? k_bvh8_level<NXB_SLOT_AUCTION> : k_bvh8_level<NXB_SLOT_GREEDY>;
     const uint32_t end = min(from + count, kMaxLevels);
     for (uint32_t l = from; l < end; ++l)
-        hipLaunchKernelGGL(level, dim3(grid), dim3(kBvh8Threads), 0, s, bvh2, n, 2 * n - 1, out, prim_idx, capacity,
-                           sc.work, sc.work2, cnt, l, sc.nsize, sc.flags, sc.rec8);
+        hipLaunchKernelGGL(level, dim3(grid), dim3(kBvh8Threads), 0, s, sc.rec8, n, 2 * n - 1, out, prim_idx, capacity,
+                           sc.work, cnt, l, sc.flags);
     return hipGetLastError();
 }
 
@@ -1097,21 +1510,6 @@ __global__ void k_bvh8_level_total(const uint32_t* cnt, uint32_t levels, unsigne
     for (uint32_t l = 0; l < levels; ++l) total += cnt[l];
     *ctr = total;
     if (cnt[levels] != 0) atomic_or_agent(flags, kFlagDeeper);
-}
-
-hipError_t launch_bvh8_forest_levels(const nxb_bvh2_node* bvh2, uint32_t n, uint32_t trees, nxb_bvh8_node* out,
-                                     uint32_t* prim_idx, uint32_t capacity, uint32_t levels, Bvh8Scratch sc,
-                                     uint32_t* cnt, hipStream_t s) {
-    if (n < 2 || levels == 0 || levels > kMaxLevels || !sc.work2) return hipErrorInvalidValue;
-    const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 3u);
-    hipLaunchKernelGGL(k_bvh8_forest_level_init, dim3(1), dim3(128), 0, s, cnt, trees);
-    auto level = sc.slot_mode == NXB_SLOT_AUCTION ? k_bvh8_level<NXB_SLOT_AUCTION, false>
-                                                  : k_bvh8_level<NXB_SLOT_GREEDY, false>;
-    for (uint32_t l = 0; l < levels; ++l)
-        hipLaunchKernelGGL(level, dim3(grid), dim3(kBvh8Threads), 0, s, bvh2, n, 2 * n - trees, out, prim_idx,
-                           capacity, sc.work, sc.work2, cnt, l, sc.nsize, sc.flags, static_cast<const uint4*>(nullptr));
-    hipLaunchKernelGGL(k_bvh8_level_total, dim3(1), dim3(1), 0, s, cnt, levels, sc.ctr, sc.flags);
-    return hipGetLastError();
 }
 
 hipError_t launch_bvh8_tree_levels(const nxb_bvh2_node* bvh2, uint32_t n, uint32_t trees, nxb_bvh8_node* out,
@@ -1136,16 +1534,21 @@ hipError_t launch_bvh8_tree_levels(const nxb_bvh2_node* bvh2, uint32_t n, uint32
     return hipGetLastError();
 }
 
-bool bvh8_levels_done(uint32_t n, const uint32_t* cnt_host, uint32_t launched, uint32_t* node_total) {
-    if (n <= 1) {
-        *node_total = n;
-        return true;
+uint32_t bvh8_launches(uint32_t n, const uint32_t* cnt_host, uint32_t below_host, uint32_t launched,
+                       uint32_t* node_total) {
+    *node_total = n;
+    if (n <= 1) return 1;
+    // the counts of launches (levels) up to `launched` are final; an empty
+    // one ends the tree
+    uint32_t total = bvh8_small(n) ? 0u : 1u;
+    for (uint32_t l = 1; l <= launched; ++l) {
+        if (cnt_host[l] == 0) {
+            *node_total = bvh8_small(n) ? 1u + below_host : total;
+            return l;
+        }
+        total += cnt_host[l];
     }
-    // counts of levels 0..launched are final; an empty one ends the tree
-    uint32_t total = 0, l = 0;
-    for (; l <= launched && l <= kMaxLevels && cnt_host[l] != 0; ++l) total += cnt_host[l];
-    *node_total = total;
-    return l <= launched;
+    return 0;
 }
 
 hipError_t launch_bvh8(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_node* out, uint32_t* prim_idx,

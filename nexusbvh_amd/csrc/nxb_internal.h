@@ -63,11 +63,10 @@ struct Bvh8Scratch {
     uint32_t* grab;           // work grab counter (own cache line)
     uint32_t* flags;
     const uint32_t* nsize;    // [n-1] primitives under each internal BVH2 node
-    uint64_t* work2;          // [capacity] (right << 32 | left) children of each work item's BVH2 node
-                              // (level-synchronous collapse only)
+    uint64_t* work2;          // [capacity] second word of a work item: (right << 32 | left) children of its BVH2
+                              // node (batches), (level << 32 | BVH8 id) (one mesh)
     uint32_t slot_mode;       // nxb_slot_assignment of the child slots
-    const uint4* rec8 = nullptr;  // wide records of the internal nodes (level-synchronous collapse of
-                                  // one mesh): read instead of the BVH2 nodes, nsize and work2
+    const uint4* rec8 = nullptr;  // wide records of the internal nodes (one mesh)
 };
 
 // indices (nullable): three vertex indices per triangle into prims, which
@@ -137,30 +136,26 @@ hipError_t launch_subtree_sizes(const nxb_bvh2_node* bvh2, uint32_t n, uint32_t*
                                 uint32_t* nsize, uint32_t* flags, hipStream_t s);
 hipError_t launch_bvh8_run(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_node* out, uint32_t* prim_idx,
                            uint32_t capacity, uint32_t spin_limit, Bvh8Scratch sc, hipStream_t s);
-// Level-synchronous BVH8 of one BVH2 (root 2n-2): enqueues the kernels of
-// levels [from, from + count) (from == 0 also initializes; count is then at
-// least kBvh8TopLevels). cnt: kBvh8LevelWords
-// device words of level counters. After reading them back (levels
-// 0..launched are final), bvh8_levels_done tells whether the tree is
-// complete and sets the node count; if not, enqueue more levels.
+// BVH8 of one mesh from its wide records (sc.rec8; n == 1: from the leaf):
+// enqueues the launches [from, from + count), of which the first is at least
+// kBvh8TopLevels long. cnt: kBvh8LevelWords device words of level or queue
+// counters; alloc: one word, the nodes below the root of a small mesh; both
+// zero before the first launch. From the words read back, bvh8_launches tells
+// how many launches the tree took and its node count; 0: more are needed. A
+// tree of more than kBvh8LevelWords - 1 levels sets the bad-index flag.
 constexpr uint32_t kBvh8LevelWords = 97;
-constexpr uint32_t kBvh8FirstLevels = 24;
-constexpr uint32_t kBvh8TopLevels = 3;  // levels 0..2 run in one single-block launch (from == 0)
-hipError_t launch_bvh8_levels(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_node* out, uint32_t* prim_idx,
-                              uint32_t capacity, Bvh8Scratch sc, uint32_t* cnt, uint32_t from, uint32_t count,
-                              hipStream_t s);
-bool bvh8_levels_done(uint32_t n, const uint32_t* cnt_host, uint32_t launched, uint32_t* node_total);
-// Level-synchronous BVH8 of a forest (roots in work[0..trees), as for
-// launch_bvh8_forest) with a fixed number of levels; the node total ends in
-// the low word of *sc.ctr, and a tree deeper than `levels` sets the
-// bad-index flag.
-hipError_t launch_bvh8_forest_levels(const nxb_bvh2_node* bvh2, uint32_t n, uint32_t trees, nxb_bvh8_node* out,
-                                     uint32_t* prim_idx, uint32_t capacity, uint32_t levels, Bvh8Scratch sc,
-                                     uint32_t* cnt, hipStream_t s);
-// As launch_bvh8_forest_levels for the forest of a batch (tree t's root is
-// its last internal node, mesh_lo[] as for launch_hploc_batch), but each
-// tree t writes its own contiguous BVH8 (root 0, tree-local child and
-// primitive bases) to out + info[t].z with at most info[t].w nodes, and its
+constexpr uint32_t kBvh8TopLevels = 3;  // large meshes: levels 0..2 run in one single-block launch
+bool bvh8_small(uint32_t n);            // few launches that follow subtrees, else one launch per level
+hipError_t launch_bvh8_collapse(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_node* out, uint32_t* prim_idx,
+                                uint32_t capacity, Bvh8Scratch sc, uint32_t* cnt, uint32_t* alloc, uint32_t from,
+                                uint32_t count, hipStream_t s);
+uint32_t bvh8_launches(uint32_t n, const uint32_t* cnt_host, uint32_t below_host, uint32_t launched,
+                       uint32_t* node_total);
+// Level-synchronous BVH8s of the forest of a batch (tree t's root is its last
+// internal node, mesh_lo[] as for launch_hploc_batch) with a fixed number of
+// levels; the queued total ends in the low word of *sc.ctr, and a tree deeper
+// than `levels` sets kFlagDeeper. Each tree t writes its own contiguous BVH8
+// (root 0, tree-local child and primitive bases) to out + info[t].z with at most info[t].w nodes, and its
 // primitives to prim_idx + info[t].x (info[t].y of them). Levels
 // 0..kTreeTopLevels-1 run in one launch, a block per few trees; their level
 // counters stay 0, so the depth of the forest is kTreeTopLevels plus the
