@@ -965,7 +965,7 @@ nxb_status nxb_build_hploc(const void* d_sorted_keys, uint32_t* d_sorted_values,
     if (d) NXB_TRY(ws_wait(*d, s));
     NXB_HIP(launch_fill_u32(w.hdr(), 0u, kHdrHplocChunks + kHplocCounterWords, s));
     NXB_HIP(launch_fill_u32(w.parent(), kInvalid, n, s));
-    HplocScratch hs{w.parent(), w.recs(), w.csizes(), w.moved(), w.moved_parent(), w.moved_size(), w.nsize(),
+    HplocScratch hs{w.parent(), w.recs(), w.csizes(), w.moved(), w.moved_parent(), w.moved_size(), nullptr,
                     w.flags(), w.hploc_chunks()};
     NXB_HIP(launch_hploc(d_sorted_keys, key_bits, d_sorted_values, n, d_nodes, cfg.merge_mode, radius_params(cfg),
                          cfg.hploc_blocks_per_cu, hs, s));

@@ -190,7 +190,8 @@ __device__ __forceinline__ uint32_t mask_rank(uint64_t m) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-__device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
+// (__ballot takes an int: the condition would go through a select and a compare)
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
 
 // Adds one count per active lane to the LDS counter sh[d]. Digits of
 // neighbouring inputs are often equal across the whole wave (high Morton

@@ -54,7 +54,18 @@
 // BVH8 builds of one mesh write each internal node as a 64-byte wide record
 // (both children's boxes, ids and primitive counts) for the collapse, in
 // place of its BVH2 node and size: at 28.1M triangles the records cost
-// H-PLOC 0.21 ms and save the collapse 0.64 ms.
+// H-PLOC 0.25 ms and save the collapse 0.64 ms.
+//
+// What bounds it: up to about a million primitives the chain of merges to the
+// root (a step is an exchange, key and record loads, 2 to 5 rounds of search
+// and merge, and the stores' completion: some 3 us each); above, the vector
+// units (60-70% busy) and requests to memory. Times in us before and after the
+// last changes (search, merge rounds, loads and stores below):
+//   BVH2, 12.7M 32-bit keys     1550 -> 1300    BVH8, 28.1M   3172 -> 2570
+//   BVH8, 300K                   177 -> 159     BVH8, 2,003     86 -> 77
+//   2,048 meshes, 19.7M         1890 -> 1690
+#include <type_traits>
+
 #include "device_common.h"
 #include "nxb_internal.h"
 
@@ -66,116 +77,143 @@ constexpr int kHplocThreads = 128;
 constexpr int kHplocWaves = kHplocThreads / 64;
 constexpr int kMaxRadius = 16;
 
+constexpr uint32_t kInfBits = 0x7F800000u;  // areas at or above it as bits: infinite, NaN or negative
 constexpr uint32_t kMoved = 0xFFFFFFFDu;  // temporary id of the node that retired n-1
 constexpr uint32_t kRefill = 32;           // free lanes that make a wave start new positions
-// Resident blocks per CU (6 waves per SIMD): at 28.1M primitives H-PLOC took
-// 4.5 ms with 12 to 14, 4.9 ms with 8 and 5.1 ms with 16.
+// Resident blocks per CU (6 waves per SIMD): at 28.1M primitives a BVH8 build's
+// H-PLOC takes 2.60 ms with 12, 2.84 with 10, 3.04 with 8; 14 (72 registers)
+// took 3.73.
 constexpr uint32_t kHplocBlocksPerCu = kHplocMaxBlocksPerCu;
 constexpr uint32_t kHplocMaxChunk = 1024;
+// Primitives from which wide records go through the stage: below, its LDS round
+// trip lengthens every merge round (1.1M primitives: 266 us direct, 284 staged;
+// 2,003: 77 and 84); above, requests for memory bound the kernel (16M blobs:
+// 1944 and 1709 us; uniform 1806 and 1436). The two meet at 2.5M to 4M. BVH2
+// nodes, two stores of 16 bytes, gained nothing staged (12.7M: 1300 and 1298).
+constexpr uint32_t kStagedPrims = 3u << 20;
 constexpr uint32_t kHplocRegions = 8;         // XCDs of the chip
 constexpr uint32_t kHplocCounterStride = 32;  // words between region counters (own 128-byte line)
 
+// What a build keeps besides the BVH2: nothing more; the primitive count of
+// every internal node; or a wide record in place of every internal node, stored
+// by the lane that merges or (kKeepStaged) through LDS by four lanes each.
+// Without counts a merge neither loads, carries nor stores them.
+enum HplocKeep { kKeepNodes, kKeepSizes, kKeepRecords, kKeepStaged };
+
+// Wide records of one merge round on their way to memory (kKeepStaged).
+// Record r's quarter q stands at column (q + r / 4) % 4 of row r, so that 16
+// lanes storing one quarter each cover all banks.
+struct RecStage {
+    uint4 q[32 * 4];
+    uint32_t at[32];  // record index, or kInvalid: nothing to store
+};
+struct NoStage {};
+
+template <int GW, HplocKeep KEEP>
 struct HplocLds {
-    // cluster boxes, 32 bytes a slot (lx ly lz hx | hy hz), so that one
-    // address serves both loads of a slot; kMaxRadius spare slots past the
-    // last, so that the neighbour search reads slot + r unconditionally
-    struct alignas(32) BoxSlot {
-        float4 a;
-        float2 b;
-    } box[64 + kMaxRadius];
-    uint32_t cid[64];
-    uint32_t rep[64];
+    // Cluster boxes by slot, in two planes (lx ly lz hx | hy hz) so that the
+    // loads of neighbouring slots are free of bank conflicts (32 bytes a slot
+    // made each take twice as long). Each group has GW slots and kMaxRadius
+    // more that always hold a NaN box, so that the neighbour search reads
+    // slot + r unconditionally.
+    static constexpr uint32_t kStride = GW + kMaxRadius;
+    float4 boxa[64 / GW * kStride];
+    float2 boxb[64 / GW * kStride];
+    uint2 id[64];                     // cluster id, representative
     uint32_t sz[64];                  // primitives in the cluster
     // in-wave hand-over of the parent exchange
     uint32_t mlane[64];               // slot & 63 -> a lane that posted it
     uint32_t mslot[64];               // lane -> slot it exchanges at rightwards this step, or kInvalid
     uint32_t mclaim[64];              // lane -> range end handed to it, or kInvalid
+    std::conditional_t<KEEP == kKeepStaged, RecStage, NoStage> rec;
 };
 
-__device__ __forceinline__ uint64_t delta_k(const uint32_t* m, uint32_t a, uint32_t b) {
-    return (((uint64_t)m[a] << 32) | a) ^ (((uint64_t)m[b] << 32) | b);
+// Delta (BinaryBuilder.cu:16-40) between the sorted positions a and a + 1, their
+// keys read by one load. 32-bit keys: the keys' bits, then the positions'.
+// 64-bit keys: the keys', or of equal keys the positions'.
+__device__ __forceinline__ uint64_t delta_next(const uint32_t* m, uint32_t a, uint32_t) {
+    struct Pair { uint32_t k[2]; } p;
+    __builtin_memcpy(&p, m + a, sizeof(p));
+    return ((uint64_t)(p.k[0] ^ p.k[1]) << 32) | (a ^ (a + 1));
 }
-__device__ __forceinline__ uint64_t delta_k(const uint64_t* m, uint32_t a, uint32_t b) {
-    uint64_t d = m[a] ^ m[b];
-    return d ? d : (uint64_t)(a ^ b);
+__device__ __forceinline__ uint64_t delta_next(const uint64_t* m, uint32_t a, uint32_t) {
+    struct Pair { uint64_t k[2]; } p;
+    __builtin_memcpy(&p, m + a, sizeof(p));
+    const uint64_t d = p.k[0] ^ p.k[1];
+    return d ? d : (uint64_t)(a ^ (a + 1));
 }
 // Batched keys (mesh << 30 | 30-bit code): the 32-bit Delta of the mesh alone,
 // with positions local to the mesh (first position lo). Both keys lie in one
 // mesh, so the mesh bits in their low words cancel in the XOR.
-__device__ __forceinline__ uint64_t delta_batch(const uint64_t* m, uint32_t a, uint32_t b, uint32_t lo) {
-    return (((uint64_t)(uint32_t)m[a] << 32) | (a - lo)) ^ (((uint64_t)(uint32_t)m[b] << 32) | (b - lo));
+__device__ __forceinline__ uint64_t delta_next_batch(const uint64_t* m, uint32_t a, uint32_t lo) {
+    struct Pair { uint32_t k[4]; } p;
+    __builtin_memcpy(&p, m + a, sizeof(p));
+    return ((uint64_t)(p.k[0] ^ p.k[2]) << 32) | ((a - lo) ^ (a + 1 - lo));
 }
 
-__device__ __forceinline__ void lds_put_box(HplocLds& s, uint32_t i, const Box& b) {
-    s.box[i].a = make_float4(b.lx, b.ly, b.lz, b.hx);
-    s.box[i].b = make_float2(b.hy, b.hz);
+template <int GW, HplocKeep KEEP>
+__device__ __forceinline__ void lds_put_box(HplocLds<GW, KEEP>& s, uint32_t i, const Box& b) {
+    s.boxa[i] = make_float4(b.lx, b.ly, b.lz, b.hx);
+    s.boxb[i] = make_float2(b.hy, b.hz);
 }
-__device__ __forceinline__ Box lds_get_box(const HplocLds& s, uint32_t i) {
-    float4 a = s.box[i].a;
-    float2 c = s.box[i].b;
+template <int GW, HplocKeep KEEP>
+__device__ __forceinline__ Box lds_get_box(const HplocLds<GW, KEEP>& s, uint32_t i) {
+    float4 a = s.boxa[i];
+    float2 c = s.boxb[i];
     Box b;
     b.lx = a.x; b.ly = a.y; b.lz = a.z; b.hx = a.w; b.hy = c.x; b.hz = c.y;
     return b;
 }
 
-// The value of the lane below (wave shift by one); lane 0 takes `first`.
-__device__ __forceinline__ uint32_t from_lane_below(uint32_t v, uint32_t first) {
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)v, 0x138, 0xF, 0xF, false);
+// The value of the lane below; lane 0 takes lane 63's.
+__device__ __forceinline__ uint32_t from_lane_below(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x13C, 0xF, 0xF, true);
 }
 
 // FindNearestNeighbor (BinaryBuilder.cu:127-163) without branching on lanes:
 // the reference's choice is the first minimum of the areas in the order
 // forward a(i, i+1), backward a(i-1, i), a(i, i+2), a(i-2, i), ... Distances
-// are taken from the largest to 1. Every forward area is computed (candidates
-// past the group's clusters read spare or stale slots); those that are not
-// clusters of the group, or lie beyond the lane's own radius R (the task's,
-// uniform over its group), become kInvalid. Lane i + r receives a(i, i + r) as
-// its backward area by r shifts of one lane: the running minimum `bb` moves up
-// a lane before distance r is taken in, so a value taken in at distance r ends
-// r lanes up after the shift that follows distance 1. A valid area's target is
-// a cluster of the same group, so nothing valid crosses into the other group.
-// Taking an equal area at a smaller distance leaves each side's first minimum;
-// between the sides an equal area goes to the smaller distance, then forward.
-// The shifts are VALU moves (DPP): with each backward area fetched through LDS
-// (ds_bpermute) and scanned in the reference's order, a radius-8 search waited
-// on eight LDS round trips and took 78 registers instead of 70. With the
-// neighbour's neighbour taken from its lane as well and the stores' wait moved
-// (k_hploc), H-PLOC went 100 -> 84 us at 2,003 primitives, 612 -> 555 us at
-// 2.9M (64-lane schedule), 3250 -> 3175 us at 28.1M, and the 2,048-mesh batch
-// 2006 -> 1885 us.
-template <uint32_t UNROLL>
-__device__ __forceinline__ uint32_t nearest(const HplocLds& s, const Box& own, uint32_t slot, uint32_t gl, int lim,
-                                            uint32_t top) {
-    uint32_t bf = kInvalid, bb = kInvalid, rf = 0, rb = 0;
+// are taken from the largest to 1. Lane i + r receives a(i, i + r) as its
+// backward area by r shifts of one lane: the running minimum `bb` and the lane
+// `src` it came from move up a lane before distance r is taken in, so what is
+// taken in at distance r ends r lanes up after the shift that follows distance
+// 1. Taking an equal area at a smaller distance leaves each side's first
+// minimum; between the sides an equal area goes to the smaller distance, then
+// forward. The shifts are VALU moves (DPP), most of them folded into the
+// minimum or the select that follows.
+//
+// Slots past the group's clusters hold NaN boxes, whose areas are NaN: as bits
+// above every finite area, so with MASK == false nothing is compared against
+// the group's end. A wave whose minima are all finite has the reference's
+// choice; any other (areas that overflow) searches with MASK == true, where
+// candidates that are not clusters of the group, or lie beyond the lane's own
+// radius (the task's, uniform over its group), become kInvalid explicitly. A
+// taken-in area's target is a slot of the same group, so nothing valid crosses
+// into another group.
+//
+// Each backward area fetched through LDS and scanned in the reference's order
+// took 8 LDS round trips and 78 registers; shifts of distances and a compare
+// with the group's end per distance 26 VALU instructions per distance, now 20.
+template <uint32_t UNROLL, bool MASK, int GW, HplocKeep KEEP>
+__device__ __forceinline__ uint32_t nearest(const HplocLds<GW, KEEP>& s, const Box& own, uint32_t slot, uint32_t gl,
+                                            int lim, uint32_t top, uint32_t& best) {
+    uint32_t bf = kInvalid, bb = kInvalid, rf = 0, src = gl;
 #pragma unroll UNROLL
     for (uint32_t r = top; r >= 1; --r) {
-        const uint32_t a = __float_as_uint(box_area(box_union(own, lds_get_box(s, slot + r))));
-        const uint32_t af = (int)r < lim ? a : kInvalid;
-        bb = min(from_lane_below(bb, kInvalid), af);
-        rb = from_lane_below(rb, 0u);
-        rb = bb == af ? r : rb;
-        bf = min(bf, af);
-        rf = bf == af ? r : rf;
+        uint32_t a = __float_as_uint(box_area(box_union(own, lds_get_box(s, slot + r))));
+        if (MASK) a = (int)r < lim ? a : kInvalid;
+        bb = min(from_lane_below(bb), a);
+        asm("" : "+v"(bb));  // one use of the shifted value, so that the shift folds into the minimum
+        src = from_lane_below(src);
+        src = bb == a ? gl : src;
+        bf = min(bf, a);
+        rf = bf == a ? r : rf;
     }
-    bb = from_lane_below(bb, kInvalid);
-    rb = from_lane_below(rb, 0u);
-    const bool fwd = bf < bb || (bf == bb && rf <= rb);
-    const uint32_t other = fwd ? gl + rf : gl - rb;
-    return min(bf, bb) == kInvalid ? kInvalid : other;
-}
-
-// Radius known at compile time: constant LDS offsets, no loop control.
-template <uint32_t R>
-__device__ __forceinline__ uint32_t nearest_fixed(const HplocLds& s, const Box& own, uint32_t slot, uint32_t gl,
-                                                  uint32_t num) {
-    return nearest<R>(s, own, slot, gl, (int)num - (int)gl, R);
-}
-
-// The loop runs to Rw, the largest radius of the wave's groups, on scalar
-// control; R is the lane's own radius.
-__device__ __forceinline__ uint32_t nearest_uniform(const HplocLds& s, const Box& own, uint32_t slot, uint32_t gl,
-                                                    uint32_t num, uint32_t Rw, uint32_t R) {
-    return nearest<2>(s, own, slot, gl, min((int)num - (int)gl, (int)R + 1), Rw);
+    bb = from_lane_below(bb);
+    src = from_lane_below(src);
+    best = min(bf, bb);
+    const bool fwd = bf < bb || (bf == bb && rf <= gl - src);
+    return fwd ? gl + rf : src;
 }
 
 struct NodeStore {
@@ -184,11 +222,11 @@ struct NodeStore {
     nxb_bvh2_node* moved;      // spare slot per mesh for kMoved
     uint32_t* moved_parent;    // per mesh: id of the node whose child is kMoved
     uint32_t* moved_size;      // per mesh: primitive count of the kMoved node
-    uint32_t* nsize;           // primitive count of internal node id (index id - n); null: not kept
+    uint32_t* nsize;           // kKeepSizes: primitive count of internal node id (index id - n)
     uint32_t n;                // leaves (all meshes)
     uint32_t node_count;       // nodes (all meshes): 2n - meshes
-    uint4* rec8 = nullptr;     // one mesh, BVH8 build: wide record of internal node id at id - n
-    uint4* moved_rec = nullptr;  // spare wide record for kMoved
+    uint4* rec8;               // kKeepRecords, kKeepStaged (one mesh): wide record of internal node id at id - n
+    uint4* moved_rec;          // spare wide record for kMoved
 };
 
 // The mesh of a merge task: sorted positions [lo, lo + cnt), local node id L
@@ -301,12 +339,14 @@ __device__ __forceinline__ void store_rec8_agent(uint4* p, const uint4 q[4]) {
 
 // Creates the node merging clusters (left, right) with box b and size
 // primitives (lb, rb, lsz, rsz: the two clusters' boxes and primitive
-// counts, for the wide record). Returns its id.
-template <bool REC>
-__device__ __forceinline__ uint32_t create_node(const NodeStore& ns, const MeshCtx& mc, const Box& b, uint32_t left,
-                                                uint32_t right, uint32_t right_rep, uint32_t size, bool root_step,
-                                                uint32_t* flags, const Box& lb, const Box& rb, uint32_t lsz,
-                                                uint32_t rsz) {
+// counts, for the wide record). Returns its id. A wide record goes to row
+// `row` of the stage; store_records() stores it.
+template <HplocKeep KEEP, typename Lds>
+__device__ __forceinline__ uint32_t create_node(Lds& s, uint32_t row, const NodeStore& ns, const MeshCtx& mc,
+                                                const Box& b, uint32_t left, uint32_t right, uint32_t right_rep,
+                                                uint32_t size, bool root_step, uint32_t* flags, const Box& lb,
+                                                const Box& rb, uint32_t lsz, uint32_t rsz) {
+    if constexpr (KEEP == kKeepStaged) s.rec.at[row] = kInvalid;
     const uint32_t n = ns.n;
     const uint32_t local = mc.cnt - 1 + (right_rep - mc.lo);
     const uint32_t root_local = 2 * mc.cnt - 2;
@@ -314,7 +354,7 @@ __device__ __forceinline__ uint32_t create_node(const NodeStore& ns, const MeshC
     uint32_t id = root_step ? mc.base + root_local : (local == root_local ? kMoved : natural);
     if (local > root_local || natural >= ns.node_count) { atomic_or_agent(flags, kFlagBadIndex); return 0; }
     uint32_t* moved_parent = ns.moved_parent + mc.mesh;
-    if (REC && ns.rec8) {
+    if constexpr (KEEP >= kKeepRecords) {
         // BVH8 build: the wide record stands for the internal node (its box
         // is the union of the children's, its size their sum); the same
         // parking of kMoved, on records.
@@ -352,8 +392,14 @@ __device__ __forceinline__ uint32_t create_node(const NodeStore& ns, const MeshC
         } else if (left == kMoved || right == kMoved) {
             store_rec8_agent(ns.rec8 + 4ull * (id - n), q);
         } else {
-            uint4* p = ns.rec8 + 4ull * (id - n);
-            p[0] = q[0]; p[1] = q[1]; p[2] = q[2]; p[3] = q[3];
+            if constexpr (KEEP == kKeepStaged) {
+                s.rec.at[row] = id - n;
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) s.rec.q[4 * row + ((i + row / 4) & 3)] = q[i];
+            } else {
+                uint4* p = ns.rec8 + 4ull * (id - n);
+                p[0] = q[0]; p[1] = q[1]; p[2] = q[2]; p[3] = q[3];
+            }
         }
         return id;
     }
@@ -364,7 +410,7 @@ __device__ __forceinline__ uint32_t create_node(const NodeStore& ns, const MeshC
         uint64_t w[4];
         load_node_agent(moved, w);
         store_words_agent(ns.nodes + natural, w);
-        if (ns.nsize) ns.nsize[natural - n] = load_agent(moved_size);
+        if constexpr (KEEP == kKeepSizes) ns.nsize[natural - n] = load_agent(moved_size);
         if (left == kMoved) {
             left = natural;
         } else if (right == kMoved) {
@@ -393,9 +439,23 @@ __device__ __forceinline__ uint32_t create_node(const NodeStore& ns, const MeshC
     if (id == kMoved) store_node_agent(moved, 0, b, left, right);
     else if (left == kMoved || right == kMoved) store_node_agent(ns.nodes, id, b, left, right);
     else store_node(ns.nodes, id, b, left, right);
-    if (id == kMoved) store_agent(moved_size, size);
-    else if (ns.nsize) ns.nsize[id - n] = size;
+    if constexpr (KEEP == kKeepSizes) {
+        if (id == kMoved) store_agent(moved_size, size);
+        else ns.nsize[id - n] = size;
+    }
     return id;
+}
+
+// Stores the staged records of a round (`count` rows), a 64-byte segment per
+// four lanes. Stored by the lane that made it, a record took four stores of 16
+// bytes to as many segments as lanes.
+__device__ __forceinline__ void store_records(const RecStage& st, const NodeStore& ns, uint32_t count) {
+    const uint32_t lane = __lane_id();
+    for (uint32_t r = lane / 4; r - lane / 4 < count; r += 16) {
+        const uint32_t at = r < count ? st.at[r] : kInvalid;
+        const uint4 v = st.q[4 * r + (lane & 3)];
+        if (at != kInvalid) ns.rec8[4ull * at + ((lane - r / 4) & 3)] = v;
+    }
 }
 
 // Per-segment radius policy: a merge task over sorted positions
@@ -417,18 +477,18 @@ __device__ __forceinline__ uint32_t radius_for(const RadiusParams& rp, uint32_t 
 // PlocMerge for the group this lane belongs to. All lanes of the wave call
 // it together; a group with has_task == false does nothing.
 //   GW  : lanes per group (32 or 64), C = GW / 2
-//   gl  : lane index within the group; gbase: first LDS slot of the group
+//   gl  : lane index within the group; gbase: first lane of the group
 //   gmask: 64-bit mask of the group's lanes
-// REC: the build may write wide records (ns.rec8); batched builds never do.
-template <int GW, bool REC>
-__device__ __forceinline__ void ploc_merge(HplocLds& s, bool has_task, uint32_t l_start, uint32_t split,
+template <int GW, HplocKeep KEEP>
+__device__ __forceinline__ void ploc_merge(HplocLds<GW, KEEP>& s, bool has_task, uint32_t l_start, uint32_t split,
                                            uint32_t r_end, bool final, uint32_t gl, uint32_t gbase,
                                            uint64_t gmask, const uint32_t* cluster, uint32_t* recs, uint32_t* csizes,
                                            const NodeStore& ns, const MeshCtx& mc, const RadiusParams& rp,
                                            uint32_t* flags) {
     constexpr uint32_t C = GW / 2;
-    const uint32_t slot = gbase + gl;
-    uint32_t cid = kInvalid, rep = 0, sz = 0, num_loaded = 0;
+    const uint32_t bbase = gbase / GW * HplocLds<GW, KEEP>::kStride;  // the group's first box slot
+    const float nan = __builtin_nanf("");
+    uint32_t num;
 
     // LoadIndices (BinaryBuilder.cu:42-57): the left child's clusters, then
     // the right child's. A child of at most C primitives was never merged:
@@ -437,7 +497,7 @@ __device__ __forceinline__ void ploc_merge(HplocLds& s, bool has_task, uint32_t 
     // records at the front of its range, their count in the first record.
     // Lanes [0, C) read the left child's clusters and lanes [C, 2C) the
     // right child's, all at once; the valid entries are then compacted in
-    // that order through LDS.
+    // that order through LDS, where the group's other slots get NaN boxes.
     {
         const bool lhalf = gl < C;
         const uint32_t k = lhalf ? gl : gl - C;
@@ -446,132 +506,125 @@ __device__ __forceinline__ void ploc_merge(HplocLds& s, bool has_task, uint32_t 
         const bool merged = span > C;
         const uint32_t pos = first + k;
         bool v = has_task && k < min(span, C);
-        uint32_t lcid = kInvalid, lrep = 0, lsz = 0;
-        Box b = {0, 0, 0, 0, 0, 0};
+        // Leaves (written by an earlier kernel: plain loads) and records are
+        // both in flight at once; one after the other cost a task that has
+        // both kinds a third memory latency.
+        uint32_t leaf = 0, lsz = 1u;
+        ClusterRec r = {};
+        if (v && !merged) leaf = cluster[pos];
         if (v && merged) {
-            const ClusterRec r = load_rec(ns, recs, pos);
-            lsz = load_agent(&csizes[pos]);
-            lcid = r.cid;
-            lrep = r.rep;
-            b = r.b;
-        } else if (v) {
-            // a leaf: written by an earlier kernel, plain loads
-            lcid = cluster[pos];
-            if (lcid >= ns.n) { atomic_or_agent(flags, kFlagBadIndex); lcid = 0; }
-            b = load_box(ns.nodes, lcid);
-            lrep = pos;
-            lsz = 1u;
+            r = load_rec(ns, recs, pos);
+            if constexpr (KEEP != kKeepNodes) lsz = load_agent(&csizes[pos]);
         }
+        Box lb = {};
+        if (v && !merged) {
+            if (leaf >= ns.n) { atomic_or_agent(flags, kFlagBadIndex); leaf = 0; }
+            lb = load_box(ns.nodes, leaf);
+        }
+        const uint32_t lcid = merged ? r.cid : leaf;
         // the half's first lane holds the child's cluster count (merged child)
-        const uint32_t count = (uint32_t)__shfl((int)lrep, (int)(gbase + (lhalf ? 0u : C)));
-        if (v) {
-            if (merged) {
-                v = k < count;
-                if (k == 0) lrep = first;
-            }
-            v = v && lcid != kInvalid;
-            if (v && lcid != kMoved && lcid >= ns.node_count) atomic_or_agent(flags, kFlagBadIndex);
-        }
+        const uint32_t count = (uint32_t)__shfl((int)r.rep, (int)(gbase + (lhalf ? 0u : C)));
+        const uint32_t lrep = merged ? (k == 0 ? first : r.rep) : pos;
+        v = v && (!merged || k < count) && lcid != kInvalid;
+        if (v && lcid - ns.node_count < kMoved - ns.node_count) atomic_or_agent(flags, kFlagBadIndex);
+        Box b = merged ? r.b : lb;
         const uint64_t vm = ballot(v) & gmask;
-        if (v) {
-            const uint32_t dst = gbase + mask_rank(vm);
-            lds_put_box(s, dst, b);
-            s.cid[dst] = lcid;
-            s.rep[dst] = lrep;
-            s.sz[dst] = lsz;
-        }
+        num = (uint32_t)__popcll(vm);
+        const uint32_t rank = mask_rank(vm), dst = v ? rank : num + gl - rank;
+        b.lx = v ? b.lx : nan;
+        lds_put_box(s, bbase + dst, b);
+        s.id[gbase + dst] = make_uint2(lcid, lrep);
+        if constexpr (KEEP != kKeepNodes) s.sz[gbase + dst] = lsz;
         wave_lds_sync();
-        const uint32_t loaded_now = (uint32_t)__popcll(vm);
-        if (gl < loaded_now) {
-            cid = s.cid[slot];
-            rep = s.rep[slot];
-            sz = s.sz[slot];
-        }
-        wave_lds_sync();
-        num_loaded = loaded_now;
     }
-    const uint32_t loaded = num_loaded;
-    uint32_t num = loaded;
+    const uint32_t slot = bbase + gl;
+    Box own = lds_get_box(s, slot);
+    uint32_t cid = s.id[gbase + gl].x, rep = s.id[gbase + gl].y, sz = 0;
+    if constexpr (KEEP != kKeepNodes) sz = s.sz[gbase + gl];
 
-    Box own = {0, 0, 0, 0, 0, 0};
-    if (gl < num) own = lds_get_box(s, slot);
     const uint32_t threshold = final ? 1u : C;
-    const uint32_t R = has_task ? radius_for(rp, l_start, r_end) : 1u;
-    // one radius for every task (no per-segment table): the unrolled search
-    // for radius 8; otherwise the loop runs to the largest radius of the
-    // wave's groups (each group's radius is uniform over it)
+    // One radius for every task (no per-segment table): the unrolled search for
+    // radius 8, a loop for others. With a table the loop runs to the largest
+    // radius of the wave's groups (each group's is uniform over it).
     const uint32_t fixed_r = rp.table ? 0u : min(rp.radius, (uint32_t)kMaxRadius);
-    const uint32_t r_wave = GW == 64 ? __builtin_amdgcn_readfirstlane(R)
-                                     : max(__builtin_amdgcn_readlane(R, 0), __builtin_amdgcn_readlane(R, 32));
+    uint32_t R = fixed_r, r_wave = fixed_r;
+    if (rp.table) {
+        R = has_task ? radius_for(rp, l_start, r_end) : 1u;
+        r_wave = GW == 64 ? __builtin_amdgcn_readfirstlane(R)
+                          : max(__builtin_amdgcn_readlane(R, 0), __builtin_amdgcn_readlane(R, 32));
+    }
 
-    // LDS slots [gbase, gbase + num) hold own/cid/rep/sz of the group's
-    // clusters here and after every compaction below.
-    while (num > threshold) {
+    // The group's first num slots hold own/id/sz of its clusters here and after
+    // every compaction below, its other slots NaN boxes. All lanes of the wave
+    // take part in every round (lane shifts read them); a group that is done
+    // (num <= threshold) merges nothing.
+    for (;;) {
+        const bool run = num > threshold && gl < num;
+        if (!ballot(run)) break;
         // ---- FindNearestNeighbor (BinaryBuilder.cu:127-163) ----
-        uint32_t nn = kInvalid;
-        if (fixed_r == 8) nn = nearest_fixed<8>(s, own, slot, gl, num);
-        else nn = nearest_uniform(s, own, slot, gl, num, r_wave, R);
-        if (gl >= num) nn = kInvalid;
+        uint32_t nn, best;
+        if (fixed_r == 8) nn = nearest<8, false>(s, own, slot, gl, 0, 8u, best);
+        else if (fixed_r) nn = nearest<2, false>(s, own, slot, gl, 0, fixed_r, best);
+        else nn = nearest<2, true>(s, own, slot, gl, (int)R + 1, r_wave, best);
+        if (ballot(run && best >= kInfBits)) {
+            nn = nearest<1, true>(s, own, slot, gl, min((int)num - (int)gl, (int)R + 1), r_wave, best);
+            if (best == kInvalid) nn = kInvalid;
+        }
 
         // ---- MergeClustersCreateBVH2Node (BinaryBuilder.cu:72-124) ----
         // the neighbour's neighbour, from its lane
         const uint32_t theirs = (uint32_t)__builtin_amdgcn_ds_bpermute((int)((gbase + nn) * 4u), (int)nn);
-        const uint32_t nnnn = nn < (uint32_t)GW ? theirs : kInvalid;
-        bool mutual = gl < num && nnnn == gl;
-        bool merge = mutual && gl < nn;
-        uint64_t mm = ballot(merge) & gmask;
-        uint32_t mcount = (uint32_t)__popcll(mm);
+        const bool mutual = run && nn < (uint32_t)GW && theirs == gl;
+        const bool merge = mutual && gl < nn;
+        const uint64_t merges = ballot(merge);
+        const uint32_t mcount = (uint32_t)__popcll(merges & gmask);
         const bool root_step = final && num - mcount == 1;
         if (merge) {
-            const Box nb = lds_get_box(s, gbase + nn);
-            const uint32_t ncid = s.cid[gbase + nn];
-            const uint32_t nrep = s.rep[gbase + nn];
-            const uint32_t nsz = s.sz[gbase + nn];
+            const Box nb = lds_get_box(s, bbase + nn);
+            const uint2 nid = s.id[gbase + nn];
+            uint32_t nsz = 0;
+            if constexpr (KEEP != kKeepNodes) nsz = s.sz[gbase + nn];
             const Box ob = own;
             own = box_union(own, nb);
-            cid = create_node<REC>(ns, mc, own, cid, ncid, nrep, sz + nsz, root_step, flags, ob, nb, sz, nsz);
+            cid = create_node<KEEP>(s, mask_rank(merges), ns, mc, own, cid, nid.x, nid.y, sz + nsz, root_step, flags,
+                                    ob, nb, sz, nsz);
             sz += nsz;
         }
-        bool valid = gl < num && (merge || !mutual);
-        uint64_t vm = ballot(valid) & gmask;
-        uint32_t pos = mask_rank(vm);
-        wave_lds_sync();
-        if (valid) {
-            lds_put_box(s, gbase + pos, own);
-            s.cid[gbase + pos] = cid;
-            s.rep[gbase + pos] = rep;
-            s.sz[gbase + pos] = sz;
-        }
+        const bool valid = gl < num && (merge || !mutual);
+        const uint64_t vm = ballot(valid) & gmask;
         num -= mcount;
+        const uint32_t rank = mask_rank(vm), dst = valid ? rank : num + gl - rank;
+        own.lx = valid ? own.lx : nan;
         wave_lds_sync();
-        if (gl < num) {
-            own = lds_get_box(s, slot);
-            cid = s.cid[slot];
-            rep = s.rep[slot];
-            sz = s.sz[slot];
-        } else {
-            cid = kInvalid;
-        }
+        lds_put_box(s, bbase + dst, own);
+        s.id[gbase + dst] = make_uint2(cid, rep);
+        if constexpr (KEEP != kKeepNodes) s.sz[gbase + dst] = sz;
+        wave_lds_sync();
+        own = lds_get_box(s, slot);
+        cid = s.id[gbase + gl].x;
+        rep = s.id[gbase + gl].y;
+        if constexpr (KEEP != kKeepNodes) sz = s.sz[gbase + gl];
+        if constexpr (KEEP == kKeepStaged) store_records(s.rec, ns, (uint32_t)__popcll(merges));
     }
 
     // StoreIndices (BinaryBuilder.cu:59-69), as records: the num clusters
     // left, the count in the first record's representative word.
     if (gl < num) {
         store_rec(ns, recs, l_start + gl, own, cid, gl == 0 ? num : rep);
-        store_agent(&csizes[l_start + gl], sz);
+        if constexpr (KEEP != kKeepNodes) store_agent(&csizes[l_start + gl], sz);
     }
 }
 
-template <typename K, int GW, bool BATCH>
+template <typename K, int GW, bool BATCH, HplocKeep KEEP>
 __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6))) void k_hploc(const K* __restrict__ keys, const uint32_t* cluster,
                                                          uint32_t* recs, uint32_t* csizes, uint32_t* parent,
                                                          NodeStore ns, const uint32_t* __restrict__ mesh_lo,
                                                          uint32_t meshes, RadiusParams rp, uint32_t* flags,
                                                          uint32_t* next_chunk, uint32_t first, uint32_t chunk) {
-    __shared__ HplocLds lds[kHplocWaves];
+    __shared__ HplocLds<GW, KEEP> lds[kHplocWaves];
     constexpr uint32_t C = GW / 2;
     const uint32_t tid = threadIdx.x;
-    HplocLds& s = lds[tid >> 6];
+    HplocLds<GW, KEEP>& s = lds[tid >> 6];
     const uint32_t lane = tid & 63;
     const uint32_t n = ns.n;
 
@@ -594,9 +647,9 @@ __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6
     uint32_t pf = 0;
     {
         const uint32_t j = (blockIdx.x / kHplocRegions) * kHplocWaves + (tid >> 6);
-        const uint64_t lo = (uint64_t)region * region_len;
-        const uint64_t hi_r = min((uint64_t)n, lo + region_len);
-        const uint64_t c = lo + (uint64_t)j * first;
+        const uint64_t lo_r = (uint64_t)region * region_len;
+        const uint64_t hi_r = min((uint64_t)n, lo_r + region_len);
+        const uint64_t c = lo_r + (uint64_t)j * first;
         if (c < hi_r) {
             next = (uint32_t)c;
             end = (uint32_t)min(hi_r, c + first);
@@ -606,11 +659,12 @@ __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6
     uint32_t left = 0, right = 0, split = 0;
     bool active = false;
     bool pending = false;        // a merge's stores may be in flight (wave-uniform)
-    MeshCtx mc{0u, n, 0u, 0u};  // this lane's mesh (the whole array for a single build)
-    uint32_t hi = n - 1;
+    uint32_t lo = 0, hi = n - 1, mesh = 0;  // this lane's mesh [lo, hi] (the whole array for a single build)
 
     s.mlane[lane] = lane;
     s.mclaim[lane] = kInvalid;
+    for (uint32_t i = lane; i < 64 / GW * HplocLds<GW, KEEP>::kStride; i += 64)
+        s.boxa[i] = make_float4(__builtin_nanf(""), 0.0f, 0.0f, 0.0f);
     wave_lds_sync();
 
     uint32_t g, gl, gbase;
@@ -637,10 +691,10 @@ __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6
             // its waves
             const uint32_t waves_r =
                 gridDim.x > region ? ((gridDim.x - region + kHplocRegions - 1) / kHplocRegions) * kHplocWaves : 0u;
-            const uint64_t lo = (uint64_t)region * region_len;
-            const uint64_t hi_r = min((uint64_t)n, lo + region_len);
+            const uint64_t lo_r = (uint64_t)region * region_len;
+            const uint64_t hi_r = min((uint64_t)n, lo_r + region_len);
             uint32_t* ctr = &next_chunk[region * kHplocCounterStride];
-            const uint64_t base = lo + (uint64_t)waves_r * first;
+            const uint64_t base = lo_r + (uint64_t)waves_r * first;
             uint32_t c = 0;
             if (have_pf) {
                 c = pf;  // lane 0's, taken with the stores of the refill that used up the last chunk
@@ -672,14 +726,13 @@ __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6
                 if constexpr (BATCH) {
                     const uint32_t m = (uint32_t)((uint64_t)keys[i] >> 30);
                     if (m < meshes) {
-                        const uint32_t lo = mesh_lo[m];
-                        mc = MeshCtx{lo, mesh_lo[m + 1] - lo, m, 0u};
-                        mc.base = n + lo - m - mc.cnt;
+                        mesh = m;
+                        lo = mesh_lo[m];
+                        hi = mesh_lo[m + 1] - 1;
                     } else {
                         atomic_or_agent(flags, kFlagBadIndex);
                         active = false;
                     }
-                    hi = mc.lo + mc.cnt - 1;
                 }
             }
             next = min(end, next + nfree);
@@ -696,15 +749,11 @@ __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6
         }
         bool to_right = false;
         if (active) {
-            if constexpr (BATCH) {
-                const uint64_t* k64 = reinterpret_cast<const uint64_t*>(keys);
-                to_right = (left == mc.lo) ||
-                           (right != hi && delta_batch(k64, right, right + 1, mc.lo) <
-                                               delta_batch(k64, left - 1, left, mc.lo));
-            } else {
-                to_right = (left == 0) ||
-                           (right != n - 1 && delta_k(keys, right, right + 1) < delta_k(keys, left - 1, left));
-            }
+            const auto d = [&](uint32_t at) {
+                if constexpr (BATCH) return delta_next_batch(keys, at, lo);
+                else return delta_next(keys, at, 0u);
+            };
+            to_right = left == lo || (right != hi && d(right) < d(left - 1));
         }
         // Two lanes of this wave that reach the same parent slot in this step
         // (the range ending at it going right, the one starting after it
@@ -745,26 +794,22 @@ __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6
             }
         }
         if (active && !handed) {
-            uint32_t prev;
-            if (to_right) {
-                prev = atomic_xchg_agent(&parent[right], left);
-                if (prev != kInvalid) {
-                    if (prev > hi || prev < mc.lo) { atomic_or_agent(flags, kFlagBadIndex); prev = hi; }
-                    split = right + 1;
-                    right = prev;
-                }
+            const uint32_t at = to_right ? right : left - 1;
+            uint32_t prev = atomic_xchg_agent(&parent[at], to_right ? left : right);
+            if (prev == kInvalid) {
+                active = false;
             } else {
-                prev = atomic_xchg_agent(&parent[left - 1], right);
-                if (prev != kInvalid) {
-                    if (prev > hi || prev < mc.lo) { atomic_or_agent(flags, kFlagBadIndex); prev = mc.lo; }
-                    split = left;
-                    left = prev;
+                if (prev > hi || prev < lo) {
+                    atomic_or_agent(flags, kFlagBadIndex);
+                    prev = to_right ? hi : lo;
                 }
+                split = at + 1;
+                if (to_right) right = prev;
+                else left = prev;
             }
-            if (prev == kInvalid) active = false;
         }
         uint32_t size = right - left + 1;
-        bool final = active && size == mc.cnt;
+        bool final = active && size == hi - lo + 1;
         uint64_t tasks = ballot(active && (size > C || final));
         if (!tasks) continue;
 
@@ -792,15 +837,16 @@ __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6
             }
             uint32_t tl = g ? l1 : l0, ts = g ? s1 : s0, tr = g ? r1 : r0;
             bool tf = (g ? f1 : f0) != 0;
-            MeshCtx tm = mc;
+            MeshCtx tm{0u, n, 0u, 0u};
             if constexpr (BATCH) {
                 // the task's mesh (lanes of the other group run another task)
-                tm.lo = __shfl(mc.lo, (int)tsel);
-                tm.cnt = __shfl(mc.cnt, (int)tsel);
-                tm.mesh = __shfl(mc.mesh, (int)tsel);
-                tm.base = __shfl(mc.base, (int)tsel);
+                tm.lo = __shfl(lo, (int)tsel);
+                tm.cnt = __shfl(hi, (int)tsel) + 1 - tm.lo;
+                tm.mesh = __shfl(mesh, (int)tsel);
+                tm.base = n + tm.lo - tm.mesh - tm.cnt;
             }
-            ploc_merge<GW, !BATCH>(s, has, tl, ts, tr + 1, tf, gl, gbase, gmask, cluster, recs, csizes, ns, tm, rp, flags);
+            ploc_merge<GW, KEEP>(s, has, tl, ts, tr + 1, tf, gl, gbase, gmask, cluster, recs, csizes, ns, tm, rp,
+                                 flags);
         }
         // Merge outputs are agent-scope atomic stores; they must be complete
         // before this wave's next parent exchange hands the subtree over. The
@@ -840,11 +886,11 @@ static HplocChunks hploc_chunks(uint32_t n, uint32_t grid) {
     return HplocChunks{(uint32_t)first, (uint32_t)(chunk > kHplocMaxChunk ? kHplocMaxChunk : chunk)};
 }
 
-template <typename K, int GW, bool BATCH>
+template <typename K, int GW, bool BATCH, HplocKeep KEEP>
 static hipError_t launch_hploc_kernel(const K* keys, uint32_t* cluster, uint32_t n, const uint32_t* mesh_lo,
                                       uint32_t meshes, const NodeStore& ns, RadiusParams rp, uint32_t blocks_per_cu,
                                       HplocScratch sc, hipStream_t s) {
-    auto kernel = k_hploc<K, GW, BATCH>;
+    auto kernel = k_hploc<K, GW, BATCH, KEEP>;
     const uint32_t grid = hploc_grid(kernel, n, blocks_per_cu);
     const HplocChunks cp = hploc_chunks(n, grid);
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kHplocThreads), 0, s, keys, cluster, sc.recs, sc.csizes, sc.parent,
@@ -852,35 +898,43 @@ static hipError_t launch_hploc_kernel(const K* keys, uint32_t* cluster, uint32_t
     return hipGetLastError();
 }
 
+template <typename K, bool BATCH, HplocKeep KEEP>
+static hipError_t launch_hploc_mode(const void* keys, uint32_t* cluster, uint32_t n, const uint32_t* mesh_lo,
+                                    uint32_t meshes, const NodeStore& ns, uint32_t merge_mode, RadiusParams rp,
+                                    uint32_t blocks_per_cu, HplocScratch sc, hipStream_t s) {
+    const K* k = static_cast<const K*>(keys);
+    return merge_mode == NXB_MERGE_WAVE64
+               ? launch_hploc_kernel<K, 64, BATCH, KEEP>(k, cluster, n, mesh_lo, meshes, ns, rp, blocks_per_cu, sc, s)
+               : launch_hploc_kernel<K, 32, BATCH, KEEP>(k, cluster, n, mesh_lo, meshes, ns, rp, blocks_per_cu, sc, s);
+}
+
 hipError_t launch_hploc(const void* keys, uint32_t key_bits, uint32_t* cluster, uint32_t n, nxb_bvh2_node* nodes,
                         uint32_t merge_mode, RadiusParams rp, uint32_t blocks_per_cu, HplocScratch sc,
                         hipStream_t s) {
     if (n == 0) return hipSuccess;
-    NodeStore ns{nodes, 2ull * n - 1 < (1ull << 27), sc.moved, sc.moved_parent, sc.moved_size, sc.nsize, n, 2 * n - 1};
-    if (sc.rec8 && sc.moved_rec) {
-        ns.rec8 = sc.rec8;
-        ns.moved_rec = sc.moved_rec;
-    }
-    const bool w64 = merge_mode == NXB_MERGE_WAVE64;
-    if (key_bits == 32) {
-        const uint32_t* k = static_cast<const uint32_t*>(keys);
-        return w64 ? launch_hploc_kernel<uint32_t, 64, false>(k, cluster, n, nullptr, 1u, ns, rp, blocks_per_cu, sc, s)
-                   : launch_hploc_kernel<uint32_t, 32, false>(k, cluster, n, nullptr, 1u, ns, rp, blocks_per_cu, sc, s);
-    }
-    const uint64_t* k = static_cast<const uint64_t*>(keys);
-    return w64 ? launch_hploc_kernel<uint64_t, 64, false>(k, cluster, n, nullptr, 1u, ns, rp, blocks_per_cu, sc, s)
-               : launch_hploc_kernel<uint64_t, 32, false>(k, cluster, n, nullptr, 1u, ns, rp, blocks_per_cu, sc, s);
+    if (sc.nsize) return hipErrorInvalidValue;  // no caller wants them for one mesh
+    const bool rec = sc.rec8 && sc.moved_rec;
+    const NodeStore ns{nodes, 2ull * n - 1 < (1ull << 27), sc.moved, sc.moved_parent, sc.moved_size, nullptr, n,
+                       2 * n - 1, sc.rec8, sc.moved_rec};
+    const auto launch = key_bits == 32
+                            ? (!rec                ? launch_hploc_mode<uint32_t, false, kKeepNodes>
+                               : n < kStagedPrims  ? launch_hploc_mode<uint32_t, false, kKeepRecords>
+                                                   : launch_hploc_mode<uint32_t, false, kKeepStaged>)
+                            : (!rec                ? launch_hploc_mode<uint64_t, false, kKeepNodes>
+                               : n < kStagedPrims  ? launch_hploc_mode<uint64_t, false, kKeepRecords>
+                                                   : launch_hploc_mode<uint64_t, false, kKeepStaged>);
+    return launch(keys, cluster, n, nullptr, 1u, ns, merge_mode, rp, blocks_per_cu, sc, s);
 }
 
 hipError_t launch_hploc_batch(const uint64_t* keys, uint32_t* cluster, uint32_t n, const uint32_t* mesh_lo,
                               uint32_t meshes, nxb_bvh2_node* nodes, uint32_t merge_mode, RadiusParams rp,
                               uint32_t blocks_per_cu, HplocScratch sc, hipStream_t s) {
     if (n == 0) return hipSuccess;
-    NodeStore ns{nodes, 2ull * n - meshes < (1ull << 27), sc.moved, sc.moved_parent, sc.moved_size, sc.nsize, n,
-                 2 * n - meshes};
-    return merge_mode == NXB_MERGE_WAVE64
-               ? launch_hploc_kernel<uint64_t, 64, true>(keys, cluster, n, mesh_lo, meshes, ns, rp, blocks_per_cu, sc, s)
-               : launch_hploc_kernel<uint64_t, 32, true>(keys, cluster, n, mesh_lo, meshes, ns, rp, blocks_per_cu, sc, s);
+    const NodeStore ns{nodes, 2ull * n - meshes < (1ull << 27), sc.moved, sc.moved_parent, sc.moved_size, sc.nsize, n,
+                       2 * n - meshes, nullptr, nullptr};
+    const auto launch =
+        sc.nsize ? launch_hploc_mode<uint64_t, true, kKeepSizes> : launch_hploc_mode<uint64_t, true, kKeepNodes>;
+    return launch(keys, cluster, n, mesh_lo, meshes, ns, merge_mode, rp, blocks_per_cu, sc, s);
 }
 
 }  // namespace nxb
