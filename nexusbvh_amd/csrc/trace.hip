@@ -16,8 +16,9 @@
 //
 // Three kernels give the same hits (a hit is the smallest distance, then the
 // smallest triangle index, whatever the order of the tests):
-//   k_trace_group  eight lanes per ray, one per child slot: few rays, where a
-//                  ray's chain of dependent steps is what takes the time;
+//   k_trace_group  eight lanes per node, one per child slot, and up to four
+//                  nodes of a ray at once: few rays, where a ray's chain of
+//                  dependent steps is what takes the time;
 //   k_trace_lane   one lane per ray: many rays, where the instructions issued
 //                  per ray count;
 //   k_trace        one lane per ray, with the counts of nodes visited and
@@ -344,26 +345,56 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_lane(const nxb_bvh8_nod
     hits[r] = nxb_hit{best_prim == NXB_INVALID_IDX ? rb.w : best_t, best_prim, bu, bv};
 }
 
-// Eight lanes per ray, lane s of a group for child slot s: one slab test, and
-// at most one triangle test, per lane and step, the hit masks from a ballot.
-// The ray, the walk and the best hit are kept alike in all eight lanes; the
-// stack is in LDS (one wave, eight rays, per block). Bound by the latency of a
-// ray's steps (a node, then a leaf's index and triangle), of which eight times
-// as many waves now overlap: 16,384 rays against 2M triangles take 87 instead
-// of 361 us (primary, surface), 160 instead of 642 us (primary, uniform).
-constexpr int kGroupThreads = 64;
-constexpr uint32_t kGroupRays = kGroupThreads / 8;
+// A group of hit children still to visit: their parent's child base, and its
+// inner mask | hits << 8 with the hit of slot s at bit s ^ oct, so that the
+// lowest is the next.
+__device__ __forceinline__ uint32_t in_octant_order(uint32_t f, uint32_t oct) {
+    f = (oct & 4u) ? ((f >> 4) | (f << 4)) & 0xFFu : f;
+    f = (oct & 2u) ? ((f >> 2) & 0x33u) | ((f << 2) & 0xCCu) : f;
+    return (oct & 1u) ? ((f >> 1) & 0x55u) | ((f << 1) & 0xAAu) : f;
+}
+__device__ __forceinline__ uint32_t take_child(uint32_t base, uint32_t& group, uint32_t oct) {
+    const uint32_t slot = (uint32_t)__builtin_ctz(group >> 8) ^ oct;
+    group &= group - 0x100u;
+    return base + (uint32_t)__popc(group & ((1u << slot) - 1u));
+}
 
-template <bool INDEXED>
+// Eight lanes per node, lane s of the eight for child slot s, and NODES nodes of
+// a ray at a time: one slab test, and at most one triangle test, per lane and
+// step, the hit masks from a ballot. The ray, the walk and the best hit are kept
+// alike in all the ray's lanes; the stack is in LDS (one wave per block). The
+// next nodes do not depend on the leaves: their loads are issued before the
+// leaves' triangles are fetched and tested.
+//
+// Bound by the latency of a ray's steps (some 1.2 us each where nodes come from
+// memory), so the longest walk decides: two nodes a step nearly halve its steps,
+// for the same instructions per node. 16,384 rays took, with one node a step and
+// the next node loaded after the leaves' tests; with it loaded before; with two
+// nodes a step (us, rays a tenth of the scene long from near its surface):
+//   2.9M slivers 955, 740, 497    28.1M blobs 493, 408, 310
+//   1.1M surface  87,  75,  56    1.9M blobs  203, 169, 127
+// and 4,096 rays in 48K slivers 45, 43 and with four nodes a step 27. Leaf tests
+// spread over the next two steps, so that every load has a step to arrive, took
+// as long or longer (738 and 481 us of the first two).
+//
+// Two or four nodes a step leave at most as many groups per level on the stack:
+// nodes are taken in the stack's order, so a step that takes k nodes of a level
+// has used up every deeper group, and leaves k groups one level down.
+constexpr int kGroupThreads = 64;
+
+template <bool INDEXED, uint32_t NODES>
 __global__ __launch_bounds__(kGroupThreads) void k_trace_group(const nxb_bvh8_node* __restrict__ nodes,
                                                                uint32_t node_count,
                                                                const uint32_t* __restrict__ prim_idx,
                                                                uint32_t prim_count, TriSource tris,
                                                                const nxb_ray* __restrict__ rays, uint32_t ray_count,
                                                                nxb_hit* __restrict__ hits) {
-    __shared__ uint2 stack[kTraceStack][kGroupRays];
-    const uint32_t lane = threadIdx.x, s = lane & 7u, g = lane >> 3;
-    const uint32_t r = blockIdx.x * kGroupRays + g;
+    static_assert(NODES == 1 || NODES == 2 || NODES == 4, "one, two or four nodes a step");
+    constexpr uint32_t kLanes = 8 * NODES, kRays = kGroupThreads / kLanes;
+    constexpr uint32_t kStack = kTraceStack * NODES;
+    __shared__ uint2 stack[kStack][kRays];
+    const uint32_t lane = threadIdx.x, s = lane & 7u, h = lane / 8 % NODES, g = lane / kLanes;
+    const uint32_t r = blockIdx.x * kRays + g;
     if (r >= ray_count) return;
     const float4* rp = reinterpret_cast<const float4*>(rays + r);
     const float4 ra = rp[0], rb = rp[1];
@@ -378,40 +409,102 @@ __global__ __launch_bounds__(kGroupThreads) void k_trace_group(const nxb_bvh8_no
     const uint32_t nox = 32u + s + (ix < 0.0f ? 24u : 0u), fox = 32u + s + (ix < 0.0f ? 0u : 24u);
     const uint32_t noy = 40u + s + (iy < 0.0f ? 24u : 0u), foy = 40u + s + (iy < 0.0f ? 0u : 24u);
     const uint32_t noz = 48u + s + (iz < 0.0f ? 24u : 0u), foz = 48u + s + (iz < 0.0f ? 0u : 24u);
-    auto group_bits = [&](bool p) { return (uint32_t)(ballot(p) >> (lane & 56u)) & 0xFFu; };
-
-    uint32_t sp = 0, visited = 0, node = 0, base = 0, group = 0;
-    while (node < node_count && visited < node_count) {  // (the bound as in k_trace_lane)
-        ++visited;
+    // bit k: lane k of the ray
+    auto ray_bits = [&](bool p) {
+        return (uint32_t)((ballot(p) >> (lane & (64u - kLanes))) & ((1ull << kLanes) - 1u));
+    };
+    struct NodeSlot {  // this slot's part of a node
+        float4 w0;
+        uint2 w1;
+        uint32_t meta, nx, ny, nz, fx, fy, fz;
+    };
+    auto load_slot = [&](uint32_t node) {
         const uint8_t* nb = reinterpret_cast<const uint8_t*>(nodes + node);
-        const float4 w0 = reinterpret_cast<const float4*>(nb)[0];
-        const uint2 w1 = reinterpret_cast<const uint2*>(nb)[2];
-        const uint32_t meta = nb[24u + s];
-        const uint32_t nx = nb[nox], ny = nb[noy], nz = nb[noz], fx = nb[fox], fy = nb[foy], fz = nb[foz];
-        const uint32_t em = __float_as_uint(w0.w), imask = em >> 24;
-        const AxisSlab x = axis_slab(w0.x, exp_scale(em & 0xFFu), o.x, ix);
-        const AxisSlab y = axis_slab(w0.y, exp_scale((em >> 8) & 0xFFu), o.y, iy);
-        const AxisSlab z = axis_slab(w0.z, exp_scale((em >> 16) & 0xFFu), o.z, iz);
-        const bool hit = meta != 0 && slab_hit(x, y, z, (float)nx, (float)ny, (float)nz, (float)fx, (float)fy,
-                                               (float)fz, tmin, best_t);
+        return NodeSlot{reinterpret_cast<const float4*>(nb)[0], reinterpret_cast<const uint2*>(nb)[2], nb[24u + s],
+                        nb[nox], nb[noy], nb[noz], nb[fox], nb[foy], nb[foz]};
+    };
+
+    uint32_t sp = 0, visited = 0, base = 0, group = 0;
+    NodeSlot cur = {};
+    bool more = node_count != 0, have = more && h == 0;  // the root
+    if (have) cur = load_slot(0);
+    while (more) {
+        const uint32_t em = __float_as_uint(cur.w0.w), imask = em >> 24;
+        const AxisSlab x = axis_slab(cur.w0.x, exp_scale(em & 0xFFu), o.x, ix);
+        const AxisSlab y = axis_slab(cur.w0.y, exp_scale((em >> 8) & 0xFFu), o.y, iy);
+        const AxisSlab z = axis_slab(cur.w0.z, exp_scale((em >> 16) & 0xFFu), o.z, iz);
+        const bool hit = have && cur.meta != 0 &&
+                         slab_hit(x, y, z, (float)cur.nx, (float)cur.ny, (float)cur.nz, (float)cur.fx, (float)cur.fy,
+                                  (float)cur.fz, tmin, best_t);
         const bool inner = (imask >> s) & 1u;
-        const uint32_t inner_hits = group_bits(hit && inner);
-        bool found = false;
-        float t = INFINITY, u = 0.0f, w = 0.0f;
+        const uint32_t inner_hits = ray_bits(hit && inner);
         uint32_t prim = NXB_INVALID_IDX;
         if (hit && !inner) {
-            const uint32_t k = w1.y + (meta & 0x1Fu);
-            if (k < prim_count) {
-                prim = prim_idx[k];
-                found = prim < prim_count && intersect<INDEXED>(tris, prim, o, d, tmin, best_t, t, u, w);
+            const uint32_t k = cur.w1.y + (cur.meta & 0x1Fu);
+            if (k < prim_count) prim = prim_idx[k];
+        }
+        // the hit children of the step's nodes, in front of what is left
+        if (inner_hits) {
+            if ((group >> 8) && sp < kStack) stack[sp++][g] = make_uint2(base, group);
+            uint32_t b0 = cur.w1.x, g0 = imask | (in_octant_order((inner_hits >> (8 * h)) & 0xFFu, oct) << 8);
+            if constexpr (NODES == 2) {
+                // the other node's, from the lane eight away
+                const uint32_t b1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b0, 0x128, 0xF, 0xF, true);
+                const uint32_t g1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)g0, 0x128, 0xF, 0xF, true);
+                const bool swap = h ? (inner_hits & 0xFFu) != 0 : (inner_hits & 0xFFu) == 0;
+                if ((inner_hits & 0xFFu) && (inner_hits >> 8) && sp < kStack)
+                    stack[sp++][g] = h ? make_uint2(b0, g0) : make_uint2(b1, g1);
+                b0 = swap ? b1 : b0;
+                g0 = swap ? g1 : g0;
+            }
+            base = b0;
+            group = g0;
+            if constexpr (NODES == 4) {
+                // all to the stack, the first node's on top
+                uint32_t z = 0;
+#pragma unroll
+                for (uint32_t i = 0; i < NODES; ++i) z |= (inner_hits >> (8 * i)) & 0xFFu ? 1u << i : 0u;
+                const uint32_t at = sp + (uint32_t)__popc(z >> (h + 1));
+                if (s == 0 && ((z >> h) & 1u) && at < kStack) stack[at][g] = make_uint2(b0, g0);
+                sp = min(sp + (uint32_t)__popc(z), kStack);
+                group = 0;
+                wave_lds_sync();
             }
         }
-        if (group_bits(found)) {
-            // the group's nearest (then smallest index), taken by all its lanes
-            float bt = found ? t : INFINITY;
-            uint32_t bp = found ? prim : NXB_INVALID_IDX, from = s;
+        // the next nodes
+        uint32_t node = 0;
+        have = false;
 #pragma unroll
-            for (uint32_t x8 = 1; x8 < 8; x8 <<= 1) {
+        for (uint32_t i = 0; i < NODES; ++i) {
+            if ((group >> 8) == 0 && sp != 0) {
+                const uint2 top = stack[--sp][g];
+                base = top.x;
+                group = top.y;
+            }
+            const bool any = (group >> 8) != 0;
+            if (i == 0) more = any;
+            if (any) {
+                const uint32_t c = take_child(base, group, oct);
+                // a tree visits each node at most once: the bound only ends a
+                // walk over a malformed node array
+                if (c >= node_count || ++visited >= node_count) more = false;
+                else if (h == i) {
+                    node = c;
+                    have = true;
+                }
+            }
+        }
+        have = have && more;
+        if (have) cur = load_slot(node);
+        bool found = false;
+        float t = INFINITY, u = 0.0f, w = 0.0f;
+        if (prim < prim_count) found = intersect<INDEXED>(tris, prim, o, d, tmin, best_t, t, u, w);
+        if (ray_bits(found)) {
+            // the ray's nearest (then smallest index), taken by all its lanes
+            float bt = found ? t : INFINITY;
+            uint32_t bp = found ? prim : NXB_INVALID_IDX, from = lane;
+#pragma unroll
+            for (uint32_t x8 = 1; x8 < kLanes; x8 <<= 1) {
                 const float ot = __shfl_xor(bt, (int)x8);
                 const uint32_t op = (uint32_t)__shfl_xor((int)bp, (int)x8);
                 const uint32_t of = (uint32_t)__shfl_xor((int)from, (int)x8);
@@ -422,35 +515,37 @@ __global__ __launch_bounds__(kGroupThreads) void k_trace_group(const nxb_bvh8_no
                 }
             }
             if (bt < best_t || bp < best_prim) {  // bt <= best_t
-                const int src = (int)((lane & 56u) | from);
                 best_t = bt;
                 best_prim = bp;
-                bu = __shfl(u, src);
-                bv = __shfl(w, src);
+                bu = __shfl(u, (int)from);
+                bv = __shfl(w, (int)from);
             }
         }
-        if (inner_hits) {
-            if ((group >> 8) && sp < kTraceStack) stack[sp++][g] = make_uint2(base, group);
-            base = w1.x;
-            group = imask | (inner_hits << 8);
-        }
-        if ((group >> 8) == 0) {
-            if (sp == 0) break;
-            const uint2 top = stack[--sp][g];
-            base = top.x;
-            group = top.y;
-        }
-        node = next_child(base, group, oct);
     }
-    if (s == 0) hits[r] = nxb_hit{best_prim == NXB_INVALID_IDX ? rb.w : best_t, best_prim, bu, bv};
+    if (s == 0 && h == 0) hits[r] = nxb_hit{best_prim == NXB_INVALID_IDX ? rb.w : best_t, best_prim, bu, bv};
 }
 
-// Rays up to which eight lanes take a ray. Over three scenes of 100K and 2M
-// triangles, primary and incoherent, k_trace_group / k_trace_lane take 0.39 to
-// 0.85 times as long at 2^16 rays, 0.48 to 1.12 times at 2^17, 0.73 to 1.51
-// times at 2^18 and 1.3 to 2.1 times at 2^20 (the wave's instructions per ray
-// are about twice k_trace_lane's).
+// Rays up to which k_trace_group takes them, with four, two or one nodes a step
+// (32, 16 or 8 lanes per ray). Over three scenes of 100K and 2M triangles,
+// primary and incoherent (12 cases), times against the kernel for more rays:
+//   four nodes against two    0.61-1.07 at 8,192 rays, 0.76-1.08 at 16,384 (but
+//                             up to 1.17 for short rays near a surface)
+//   two against one           0.69-0.98 at 32,768, 0.83-1.20 at 65,536
+//   one against k_trace_lane  0.48-1.12 at 2^17, 0.73-1.51 at 2^18 (its wave's
+//                             instructions per ray are about twice as many)
+constexpr uint32_t kQuadMaxRays = 1u << 13;
+constexpr uint32_t kPairMaxRays = 1u << 15;
 constexpr uint32_t kGroupMaxRays = 1u << 17;
+
+template <bool INDEXED, uint32_t NODES>
+hipError_t launch_trace_group(const nxb_bvh8_node* nodes, uint32_t node_count, const uint32_t* prim_idx,
+                              uint32_t prim_count, const TriSource& ts, const nxb_ray* rays, uint32_t ray_count,
+                              nxb_hit* hits, hipStream_t s) {
+    constexpr uint32_t per_block = kGroupThreads / (8 * NODES);
+    hipLaunchKernelGGL((k_trace_group<INDEXED, NODES>), dim3((ray_count + per_block - 1) / per_block),
+                       dim3(kGroupThreads), 0, s, nodes, node_count, prim_idx, prim_count, ts, rays, ray_count, hits);
+    return hipGetLastError();
+}
 
 }  // namespace
 
@@ -461,10 +556,10 @@ hipError_t launch_trace(const nxb_bvh8_node* nodes, uint32_t node_count, const u
     if (ray_count == 0) return hipSuccess;
     const TriSource ts{tris, indices, vertex_count};
     if (!stats && ray_count <= kGroupMaxRays) {
-        const uint32_t grid = (ray_count + kGroupRays - 1) / kGroupRays;
-        hipLaunchKernelGGL(indices ? k_trace_group<true> : k_trace_group<false>, dim3(grid), dim3(kGroupThreads), 0, s,
-                           nodes, node_count, prim_idx, prim_count, ts, rays, ray_count, hits);
-        return hipGetLastError();
+        auto launch = indices ? launch_trace_group<true, 1> : launch_trace_group<false, 1>;
+        if (ray_count <= kPairMaxRays) launch = indices ? launch_trace_group<true, 2> : launch_trace_group<false, 2>;
+        if (ray_count <= kQuadMaxRays) launch = indices ? launch_trace_group<true, 4> : launch_trace_group<false, 4>;
+        return launch(nodes, node_count, prim_idx, prim_count, ts, rays, ray_count, hits, s);
     }
     const uint32_t grid = (ray_count + kTraceThreads - 1) / kTraceThreads;
     if (!stats)
