@@ -79,7 +79,7 @@ uint32_t bvh8_first_launches(uint32_t n, uint32_t last_n, uint32_t last_launches
 // Scratch carved from one device buffer. Sizes depend on (n, key bytes).
 struct Layout {
     size_t header, partials, hist, counts, keys_a, keys_b, keys_tmp, vals_b, vals_tmp, parent, recs, csizes, nsize,
-        parent2, work, work2, feat, rtable, rec8;
+        parent2, work, work2, feat, rtable, rec8, ex_node;
     size_t counts_bytes;
     size_t total;
 };
@@ -136,6 +136,7 @@ Layout make_layout(uint32_t n, uint32_t key_bytes, bool full, bool bvh8 = true, 
     L.feat = take(segs * NXB_MLP_FEATURES * sizeof(float));
     L.rtable = take(segs);
     L.rec8 = rec8 && n > 1 ? take((size_t)(n - 1) * 64) : 0;
+    L.ex_node = L.rec8 && bvh8_expands(n) ? take((size_t)(n - 1) * 80) : 0;
     L.total = off;
     return L;
 }
@@ -174,6 +175,10 @@ struct Carved {
     float* feat() const { return reinterpret_cast<float*>(base + L.feat); }
     uint8_t* rtable() const { return base + L.rtable; }
     uint4* rec8() const { return L.rec8 ? reinterpret_cast<uint4*>(base + L.rec8) : nullptr; }
+    // 64 bytes per internal node over the keys, values and H-PLOC's arrays, which
+    // are done with: at least 12 + 8 + 4 + 32 + 8 bytes a primitive
+    uint4* ex_kids() const { return L.ex_node ? reinterpret_cast<uint4*>(base + L.keys_a) : nullptr; }
+    uint4* ex_node() const { return L.ex_node ? reinterpret_cast<uint4*>(base + L.ex_node) : nullptr; }
     uint4* moved_rec() const { return reinterpret_cast<uint4*>(hdr() + kHdrMovedRec); }
 };
 
@@ -514,7 +519,7 @@ nxb_status build_common(const void* prims, nxb_prim_type type, uint32_t n, const
 
     uint32_t cap = nxb_bvh8_capacity(n);
     Bvh8Scratch bs{w.work(), w.bvh8_ctr(), w.bvh8_grab(), w.flags(), w.nsize(), w.work2(), cfg.slot_assignment,
-                   w.rec8()};
+                   w.rec8(), w.ex_kids(), w.ex_node()};
     st = prep_bvh2(n, cfg, w, s);
     if (!st && out8) {
         st = alloc_out((void**)&ob.n8, (size_t)cap * sizeof(nxb_bvh8_node), s);

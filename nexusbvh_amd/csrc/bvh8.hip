@@ -445,15 +445,32 @@ __device__ __forceinline__ void emit_node(const ChildBoxes& cbx, uint32_t tid, c
     write_bvh8_node(out, k, c.pb, cbx, tid, child_base, leaf_count ? prim_base : 0u, c.assign, c.im, c.lm);
 }
 
-// Inclusive sum over the 64 lanes of a wave.
+// The value N lanes back in the same row of 16 (row_shr:N), 0 at its start and
+// from inactive lanes: never inside a branch or a ?: arm.
+template <int N>
+__device__ __forceinline__ uint32_t lane_back(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x110 + N, 0xF, 0xF, true);
+}
+
+// Inclusive sum over the 64 lanes of a wave, by lane shifts of the vector units
+// (rows of 16, then the rows' totals); six shuffles through LDS took six round
+// trips. All lanes of the wave are active.
 __device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
-    const uint32_t lane = lane_id();
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        uint32_t y = __shfl_up(v, off);
-        if (lane >= (uint32_t)off) v += y;
-    }
+    v += lane_back<1>(v);
+    v += lane_back<2>(v);
+    v += lane_back<4>(v);
+    v += lane_back<8>(v);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);  // row_bcast:15 to rows 1, 3
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);  // row_bcast:31 to rows 2, 3
     return v;
+}
+
+// Barrier of the block for data in LDS alone: global stores in flight, which
+// only later kernels read, are not waited for as __syncthreads() does.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // n leaves; node_count = 2n - 1 for one BVH2, 2n - (trees) for a forest
@@ -588,11 +605,13 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8(const nxb_bvh2_node* __re
 constexpr uint32_t kMaxLevels = kBvh8LevelWords - 1;  // BVH8 levels; each consumes at least one BVH2 level
 
 // Exclusive scan over a 256-thread block; *total gets the block sum.
+template <bool LDS_ONLY = false>
 __device__ __forceinline__ uint32_t block_scan_256(uint32_t v, uint32_t* tmp, uint32_t* total) {
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const uint32_t incl = wave_inclusive_sum(v);
     if (lane == 63) tmp[w] = incl;
-    __syncthreads();
+    if (LDS_ONLY) lds_barrier();
+    else __syncthreads();
     uint32_t before = 0, all = 0;
 #pragma unroll
     for (uint32_t k = 0; k < kBvh8Threads / 64; ++k) {
@@ -600,7 +619,8 @@ __device__ __forceinline__ uint32_t block_scan_256(uint32_t v, uint32_t* tmp, ui
         if (k < w) before += t;
         all += t;
     }
-    __syncthreads();
+    if (LDS_ONLY) lds_barrier();
+    else __syncthreads();
     *total = all;
     return before + incl - v;
 }
@@ -705,7 +725,7 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_level(const uint4* __rest
     }
 }
 
-// ---- few launches (single builds of small meshes) ---------------------------
+// ---- few launches (single builds up to 2^21 primitives) ----------------------
 //
 // One lane collapses one node; a block reserves the ids of its nodes' inner
 // children with one atomic add on the node counter and passes the children on
@@ -717,9 +737,10 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_level(const uint4* __rest
 //
 // What bounds it is latency: a node costs its lane up to seven dependent record
 // loads (~1,300 cycles each with the choice of the next), then the slots and
-// the quantization. A level took 15 to 17 us as a launch of its own (counters,
-// queue and a cold L2 first), and a mesh has log2(n) of them, since a node's
-// largest child keeps half of its primitives. Inside a block a level is ~7 us.
+// the quantization, and a mesh has log2(n) levels, since a node's largest child
+// keeps half of its primitives. A level took 15 to 17 us as a launch of its own
+// (counters, queue and a cold L2 first), ~7 us inside a block. Up to
+// kExpandPrims that work is taken out of the levels (k_bvh8_expand).
 // The children of the node each lane collapses, in LDS (child t of lane i at
 // [t][i]): box, id (a leaf is an id below n, its primitive index) and
 // primitive count. Indexed by slot when they are read back, which in
@@ -744,8 +765,9 @@ __device__ __forceinline__ Box get_child_box(const RecChildren& ch, uint32_t t, 
 // Collapse of internal node x (record x - n). Same push/pop order as
 // collapse_node; the node's box is the union of its children's (as H-PLOC
 // formed it, bit for bit). False for an id out of range.
-__device__ __forceinline__ bool collapse_children(const uint4* rec, uint32_t n, uint32_t node_count, uint32_t x, Box& pb,
-                                             uint32_t& count, uint32_t& inner, RecChildren& ch, uint32_t tid) {
+__device__ __forceinline__ bool collapse_children(const uint4* rec, uint32_t n, uint32_t node_count, uint32_t x,
+                                                  Box& pb, uint32_t& count, uint32_t& inner, RecChildren& ch,
+                                                  uint32_t tid) {
     if (x < n || x >= node_count) return false;
     inner = 0;
     uint32_t top = 0, msb = 0, cur = x;  // top: the last slot in use
@@ -826,13 +848,6 @@ __device__ __forceinline__ uint32_t auction_slots(const Box& pb, const RecChildr
     return auction_assign(pb, ox, oy, oz, count);
 }
 
-// What the lanes that emit a node need to know of it.
-struct RecNodes {
-    float4 a[kBvh8Threads];  // box: lx, ly, lz, hx
-    uint4 b[kBvh8Threads];   // hy, hz, children | inner-child bits << 8, first primitive
-    uint2 c[kBvh8Threads];   // BVH8 id, inner children of the block's earlier nodes
-};
-
 // Work items passed on inside a block.
 struct BlockQueue {
     uint32_t x[kBvh8Threads], base[kBvh8Threads], id[kBvh8Threads];
@@ -877,20 +892,20 @@ __device__ __forceinline__ uint32_t grid_exponents(const Box& pb, float& ix, flo
     return e0 | (e1 << 8) | (e2 << 16);
 }
 
-// Emits the node of one lane: primIdx entries of its leaves, work items of its
-// inner children, the 80 bytes. Primitive ranges are fixed top-down: a node's
-// leaves take the front of its range, then each inner child, in slot order, a
-// range of its primitive count.
-__device__ __forceinline__ bool emit_lane(const RecChildren& ch, uint32_t tid, const Box& pb, uint32_t count,
-                                          uint32_t inner, uint32_t assign, uint32_t base, uint32_t id, uint32_t excl,
-                                          const ChildSink& sink, nxb_bvh8_node* out, uint32_t* prim_idx) {
-    const uint32_t ic = (uint32_t)__popc(inner), leaf_count = count - ic;
+// A node's 80 bytes without the child and primitive bases, and its children by
+// slot: id (kInvalid: free) and primitive count (0: a leaf or free).
+struct PackedNode {
+    uint4 w[5];
+    uint32_t kid[8], prims[8];
+};
+__device__ __forceinline__ PackedNode pack_node(const RecChildren& ch, uint32_t tid, const Box& pb, uint32_t inner,
+                                                uint32_t assign) {
+    PackedNode r;
     float ix, iy, iz;
     const uint32_t e = grid_exponents(pb, ix, iy, iz);
-    uint32_t next_base = base + leaf_count, leaves = 0, nth = 0, im = 0;
+    uint32_t leaves = 0, im = 0;
     uint32_t meta[2] = {0, 0}, qlx[2] = {0, 0}, qly[2] = {0, 0}, qlz[2] = {0, 0};
     uint32_t qhx[2] = {0, 0}, qhy[2] = {0, 0}, qhz[2] = {0, 0};
-    bool good = true;
 #pragma unroll
     for (uint32_t s = 0; s < 8; ++s) {
         // (an empty slot computes on child 7's words and keeps zeros)
@@ -907,133 +922,66 @@ __device__ __forceinline__ bool emit_lane(const RecChildren& ch, uint32_t tid, c
         put(qhy, q_ceil((__uint_as_float(cb.x) - pb.ly) * iy));
         put(qhz, q_ceil((__uint_as_float(cb.y) - pb.lz) * iz));
         put(meta, (1u << 5) | (in ? 24u + s : leaves));
-        if (in) {
-            im |= 1u << s;
-            good &= sink.put(excl + nth, cb.z, next_base, cb.w);
-            next_base += cb.w;
+        r.kid[s] = used ? cb.z : kInvalid;
+        r.prims[s] = in ? cb.w : 0u;
+        im |= in ? 1u << s : 0u;
+        leaves += used && !in ? 1u : 0u;
+    }
+    r.w[0] = make_uint4(__float_as_uint(pb.lx), __float_as_uint(pb.ly), __float_as_uint(pb.lz), e | (im << 24));
+    r.w[1] = make_uint4(0u, 0u, meta[0], meta[1]);
+    r.w[2] = make_uint4(qlx[0], qlx[1], qly[0], qly[1]);
+    r.w[3] = make_uint4(qlz[0], qlz[1], qhx[0], qhx[1]);
+    r.w[4] = make_uint4(qhy[0], qhy[1], qhz[0], qhz[1]);
+    return r;
+}
+
+// Emits the node of one lane: primIdx entries of its leaves, work items of its
+// inner children, the 80 bytes. Primitive ranges are fixed top-down: a node's
+// leaves take the front of its range, then each inner child, in slot order, a
+// range of its primitive count.
+__device__ __forceinline__ bool emit_lane(const RecChildren& ch, uint32_t tid, const Box& pb, uint32_t count,
+                                          uint32_t inner, uint32_t assign, uint32_t base, uint32_t id, uint32_t excl,
+                                          const ChildSink& sink, nxb_bvh8_node* out, uint32_t* prim_idx) {
+    const uint32_t ic = (uint32_t)__popc(inner), leaf_count = count - ic;
+    PackedNode r = pack_node(ch, tid, pb, inner, assign);
+    uint32_t next_base = base + leaf_count, leaves = 0, nth = 0;
+    bool good = true;
+#pragma unroll
+    for (uint32_t s = 0; s < 8; ++s) {
+        if (r.prims[s]) {
+            good &= sink.put(excl + nth, r.kid[s], next_base, r.prims[s]);
+            next_base += r.prims[s];
             ++nth;
-        } else if (used) {
-            if (base + leaves < sink.n) prim_idx[base + leaves] = cb.z;
+        } else if (r.kid[s] != kInvalid) {
+            if (base + leaves < sink.n) prim_idx[base + leaves] = r.kid[s];
             else good = false;
             ++leaves;
         }
     }
+    r.w[1].x = ic ? sink.ids + excl : 0u;
+    r.w[1].y = leaf_count ? base : 0u;
     uint4* o = reinterpret_cast<uint4*>(out + id);
-    o[0] = make_uint4(__float_as_uint(pb.lx), __float_as_uint(pb.ly), __float_as_uint(pb.lz), e | (im << 24));
-    o[1] = make_uint4(ic ? sink.ids + excl : 0u, leaf_count ? base : 0u, meta[0], meta[1]);
-    o[2] = make_uint4(qlx[0], qlx[1], qly[0], qly[1]);
-    o[3] = make_uint4(qlz[0], qlz[1], qhx[0], qhx[1]);
-    o[4] = make_uint4(qhy[0], qhy[1], qhz[0], qhz[1]);
-    return good;
-}
-
-// Value of another lane of the same eight: lane ^ 1, lane ^ 2, and (for values
-// alike in each four lanes) lane ^ 4.
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141;
-// Lane K of each eight (ds_swizzle, bit-mask mode: lane & 0x18 | K).
-template <int K>
-__device__ __forceinline__ float lane_of_8(float v) {
-    return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (K << 5) | 0x18));
-}
-
-// Slot choice of child K (greedy_assign): lane s holds slot s (mine: its child,
-// 8 while free) and, as child s, the offsets ox, oy, oz.
-template <uint32_t K>
-__device__ __forceinline__ void greedy_step(float ox, float oy, float oz, uint32_t s, uint32_t count, uint64_t lower,
-                                            uint32_t& mine) {
-    const float lowest = -3.402823466e+38f;
-    const float kx = lane_of_8<K>(ox), ky = lane_of_8<K>(oy), kz = lane_of_8<K>(oz);
-    const float cost = ((s & 4u ? -kx : kx) + (s & 2u ? -ky : ky)) + (s & 1u ? -kz : kz);
-    const bool free_slot = mine == 8u;
-    float most = free_slot ? fmaxf(cost, lowest) : lowest;
-    most = fmaxf(most, dpp_f<kDppXor1>(most));
-    most = fmaxf(most, dpp_f<kDppXor2>(most));
-    most = fmaxf(most, dpp_f<kDppHalfMirror>(most));
-    const bool fits = K < count && free_slot && (cost == most || !(most > lowest));
-    if (fits && (ballot(fits) & lower) == 0) mine = K;
-    if constexpr (K < 7) greedy_step<K + 1>(ox, oy, oz, s, count, lower, mine);
-}
-
-// Emits `nodes` nodes of the block, eight lanes per node and one slot per lane
-// (greedy slots): the same results as greedy_assign and emit_lane. A wave takes
-// eight nodes at a time; their 640 bytes are put together in LDS.
-__device__ __forceinline__ bool emit_groups(const RecChildren& ch, const RecNodes& nd, uint32_t nodes,
-                                            uint8_t (*stage)[8 * sizeof(nxb_bvh8_node)], const ChildSink& sink,
-                                            nxb_bvh8_node* out, uint32_t* prim_idx) {
-    const uint32_t tid = threadIdx.x, w = tid >> 6, lane = tid & 63u, s = lane & 7u, g = lane >> 3;
-    const uint64_t lower = ((1ull << lane) - 1ull) & (0xFFull << (lane & 56u));  // earlier lanes of the eight
-    uint8_t* st = stage[w] + g * sizeof(nxb_bvh8_node);
-    bool good = true;
-    for (uint32_t j0 = w * 8; j0 < nodes; j0 += kBvh8Threads / 8) {
-        const uint32_t j = min(j0 + g, nodes - 1);
-        const float4 na = nd.a[j];
-        const uint4 nb = nd.b[j];
-        const uint2 nc = nd.c[j];
-        const Box pb = {na.x, na.y, na.z, na.w, __uint_as_float(nb.x), __uint_as_float(nb.y)};
-        const uint32_t count = j0 + g < nodes ? nb.z & 0xFFu : 0u, inner = nb.z >> 8, base = nb.w;
-        // as child s
-        uint32_t mine = 8u;
-        {
-            const Box cb = get_child_box(ch, s, j);
-            greedy_step<0>((pb.lx + pb.hx) - (cb.hx + cb.lx), (pb.ly + pb.hy) - (cb.hy + cb.ly),
-                           (pb.lz + pb.hz) - (cb.hz + cb.lz), s, count, lower, mine);
-        }
-        // as slot s
-        const bool used = mine < 8u, in = used && ((inner >> (mine & 7u)) & 1u);
-        const float4 ca = ch.a[mine & 7u][j];
-        const uint4 cb = ch.b[mine & 7u][j];
-        const uint32_t im = (uint32_t)(ballot(in) >> (lane & 56u)) & 0xFFu;
-        const uint32_t lm = (uint32_t)(ballot(used && !in) >> (lane & 56u)) & 0xFFu;
-        const uint32_t leaf_count = (uint32_t)__popc(lm), leaf = bits_below(lm, s);
-        uint32_t before = in ? cb.w : 0u;  // primitives of the inner slots up to this one
 #pragma unroll
-        for (uint32_t off = 1; off < 8; off <<= 1) {
-            const uint32_t v = (uint32_t)__shfl_up((int)before, off);
-            before += s >= off ? v : 0u;
-        }
-        if (in) good &= sink.put(nc.y + bits_below(im, s), cb.z, base + leaf_count + before - cb.w, cb.w);
-        if (used && !in) {
-            if (base + leaf < sink.n) prim_idx[base + leaf] = cb.z;
-            else good = false;
-        }
-        float ix, iy, iz;
-        const uint32_t e = grid_exponents(pb, ix, iy, iz);
-        auto put = [&](uint32_t k, uint32_t v) { st[24 + 8 * k + s] = (uint8_t)(used ? v : 0u); };
-        put(0, (1u << 5) | (in ? 24u + s : leaf));
-        put(1, q_floor((ca.x - pb.lx) * ix));
-        put(2, q_floor((ca.y - pb.ly) * iy));
-        put(3, q_floor((ca.z - pb.lz) * iz));
-        put(4, q_ceil((ca.w - pb.lx) * ix));
-        put(5, q_ceil((__uint_as_float(cb.x) - pb.ly) * iy));
-        put(6, q_ceil((__uint_as_float(cb.y) - pb.lz) * iz));
-        if (s == 0) {
-            uint2* h = reinterpret_cast<uint2*>(st);
-            h[0] = make_uint2(__float_as_uint(pb.lx), __float_as_uint(pb.ly));
-            h[1] = make_uint2(__float_as_uint(pb.lz), e | (im << 24));
-            h[2] = make_uint2(im ? sink.ids + nc.y : 0u, leaf_count ? base : 0u);
-        }
-        wave_lds_sync();
-        const uint32_t k = lane / 5u, part = lane - 5u * k;  // 16 bytes of node j0 + k
-        if (k < 8 && j0 + k < nodes && (nd.b[j0 + k].z & 0xFFu) != 0)
-            reinterpret_cast<uint4*>(out + nd.c[j0 + k].x)[part] =
-                *reinterpret_cast<const uint4*>(stage[w] + k * sizeof(nxb_bvh8_node) + part * 16);
-        wave_lds_sync();
-    }
+    for (uint32_t i = 0; i < 5; ++i) o[i] = r.w[i];
     return good;
 }
 
-// Primitives up to which a build takes the kernel below; above, one launch per
-// level (three blocks of 48 KB LDS per CU where this one has two). Collapse
-// stage, us, launches that follow subtrees / a launch per level, on a surface,
-// blobs and slivers: 82/147, 65/109, 66/110 at 2,003; 119/201, 113/193, 101/169
-// at 48K; 134/207, 165/245, 140/209 at 300K; 240/254, 262/300, 244/265 at 1.1M;
-// 269/296, 318/343, 280/307 at 2M; 345/357, 415/388, 325/337 at 3M.
+// Primitives up to which a build takes launches that follow subtrees; above, one
+// launch per level (three blocks of 48 KB LDS per CU where k_bvh8_collapse has
+// two). Collapse stage in us, k_bvh8_collapse / a launch per level, on a
+// surface, blobs and slivers: 250/254, 273/300, 259/265 at 1.1M; 276/296,
+// 323/343, 287/307 at 2M; 345/357, 415/388, 325/337 at 3M.
 constexpr uint32_t kSmallPrims = 1u << 21;
 bool bvh8_small(uint32_t n) { return n <= kSmallPrims; }
+
+// Primitives up to which every internal BVH2 node is expanded first: all of them
+// is about five times the nodes that the BVH8 needs, but at once instead of
+// level after level. Collapse stage in us, surface, blobs and slivers,
+// k_bvh8_expand and k_bvh8_place / k_bvh8_collapse: 32/92, 28/72, 28/71 at
+// 2,003; 53/136, 51/132, 47/117 at 48K; 96/148, 109/179, 102/156 at 300K;
+// 211/250, 246/273, 215/259 at 1.1M; 347/276, 389/323, 353/287 at 2M.
+constexpr uint32_t kExpandPrims = 5u << 18;
+bool bvh8_expands(uint32_t n) { return n <= kExpandPrims; }
 
 // Levels that a block follows while the queue grows, by queued nodes: a node's
 // children hold about 1/2, 1/4, 1/8, ... of its primitives (the larger child is
@@ -1041,11 +989,9 @@ bool bvh8_small(uint32_t n) { return n <= kSmallPrims; }
 // hold up the launch (300K triangles: 181 to 230 us without the limits). 4096
 // and 16384 instead measured within 5%.
 constexpr uint32_t kThreeLevelNodes = 2048, kTwoLevelNodes = 32768;
-
-// Nodes of a block up to which eight lanes emit a node (emit_groups: ~2,000
-// cycles per 32 nodes of a block; greedy_assign and emit_lane: ~8,500 cycles
-// however few). 32 and 96 measured alike, 256 a tenth slower.
-constexpr uint32_t kGroupNodes = 96;
+__device__ __forceinline__ uint32_t levels_to_follow(uint32_t m) {
+    return m <= kThreeLevelNodes ? 3u : m <= kTwoLevelNodes ? 2u : 1u;
+}
 
 // work[q] = (first primitive << 32 | BVH2 id), work2[q] = (level << 32 | BVH8
 // id) of queue position q. alloc counts the nodes below the root (the root is
@@ -1057,9 +1003,7 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_collapse(const uint4* __r
                                                                 uint64_t* work, uint64_t* work2, uint32_t* cnt,
                                                                 uint32_t launch, uint32_t* alloc, uint32_t* flags) {
     __shared__ RecChildren ch;
-    __shared__ RecNodes nd;
     __shared__ BlockQueue bq;
-    __shared__ __attribute__((aligned(16))) uint8_t stage[kBvh8Threads / 64][8 * sizeof(nxb_bvh8_node)];
     __shared__ uint32_t scan_tmp[kBvh8Threads / 64];
     __shared__ uint32_t sids, squeue, slevel;
     const uint32_t tid = threadIdx.x;
@@ -1074,7 +1018,7 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_collapse(const uint4* __r
     // levels before the rest goes to the queue: all in the first launch and
     // once the queue shrinks, else few enough that no block runs on alone
     uint32_t left = kMaxLevels;
-    if (launch != 0 && (launch == 1 || m >= cnt[launch - 1])) left = m <= kThreeLevelNodes ? 3u : m <= kTwoLevelNodes ? 2u : 1u;
+    if (launch != 0 && (launch == 1 || m >= cnt[launch - 1])) left = levels_to_follow(m);
     const uint32_t per = follow ? (m + gridDim.x - 1) / gridDim.x : (uint32_t)kBvh8Threads;
     for (uint32_t i0 = blockIdx.x * per; i0 < m; i0 += gridDim.x * per) {
         uint32_t nodes = min(per, m - i0);
@@ -1103,26 +1047,15 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_collapse(const uint4* __r
             uint32_t total = 0;
             const uint32_t excl = block_scan_256(ic, scan_tmp, &total);
             const bool keep = follow && --left != 0 && total <= (uint32_t)kBvh8Threads;
-            const bool groups = SLOT == NXB_SLOT_GREEDY && nodes <= kGroupNodes;
             if (tid == 0) sids = total ? 1u + atomic_add_agent(alloc, total) : 0u;
             if (tid == 64) squeue = total && !keep ? hi + atomic_add_agent(&cnt[launch + 1], total) : 0u;
             uint32_t assign = 0xFFFFFFFFu;
-            if (groups) {
-                if (has) {
-                    nd.a[tid] = make_float4(pb.lx, pb.ly, pb.lz, pb.hx);
-                    nd.b[tid] = make_uint4(__float_as_uint(pb.hy), __float_as_uint(pb.hz),
-                                           ok ? count | (inner << 8) : 0u, base);
-                    nd.c[tid] = make_uint2(id, excl);
-                }
-            } else if (ok) {
+            if (ok)
                 assign = SLOT == NXB_SLOT_AUCTION ? auction_slots(pb, ch, tid, count)
                                                   : greedy_assign(pb, ch, tid, count);
-            }
             __syncthreads();
             const ChildSink sink{&bq, keep, sids, squeue, level + 1, work, work2, capacity, n};
-            if (groups)
-                good &= emit_groups(ch, nd, nodes, stage, sink, out, prim_idx);
-            else if (ok)
+            if (ok)
                 good &= emit_lane(ch, tid, pb, count, inner, assign, base, id, excl, sink, out, prim_idx);
             if (!good) atomic_or_agent(flags, kFlagBadIndex);
             __syncthreads();  // the block's queue is written, sids and squeue are read
@@ -1135,6 +1068,207 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_collapse(const uint4* __r
                 id = bq.id[tid];
             }
         }
+    }
+}
+
+// ---- every node expanded first (single builds of small meshes) --------------
+//
+// What a BVH8 node looks like depends on its BVH2 node alone, except for the
+// numbers of its children and primitives. So one launch makes the BVH8 node of
+// every internal BVH2 node, side by side: the chain of seven record loads, the
+// slots and the quantization are waited for once instead of once per level. The
+// levels that follow only hand out numbers: a level inside a block is two loads,
+// a count and the writes (~2,500 cycles, 1,300 to 2,700 of them the loads'),
+// where collapsing the nodes took ~17,000. 2,003 primitives: 10 us and 18 us;
+// 300K: 34 us and four launches of 6 to 20 us.
+
+// Per internal BVH2 node x, at x - n: its BVH8 node.
+//   kids: 8 ids by slot (kInvalid: free), 8 primitive counts (0: a leaf or free)
+//   node: its 80 bytes, without the child and primitive bases
+struct Expanded {
+    uint4* kids;  // 4 each
+    uint4* node;  // 5 each
+};
+
+template <uint32_t SLOT>
+__global__ __launch_bounds__(kBvh8Threads) void k_bvh8_expand(const uint4* __restrict__ rec, uint32_t n,
+                                                              uint32_t node_count, Expanded ex, uint32_t* flags) {
+    __shared__ RecChildren ch;
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t i = blockIdx.x * kBvh8Threads + tid; i < n - 1; i += gridDim.x * kBvh8Threads) {
+        Box pb = {0, 0, 0, 0, 0, 0};
+        uint32_t count = 0, inner = 0;
+        if (!collapse_children(rec, n, node_count, n + i, pb, count, inner, ch, tid)) {
+            atomic_or_agent(flags, kFlagBadIndex);
+            const uint4 none = make_uint4(kInvalid, kInvalid, kInvalid, kInvalid), zero = make_uint4(0, 0, 0, 0);
+            ex.kids[4ull * i] = none;
+            ex.kids[4ull * i + 1] = none;
+            ex.kids[4ull * i + 2] = zero;
+            ex.kids[4ull * i + 3] = zero;
+            continue;
+        }
+        const uint32_t assign =
+            SLOT == NXB_SLOT_AUCTION ? auction_slots(pb, ch, tid, count) : greedy_assign(pb, ch, tid, count);
+        const PackedNode r = pack_node(ch, tid, pb, inner, assign);
+        uint4* k = ex.kids + 4ull * i;
+        k[0] = make_uint4(r.kid[0], r.kid[1], r.kid[2], r.kid[3]);
+        k[1] = make_uint4(r.kid[4], r.kid[5], r.kid[6], r.kid[7]);
+        k[2] = make_uint4(r.prims[0], r.prims[1], r.prims[2], r.prims[3]);
+        k[3] = make_uint4(r.prims[4], r.prims[5], r.prims[6], r.prims[7]);
+        uint4* o = ex.node + 5ull * i;
+#pragma unroll
+        for (uint32_t j = 0; j < 5; ++j) o[j] = r.w[j];
+    }
+}
+
+// Numbers the nodes from the root down, launches and queues as in
+// k_bvh8_collapse. Eight lanes take a node, one its slot: a block's pass places
+// 32 nodes, and the node's words go out in three coalesced stores. (One lane per
+// node: 38 us at 2,003 primitives and 105 at 300K for both kernels, now 31 and
+// 96.) At least kPlaceShare nodes per block: each block and level costs two
+// atomic adds on the same two counters (10 ns each).
+__global__ __launch_bounds__(kBvh8Threads) void k_bvh8_place(Expanded ex, uint32_t n, uint32_t node_count,
+                                                             nxb_bvh8_node* __restrict__ out,
+                                                             uint32_t* __restrict__ prim_idx, uint32_t capacity,
+                                                             uint64_t* work, uint64_t* work2, uint32_t* cnt,
+                                                             uint32_t launch, uint32_t* alloc, uint32_t* flags) {
+    constexpr uint32_t kPlaceNodes = kBvh8Threads / 8, kPlacePasses = 8, kPlaceShare = 4;
+    __shared__ BlockQueue bq[2];
+    __shared__ uint32_t scan_tmp[2][kBvh8Threads / 64];
+    __shared__ uint32_t sids, squeue, slevel;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6, s = tid & 7u, g = tid >> 3;
+    const uint32_t m = launch == 0 ? 1u : min(cnt[launch], capacity);
+    if (m == 0) return;
+    uint32_t lo = 0;
+    for (uint32_t j = 1; j < launch; ++j) lo += cnt[j];
+    const uint32_t hi = launch == 0 ? 0u : lo + m;
+    const bool follow = m <= gridDim.x * kBvh8Threads;
+    uint32_t left = kMaxLevels;
+    if (launch != 0 && (launch == 1 || m >= cnt[launch - 1])) left = levels_to_follow(m);
+    const uint32_t per = follow ? max((m + gridDim.x - 1) / gridDim.x, kPlaceShare) : (uint32_t)kBvh8Threads;
+    for (uint32_t i0 = blockIdx.x * per; i0 < m; i0 += gridDim.x * per) {
+        uint32_t nodes = min(per, m - i0), level = 0, cur = 0;
+        uint32_t below = 1;  // launch 0, one block: ids given out
+        if (launch == 0) {
+            if (tid == 0) {  // the root
+                bq[0].x[0] = node_count - 1;
+                bq[0].base[0] = 0;
+                bq[0].id[0] = 0;
+            }
+        } else {
+            if (tid == 0) slevel = 0;
+            lds_barrier();
+            if (tid < nodes) {
+                const bool has = lo + i0 + tid < capacity;
+                const uint64_t v = has ? work[lo + i0 + tid] : (uint64_t)kInvalid;
+                const uint64_t v2 = has ? work2[lo + i0 + tid] : 0ull;
+                bq[0].x[tid] = (uint32_t)v;
+                bq[0].base[tid] = (uint32_t)(v >> 32);
+                bq[0].id[tid] = (uint32_t)v2;
+                atomicMax(&slevel, (uint32_t)(v2 >> 32));
+            }
+        }
+        lds_barrier();
+        if (launch != 0) level = slevel;  // the deepest of the share: a bound for its levels
+        for (;;) {
+            // what each lane places: slot s of the node of its eight in pass p
+            uint32_t kid[kPlacePasses], prims[kPlacePasses], img[kPlacePasses][3], ic = 0;
+#pragma unroll
+            for (uint32_t p = 0; p < kPlacePasses; ++p) {
+                kid[p] = kInvalid;
+                prims[p] = 0;
+                img[p][0] = img[p][1] = img[p][2] = 0;
+                const uint32_t j = p * kPlaceNodes + g;
+                if (p * kPlaceNodes < nodes && j < nodes) {
+                    const uint32_t x = bq[cur].x[j];
+                    if (x >= n && x < node_count && bq[cur].id[j] < capacity && level < kMaxLevels) {
+                        const uint32_t* k = reinterpret_cast<const uint32_t*>(ex.kids + 4ull * (x - n));
+                        const uint32_t* o = reinterpret_cast<const uint32_t*>(ex.node + 5ull * (x - n));
+                        prims[p] = k[8 + s];
+                        kid[p] = k[s];
+                        img[p][0] = o[s];
+                        img[p][1] = o[8 + s];
+                        img[p][2] = o[16 + (s & 3u)];
+                    } else {
+                        atomic_or_agent(flags, kFlagBadIndex);
+                    }
+                }
+            }
+#pragma unroll
+            for (uint32_t p = 0; p < kPlacePasses; ++p)
+                if (p * kPlaceNodes < nodes) ic += (uint32_t)__popcll(ballot(prims[p] != 0));
+            if (lane == 0) scan_tmp[cur][w] = ic;
+            lds_barrier();
+            uint32_t at = 0, total = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < kBvh8Threads / 64; ++k) {
+                const uint32_t t = scan_tmp[cur][k];
+                at += k < w ? t : 0u;
+                total += t;
+            }
+            const bool keep = follow && --left != 0 && total <= (uint32_t)kBvh8Threads;
+            uint32_t ids = below, queue = 0;
+            if (launch == 0) {
+                below += total;
+                if (tid == 0 && !(keep && total)) {
+                    *alloc = below - 1;
+                    cnt[1] = total;
+                }
+            } else {
+                if (tid == 0) sids = total ? 1u + atomic_add_agent(alloc, total) : 0u;
+                if (tid == 64) squeue = total && !keep ? hi + atomic_add_agent(&cnt[launch + 1], total) : 0u;
+                lds_barrier();
+                ids = sids;
+                queue = squeue;
+            }
+            const ChildSink sink{&bq[cur ^ 1], keep, ids, queue, level + 1, work, work2, capacity, n};
+            bool good = true;
+#pragma unroll
+            for (uint32_t p = 0; p < kPlacePasses; ++p) {
+                if (p * kPlaceNodes >= nodes) break;
+                const uint32_t j = min(p * kPlaceNodes + g, nodes - 1);
+                const uint32_t x = bq[cur].x[j], base = bq[cur].base[j], id = bq[cur].id[j];
+                const bool ok = p * kPlaceNodes + g < nodes && x >= n && x < node_count && id < capacity &&
+                                level < kMaxLevels;
+                const bool in = prims[p] != 0, leaf = !in && kid[p] != kInvalid;
+                const uint64_t ib = ballot(in);
+                const uint32_t im = (uint32_t)(ib >> (lane & 56u)) & 0xFFu;
+                const uint32_t lm = (uint32_t)(ballot(leaf) >> (lane & 56u)) & 0xFFu;
+                const uint32_t leaves = (uint32_t)__popc(lm);
+                const uint32_t first = at + (uint32_t)__popcll(ib & ((1ull << (lane & 56u)) - 1ull));  // its children
+                uint32_t before = prims[p];  // primitives of the inner slots up to this one
+                const uint32_t back1 = lane_back<1>(before);  // (all lanes take part in each shift)
+                before += s >= 1 ? back1 : 0u;
+                const uint32_t back2 = lane_back<2>(before);
+                before += s >= 2 ? back2 : 0u;
+                const uint32_t back4 = lane_back<4>(before);
+                before += s >= 4 ? back4 : 0u;
+                if (in)
+                    good &= sink.put(first + bits_below(im, s), kid[p], base + leaves + before - prims[p], prims[p]);
+                if (leaf) {
+                    const uint32_t q = base + bits_below(lm, s);
+                    if (q < n) prim_idx[q] = kid[p];
+                    else good = false;
+                }
+                if (ok) {
+                    uint32_t* dst = reinterpret_cast<uint32_t*>(out + id);
+                    uint32_t v = img[p][0];
+                    if (s == 4) v = im ? ids + first : 0u;
+                    if (s == 5) v = leaves ? base : 0u;
+                    dst[s] = v;
+                    dst[8 + s] = img[p][1];
+                    if (s < 4) dst[16 + s] = img[p][2];
+                }
+                at += (uint32_t)__popcll(ib);
+            }
+            if (!good) atomic_or_agent(flags, kFlagBadIndex);
+            if (!keep || total == 0) break;
+            lds_barrier();  // the next level's queue is written
+            nodes = total;
+            ++level;
+            cur ^= 1;
+        }
+        lds_barrier();  // the queue is read before the next share fills it
     }
 }
 
@@ -1471,10 +1605,23 @@ hipError_t launch_bvh8_collapse(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_
     if (!sc.rec8 || !sc.work2) return hipErrorInvalidValue;
     const bool auction = sc.slot_mode == NXB_SLOT_AUCTION;
     if (bvh8_small(n)) {
-        auto kernel = auction ? k_bvh8_collapse<NXB_SLOT_AUCTION> : k_bvh8_collapse<NXB_SLOT_GREEDY>;
-        // two blocks of 80 KB LDS per CU
-        const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 2u);
         const uint32_t end = min(from + count, kMaxLevels);
+        if (bvh8_expands(n)) {
+            if (!sc.ex_kids || !sc.ex_node) return hipErrorInvalidValue;
+            const Expanded ex{sc.ex_kids, sc.ex_node};
+            if (from == 0)  // two blocks of 64 KB LDS per CU
+                hipLaunchKernelGGL(auction ? k_bvh8_expand<NXB_SLOT_AUCTION> : k_bvh8_expand<NXB_SLOT_GREEDY>,
+                                   dim3(min((n - 2) / kBvh8Threads + 1, device_cu_count() * 2u)), dim3(kBvh8Threads),
+                                   0, s, sc.rec8, n, 2 * n - 1, ex, sc.flags);
+            const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 4u);
+            for (uint32_t l = from; l < end; ++l)
+                hipLaunchKernelGGL(k_bvh8_place, dim3(l == 0 ? 1u : grid), dim3(kBvh8Threads), 0, s, ex, n, 2 * n - 1,
+                                   out, prim_idx, capacity, sc.work, sc.work2, cnt, l, alloc, sc.flags);
+            return hipGetLastError();
+        }
+        auto kernel = auction ? k_bvh8_collapse<NXB_SLOT_AUCTION> : k_bvh8_collapse<NXB_SLOT_GREEDY>;
+        // two blocks of 67 KB LDS per CU
+        const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 2u);
         for (uint32_t l = from; l < end; ++l)
             hipLaunchKernelGGL(kernel, dim3(l == 0 ? 1u : grid), dim3(kBvh8Threads), 0, s, sc.rec8, n, 2 * n - 1, out,
                                prim_idx, capacity, sc.work, sc.work2, cnt, l, alloc, sc.flags);
