@@ -136,7 +136,7 @@ Layout make_layout(uint32_t n, uint32_t key_bytes, bool full, bool bvh8 = true, 
     L.feat = take(segs * NXB_MLP_FEATURES * sizeof(float));
     L.rtable = take(segs);
     L.rec8 = rec8 && n > 1 ? take((size_t)(n - 1) * 64) : 0;
-    L.ex_node = L.rec8 && bvh8_expands(n) ? take((size_t)(n - 1) * 80) : 0;
+    L.ex_node = L.rec8 && bvh8_small(n) ? take((size_t)(n - 1) * 80) : 0;
     L.total = off;
     return L;
 }

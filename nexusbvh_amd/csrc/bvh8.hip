@@ -304,13 +304,8 @@ __device__ __forceinline__ bool collapse_node(const nxb_bvh2_node* b2, uint32_t 
     return true;
 }
 
-// Collapse of internal node x from the wide records of a BVH8 build (record
-// x - n: both children's boxes, ids and primitive counts). Same push/pop
-// order as collapse_node; each expansion is one 64-byte load, the node's box
-// is the union of its children's (as H-PLOC formed it, bit for bit), and the
-// children's primitive counts come with them: cleft[t] holds child t's count
-// if it is internal (id >= n), kInvalid for a leaf; cright[t] its id (the
-// primitive index of a leaf).
+// The wide record of a BVH8 build's internal node: both children's boxes, ids
+// (a leaf's is its primitive index, below n) and primitive counts.
 __device__ __forceinline__ void load_rec8(const uint4* rec, uint32_t i, Box& l, Box& r, uint32_t& li, uint32_t& ri,
                                           uint32_t& ls, uint32_t& rs) {
     const uint4* p = rec + 4ull * i;
@@ -320,62 +315,6 @@ __device__ __forceinline__ void load_rec8(const uint4* rec, uint32_t i, Box& l, 
     r.lx = __uint_as_float(q1.z); r.ly = __uint_as_float(q1.w); r.lz = __uint_as_float(q2.x);
     r.hx = __uint_as_float(q2.y); r.hy = __uint_as_float(q2.z); r.hz = __uint_as_float(q2.w);
     li = q3.x; ri = q3.y; ls = q3.z; rs = q3.w;
-}
-
-__device__ __forceinline__ bool collapse_rec(const uint4* rec, uint32_t n, uint32_t node_count, uint32_t x,
-                                             Collapsed& c, ChildBoxes& cbx, uint32_t tid, uint32_t slot_mode) {
-    if (x < n || x >= node_count) return false;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) { c.child[t] = 0; c.cright[t] = 0; c.cleft[t] = 0; }
-    uint32_t inner = 0, count = 0;
-    int msb = 0;
-    uint32_t cur = x;
-    for (;;) {
-        Box b0, b1;
-        uint32_t i0, i1, s0, s1;
-        load_rec8(rec, cur - n, b0, b1, i0, i1, s0, s1);
-        if (cur == x) c.pb = box_union(b0, b1);
-        if (i0 >= node_count || i1 >= node_count) return false;
-        bool first_is_1 = !(box_area(b0) < box_area(b1));
-        uint32_t ia = (uint32_t)msb, ib = count + 1;
-        uint32_t na = first_is_1 ? i1 : i0, nb = first_is_1 ? i0 : i1;
-        uint32_t sa = first_is_1 ? s1 : s0, sb = first_is_1 ? s0 : s1;
-        put_child_box(cbx, ia, tid, first_is_1 ? b1 : b0);
-        put_child_box(cbx, ib, tid, first_is_1 ? b0 : b1);
-        const bool ia_inner = na >= n, ib_inner = nb >= n;
-#pragma unroll
-        for (uint32_t t = 0; t < 8; ++t) {
-            if (t == ia) { c.child[t] = na; c.cleft[t] = ia_inner ? sa : kInvalid; c.cright[t] = na; }
-            if (t == ib) { c.child[t] = nb; c.cleft[t] = ib_inner ? sb : kInvalid; c.cright[t] = nb; }
-        }
-        if (ia_inner) inner |= 1u << ia;
-        if (ib_inner) inner |= 1u << ib;
-        count += 2;
-        msb = inner ? 31 - __clz(inner) : -1;
-        if (msb < 0 || count == 8) break;
-        inner &= ~(1u << msb);
-        --count;
-#pragma unroll
-        for (uint32_t t = 0; t < 8; ++t)
-            if (t == (uint32_t)msb) cur = c.child[t];
-    }
-    c.count = count;
-    assign_slots(c, cbx, tid, slot_mode, inner);
-    return true;
-}
-
-// Primitive counts of a node's inner children per output slot, from the
-// record collapse (0 for leaf and free slots).
-__device__ __forceinline__ void rec_child_sizes(const Collapsed& c, uint32_t sz[8]) {
-#pragma unroll
-    for (uint32_t s = 0; s < 8; ++s) {
-        sz[s] = 0;
-        const uint32_t a = nib(c.assign, s);
-        if (a == 0xFu || !(c.im & (1u << s))) continue;
-#pragma unroll
-        for (uint32_t t = 0; t < 8; ++t)
-            if (t == a) sz[s] = c.cleft[t];
-    }
 }
 
 // Publishes the inner children of BVH8 node k (the first one is kept by this
@@ -401,7 +340,6 @@ __device__ __forceinline__ void load_child_sizes(const Collapsed& c, const uint3
     }
 }
 
-template <bool KEEP = true>
 __device__ __forceinline__ void emit_node(const ChildBoxes& cbx, uint32_t tid, const Collapsed& c, uint32_t k,
                                           uint32_t child_base, uint32_t prim_base, uint32_t leaf_count,
                                           const uint32_t sz[8], nxb_bvh8_node* out, uint32_t* prim_idx,
@@ -424,9 +362,6 @@ __device__ __forceinline__ void emit_node(const ChildBoxes& cbx, uint32_t tid, c
             const uint32_t size = sz[s];
             if (slot >= capacity || size < 2 || next_base + size > n) {
                 atomic_or_agent(flags, kFlagBadIndex);
-            } else if (!KEEP) {
-                // read by the next level's kernel
-                work[slot] = ((uint64_t)next_base << 32) | ch;
             } else if (keep_slot == kNoSlot) {
                 keep_slot = slot;
                 keep_x = ch;
@@ -602,6 +537,16 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8(const nxb_bvh2_node* __re
 // loads (leaves in input order, a line each) and the size lookups. At 28.1M
 // triangles this took the collapse from 1.94 to 1.31 ms. The stage entry
 // point and batched forests collapse BVH2 nodes.
+//
+// What bounds it: every record is read once and every node written once (2.2 GB
+// at 28.1M triangles), 64 bytes at a time all over memory, by lanes that wait
+// for one record before they ask for the next. The children are kept in
+// registers and a node is put together in LDS (36 KB a block, four blocks per
+// CU; the children's boxes in LDS took 48 KB, three blocks, and 2,970 vector
+// instructions per wave, now 2,400), and four lanes fetch a record in one
+// request. Collapse of 28.1M triangles 1323 -> 1278 -> 1165 us, 12.7M 828 -> 770
+// -> 722, 2.9M 338 -> 308 -> 293; queued children put in order before their
+// store, 1% less, was not worth its lines.
 constexpr uint32_t kMaxLevels = kBvh8LevelWords - 1;  // BVH8 levels; each consumes at least one BVH2 level
 
 // Exclusive scan over a 256-thread block; *total gets the block sum.
@@ -625,17 +570,309 @@ __device__ __forceinline__ uint32_t block_scan_256(uint32_t v, uint32_t* tmp, ui
     return before + incl - v;
 }
 
+// The children of the node a lane collapses, in registers: box, id and primitive
+// count (0: a leaf). Only ever indexed by constants.
+struct Kids {
+    Box box[8];
+    uint32_t id[8], prims[8];
+};
+
+// Records idx of the wave's lanes (kInvalid: none), four lanes fetching each:
+// straight to LDS, 16 bytes a lane, so that a record is one 64-byte request. Its
+// own lane fetching it made four of as many lines as lanes. buf: 260 words of
+// the wave's own; record of lane 4i + j at 65 j + 4 i (conflict-free). All lanes
+// of the wave take part.
+template <uint32_t J>
+__device__ __forceinline__ void fetch_quad(const uint4* rec, uint32_t idx, uint4* buf) {
+    const uint32_t of = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)idx, J * 0x55, 0xF, 0xF, true);  // quad's lane J
+    if (of != kInvalid)
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)(rec + 4ull * of + (__lane_id() & 3u)),
+            (__attribute__((address_space(3))) void*)(buf + 65 * J), 16, 0, 0);
+}
+__device__ __forceinline__ void load_rec8_quads(const uint4* rec, uint32_t idx, uint4* buf, Box& l, Box& r,
+                                                uint32_t& li, uint32_t& ri, uint32_t& ls, uint32_t& rs) {
+    fetch_quad<0>(rec, idx, buf);
+    fetch_quad<1>(rec, idx, buf);
+    fetch_quad<2>(rec, idx, buf);
+    fetch_quad<3>(rec, idx, buf);
+    wait_memory_ops();
+    wave_lds_sync();
+    const uint32_t lane = __lane_id();
+    const uint4* p = buf + 65 * (lane & 3u) + 4 * (lane >> 2);
+    const uint4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3];
+    wave_lds_sync();
+    l.lx = __uint_as_float(q0.x); l.ly = __uint_as_float(q0.y); l.lz = __uint_as_float(q0.z);
+    l.hx = __uint_as_float(q0.w); l.hy = __uint_as_float(q1.x); l.hz = __uint_as_float(q1.y);
+    r.lx = __uint_as_float(q1.z); r.ly = __uint_as_float(q1.w); r.lz = __uint_as_float(q2.x);
+    r.hx = __uint_as_float(q2.y); r.hy = __uint_as_float(q2.z); r.hz = __uint_as_float(q2.w);
+    li = q3.x; ri = q3.y; ls = q3.z; rs = q3.w;
+}
+
+// Collapse of internal node x (record x - n), in the push/pop order of
+// collapse_node: the pair's larger child goes on top (slot t + 1 in step t), the
+// smaller into the popped slot, which selects find. The node's box is the union
+// of its children's (as H-PLOC formed it, bit for bit). False for an id out of
+// range.
+__device__ __forceinline__ bool collapse_kids(const uint4* rec, uint32_t n, uint32_t node_count, uint32_t x, Kids& K,
+                                              Box& pb, uint32_t& count, uint32_t& inner, uint4* buf) {
+    count = 0;
+    inner = 0;
+    bool ok = x >= n && x < node_count, live = ok;
+    uint32_t msb = 0, cur = x;
+#pragma unroll
+    for (uint32_t t = 0; t < 7; ++t) {
+        if (!ballot(live)) break;
+        Box b0, b1;
+        uint32_t i0, i1, s0, s1;
+        load_rec8_quads(rec, live ? cur - n : kInvalid, buf, b0, b1, i0, i1, s0, s1);
+        if (live && max(i0, i1) >= node_count) {
+            ok = false;
+            live = false;
+        }
+        if (!live) continue;
+        if (t == 0) pb = box_union(b0, b1);
+        const bool first_is_1 = !(box_area(b0) < box_area(b1));
+        const uint32_t small = first_is_1 ? i1 : i0, large = first_is_1 ? i0 : i1;
+        const uint32_t psmall = small >= n ? (first_is_1 ? s1 : s0) : 0u;
+        const Box bs = first_is_1 ? b1 : b0;
+        K.box[t + 1] = first_is_1 ? b0 : b1;
+        K.id[t + 1] = large;
+        K.prims[t + 1] = large >= n ? (first_is_1 ? s0 : s1) : 0u;
+        uint32_t older = 0;  // the highest inner child below the popped slot
+        inner |= (small >= n ? 1u << msb : 0u) | (large >= n ? 2u << t : 0u);
+        const uint32_t top = 31u - (uint32_t)__clz(inner | 1u);
+#pragma unroll
+        for (uint32_t j = 0; j <= t; ++j) {
+            const bool here = msb == j;
+            K.box[j].lx = here ? bs.lx : K.box[j].lx;
+            K.box[j].ly = here ? bs.ly : K.box[j].ly;
+            K.box[j].lz = here ? bs.lz : K.box[j].lz;
+            K.box[j].hx = here ? bs.hx : K.box[j].hx;
+            K.box[j].hy = here ? bs.hy : K.box[j].hy;
+            K.box[j].hz = here ? bs.hz : K.box[j].hz;
+            K.id[j] = here ? small : K.id[j];
+            K.prims[j] = here ? psmall : K.prims[j];
+            older = top == j ? K.id[j] : older;
+        }
+        count = t + 2;
+        live = inner != 0;
+        if (t < 6 && live) {
+            cur = large >= n ? large : older;
+            msb = top;
+            inner &= ~(1u << top);
+        }
+    }
+    return ok;
+}
+
+// GreedyAssignment (WideConverter.cu:106-153): each child in push order takes
+// the free slot of the largest cost (GetCost 25-30), the lowest on a tie; with
+// no comparable cost the first free slot. Slots s and 7 - s have opposite
+// costs, bit for bit, so four sums give all eight. box(k): child k's box (any
+// from count on). Nibble k of the result is child k's slot; used: the slots.
+template <typename BoxOf>
+__device__ __forceinline__ uint32_t greedy_slots(const Box& pb, uint32_t count, uint32_t& used, const BoxOf& box) {
+    const float lowest = -3.402823466e+38f;
+    const float pcx = pb.lx + pb.hx, pcy = pb.ly + pb.hy, pcz = pb.lz + pb.hz;
+    uint32_t slots = 0, taken = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+        const Box cb = box(k);
+        const float ox = pcx - (cb.hx + cb.lx), oy = pcy - (cb.hy + cb.ly), oz = pcz - (cb.hz + cb.lz);
+        const float p = ox + oy, m = ox - oy;
+        const float c[4] = {p + oz, p - oz, m + oz, m - oz};
+        // the largest cost of the free slots (a NaN is dropped), then the
+        // lowest slot that has it
+        float cost[8], most = lowest;
+#pragma unroll
+        for (uint32_t s = 0; s < 8; ++s) {
+            cost[s] = (taken & (1u << s)) ? lowest : (s < 4 ? c[s & 3] : -c[(7 - s) & 3]);
+            most = fmaxf(most, cost[s]);
+        }
+        uint32_t best = 8u;
+#pragma unroll
+        for (int s = 7; s >= 0; --s) best = cost[s] == most ? (uint32_t)s : best;
+        if (!(most > lowest)) best = (uint32_t)__builtin_ctz(~taken | 0x100u);
+        if (k < count) {
+            taken |= 1u << best;
+            slots |= best << (4 * k);
+        }
+    }
+    used = taken;
+    return slots;
+}
+
+// Auction slots (auction_assign) of the same.
+template <typename BoxOf>
+__device__ __forceinline__ uint32_t auction_slots(const Box& pb, uint32_t count, uint32_t& used, const BoxOf& box) {
+    const float pcx = pb.lx + pb.hx, pcy = pb.ly + pb.hy, pcz = pb.lz + pb.hz;
+    float ox[8], oy[8], oz[8];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+        const Box cb = box(k);
+        ox[k] = k < count ? pcx - (cb.lx + cb.hx) : 0.0f;
+        oy[k] = k < count ? pcy - (cb.ly + cb.hy) : 0.0f;
+        oz[k] = k < count ? pcz - (cb.lz + cb.hz) : 0.0f;
+    }
+    const uint32_t assign = auction_assign(pb, ox, oy, oz, count);
+    uint32_t slots = 0, taken = 0;
+#pragma unroll
+    for (uint32_t s = 0; s < 8; ++s) {
+        const uint32_t a = nib(assign, s);
+        if (a == 0xFu) continue;
+        taken |= 1u << s;
+        slots |= s << (4 * a);
+    }
+    used = taken;
+    return slots;
+}
+template <uint32_t SLOT, typename BoxOf>
+__device__ __forceinline__ uint32_t choose_slots(const Box& pb, uint32_t count, uint32_t& used, const BoxOf& box) {
+    if constexpr (SLOT == NXB_SLOT_AUCTION) return auction_slots(pb, count, used, box);
+    else return greedy_slots(pb, count, used, box);
+}
+
+// A wave's nodes on their way to memory, and their children by slot.
+struct NodeStage {
+    uint4 w[5 * kBvh8Threads];  // lane's node: five words from 5 * lane
+    uint2 kid[8][kBvh8Threads];  // id, primitive count (0: a leaf)
+};
+
+// Exponents of a node's quantization grid (CreateBVH8Node, WideConverter.cu:156-206).
+__device__ __forceinline__ uint32_t grid_exponents(const Box& pb, float& ix, float& iy, float& iz) {
+    const float qstep = 1.0f / 255.0f;
+    const uint32_t e0 = ceil_log2((pb.hx - pb.lx) * qstep) & 0xFFu;
+    const uint32_t e1 = ceil_log2((pb.hy - pb.ly) * qstep) & 0xFFu;
+    const uint32_t e2 = ceil_log2((pb.hz - pb.lz) * qstep) & 0xFFu;
+    ix = inv_pow2(e0);
+    iy = inv_pow2(e1);
+    iz = inv_pow2(e2);
+    return e0 | (e1 << 8) | (e2 << 16);
+}
+
+// Puts the lane's node into the stage, byte by byte at its slots, without the
+// child and primitive bases, and its children.
+__device__ __forceinline__ void stage_node(NodeStage& st, uint32_t tid, const Box& pb, const Kids& K, uint32_t count,
+                                           uint32_t slots, uint32_t im, uint32_t lm) {
+    float ix, iy, iz;
+    const uint32_t e = grid_exponents(pb, ix, iy, iz);
+    uint4* w = st.w + 5 * tid;
+    w[0] = make_uint4(__float_as_uint(pb.lx), __float_as_uint(pb.ly), __float_as_uint(pb.lz), e | (im << 24));
+#pragma unroll
+    for (uint32_t i = 1; i < 5; ++i) w[i] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+        if (k >= count) break;
+        const uint32_t s = nib(slots, k);
+        const Box& b = K.box[k];
+        uint8_t* q = reinterpret_cast<uint8_t*>(w) + 24 + s;
+        q[0] = (uint8_t)((1u << 5) | ((im >> s) & 1u ? 24u + s : bits_below(lm, s)));
+        q[8] = (uint8_t)q_floor((b.lx - pb.lx) * ix);
+        q[16] = (uint8_t)q_floor((b.ly - pb.ly) * iy);
+        q[24] = (uint8_t)q_floor((b.lz - pb.lz) * iz);
+        q[32] = (uint8_t)q_ceil((b.hx - pb.lx) * ix);
+        q[40] = (uint8_t)q_ceil((b.hy - pb.ly) * iy);
+        q[48] = (uint8_t)q_ceil((b.hz - pb.lz) * iz);
+        st.kid[s][tid] = make_uint2(K.id[k], K.prims[k]);
+    }
+}
+
+// What collapse_nodes works on: a level's nodes and where they go.
+struct LevelIo {
+    const uint4* rec;
+    uint32_t n, node_count;
+    nxb_bvh8_node* out;
+    uint32_t* prim_idx;
+    uint32_t capacity;
+    uint64_t* work;
+    uint32_t* flags;
+};
+
+// Makes the BVH8 nodes k0 + lane < hi of the block (a whole block, one node a
+// lane): x and pbase of each lane's node, ids(total) the first id of the block's
+// inner children, in LDS or known to all lanes after its barrier.
+template <uint32_t SLOT, typename Ids>
+__device__ __forceinline__ uint32_t collapse_nodes(NodeStage& st, uint32_t* scan_tmp, const LevelIo& io, uint32_t k0,
+                                                   bool has, uint32_t x, uint32_t pbase, const Ids& ids) {
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w0 = tid & ~63u;
+    Kids K = {};
+    Box pb = {0, 0, 0, 0, 0, 0};
+    uint32_t count = 0, inner = 0;
+    const bool ok =
+        collapse_kids(io.rec, io.n, io.node_count, has ? x : 0u, K, pb, count, inner, st.w + 5 * w0);
+    if (has && !ok) atomic_or_agent(io.flags, kFlagBadIndex);
+    const uint32_t ic = ok ? (uint32_t)__popc(inner) : 0u;
+    uint32_t total = 0;
+    const uint32_t excl = block_scan_256<true>(ic, scan_tmp, &total);
+    ids.take(total);
+    uint32_t im = 0, used = 0;
+    if (ok) {
+        const uint32_t slots = choose_slots<SLOT>(pb, count, used, [&](uint32_t i) { return K.box[i]; });
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) im |= ((inner >> i) & 1u) << nib(slots, i);
+        stage_node(st, tid, pb, K, count, slots, im, used & ~im);
+    }
+    lds_barrier();
+    const uint32_t base = ids.first() + excl;
+    if (ok) {
+        const uint32_t leaves = count - ic;
+        uint32_t next_base = pbase + leaves, leaf = pbase, child = base;
+        bool good = true;
+#pragma unroll
+        for (uint32_t s = 0; s < 8; ++s) {
+            const uint2 kid = st.kid[s][tid];
+            if ((im >> s) & 1u) {
+                if (child < io.capacity && kid.y >= 2 && next_base + kid.y <= io.n)
+                    io.work[child] = ((uint64_t)next_base << 32) | kid.x;  // read by the next level
+                else good = false;
+                next_base += kid.y;
+                ++child;
+            } else if ((used >> s) & 1u) {
+                if (leaf < io.n) io.prim_idx[leaf] = kid.x;
+                else good = false;
+                ++leaf;
+            }
+        }
+        if (!good) atomic_or_agent(io.flags, kFlagBadIndex);
+        *reinterpret_cast<uint2*>(&st.w[5 * tid + 1]) = make_uint2(ic ? base : 0u, leaves ? pbase : 0u);
+    }
+    const uint64_t oks = ballot(ok);
+    wave_lds_sync();
+    // the wave's nodes are consecutive: 16 bytes a lane, five times
+    uint4* o = reinterpret_cast<uint4*>(io.out + k0 + w0);
+#pragma unroll
+    for (uint32_t i = 0; i < 5; ++i) {
+        const uint32_t c = lane + 64 * i;
+        if ((oks >> (c / 5u)) & 1ull) o[c] = st.w[5 * w0 + c];
+    }
+    return total;
+}
+
+// Ids of a block's inner children from the next level's counter.
+struct IdsFromCounter {
+    uint32_t* slot;     // one word of LDS
+    uint32_t* counter;
+    uint32_t from;      // the next level's first id
+    __device__ __forceinline__ void take(uint32_t total) const {
+        if (threadIdx.x == 0) *slot = total ? from + atomic_add_agent(counter, total) : 0u;
+    }
+    __device__ __forceinline__ uint32_t first() const { return *slot; }
+};
+struct IdsInOrder {
+    uint32_t from;
+    __device__ __forceinline__ void take(uint32_t) const {}
+    __device__ __forceinline__ uint32_t first() const { return from; }
+};
+
 // The top levels of one tree in one block: the level counters initialized
-// (cnt[0] = 1, the root; the rest 0), then levels 0..kBvh8TopLevels-1 (at most 1, 8 and 64
-// nodes) one after another, the children's ids taken from a running count
-// instead of a global atomic. Saves the launches and counter round trips of
-// the levels whose time is all latency.
+// (cnt[0] = 1, the root; the rest 0), then levels 0..kBvh8TopLevels-1 (at most 1,
+// 8 and 64 nodes) one after another, the children's ids taken from a running
+// count instead of a global atomic. Saves the launches and counter round trips
+// of the levels whose time is all latency.
 template <uint32_t SLOT>
-__global__ __launch_bounds__(kBvh8Threads) void k_bvh8_top(const uint4* __restrict__ rec, uint32_t n,
-                                                           uint32_t node_count, nxb_bvh8_node* __restrict__ out,
-                                                           uint32_t* prim_idx, uint32_t capacity, uint64_t* work,
-                                                           uint32_t* cnt, uint32_t* flags) {
-    __shared__ ChildBoxes cbx;
+__global__ __launch_bounds__(kBvh8Threads) void k_bvh8_top(LevelIo io, uint32_t* cnt) {
+    __shared__ NodeStage st;
     __shared__ uint32_t scan_tmp[kBvh8Threads / 64];
     const uint32_t tid = threadIdx.x;
     for (uint32_t i = tid; i <= kMaxLevels; i += kBvh8Threads) cnt[i] = i == 0 ? 1u : 0u;
@@ -644,47 +881,26 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_top(const uint4* __restri
         const uint32_t hi = lo + m;
         uint32_t next = 0;
         for (uint32_t k0 = lo; k0 < hi; k0 += kBvh8Threads) {
-            const uint32_t k = k0 + tid;
-            Collapsed c;
-            bool ok = false;
-            uint32_t pbase = 0;
-            if (k < hi) {
-                uint32_t x = node_count - 1;  // the root, primitive base 0
-                if (level > 0) {
-                    // written by this block's previous level (agent-scope
-                    // loads: not through the CU's L1)
-                    const uint64_t v = load_agent64(&work[k]);
-                    x = (uint32_t)v;
-                    pbase = (uint32_t)(v >> 32);
-                }
-                ok = collapse_rec(rec, n, node_count, x, c, cbx, tid, SLOT);
-                if (!ok) atomic_or_agent(flags, kFlagBadIndex);
-            }
-            const uint32_t ic = ok ? (uint32_t)__popc(c.im) : 0u;
-            uint32_t sz[8];
-            if (ok) rec_child_sizes(c, sz);
-            uint32_t total = 0;
-            const uint32_t excl = block_scan_256(ic, scan_tmp, &total);
-            if (ok) {
-                uint32_t ks, kx, kb;
-                emit_node<false>(cbx, tid, c, k, ic ? hi + next + excl : 0u, pbase, c.count - ic, sz, out, prim_idx,
-                                 n, capacity, work, flags, ks, kx, kb);
-            }
-            next += total;
+            const bool has = k0 + tid < hi && k0 + tid < io.capacity;
+            // the root, primitive base 0; below, written by this block's previous
+            // level (agent-scope loads: not through the CU's L1)
+            uint64_t v = io.node_count - 1;
+            if (level > 0 && has) v = load_agent64(&io.work[k0 + tid]);
+            next += collapse_nodes<SLOT>(st, scan_tmp, io, k0, has, (uint32_t)v, (uint32_t)(v >> 32),
+                                         IdsInOrder{hi + next});
+            __syncthreads();  // the work items are written before the next level reads them
         }
         if (tid == 0) cnt[level + 1] = next;
-        __syncthreads();  // the level's work items are written before the next level reads them
         lo = hi;
         m = next;
     }
 }
 
+// (second bound: waves per SIMD, four as the LDS allows; the auction needs the
+// registers of three)
 template <uint32_t SLOT>
-__global__ __launch_bounds__(kBvh8Threads) void k_bvh8_level(const uint4* __restrict__ rec, uint32_t n,
-                                                             uint32_t node_count, nxb_bvh8_node* __restrict__ out,
-                                                             uint32_t* prim_idx, uint32_t capacity, uint64_t* work,
-                                                             uint32_t* cnt, uint32_t level, uint32_t* flags) {
-    __shared__ ChildBoxes cbx;
+__global__ __launch_bounds__(kBvh8Threads, SLOT == NXB_SLOT_AUCTION ? 3 : 4) void k_bvh8_level(LevelIo io, uint32_t* cnt, uint32_t level) {
+    __shared__ NodeStage st;
     __shared__ uint32_t scan_tmp[kBvh8Threads / 64];
     __shared__ uint32_t sbase;
     const uint32_t tid = threadIdx.x;
@@ -694,53 +910,38 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_level(const uint4* __rest
     for (uint32_t j = 0; j < level; ++j) lo += cnt[j];
     const uint32_t hi = lo + m;
     if (level + 1 > kMaxLevels) {
-        if (blockIdx.x == 0 && tid == 0) atomic_or_agent(flags, kFlagBadIndex);
+        if (blockIdx.x == 0 && tid == 0) atomic_or_agent(io.flags, kFlagBadIndex);
         return;
     }
     for (uint32_t k0 = lo + blockIdx.x * kBvh8Threads; k0 < hi; k0 += gridDim.x * kBvh8Threads) {
-        const uint32_t k = k0 + tid;
-        Collapsed c;
-        bool ok = false;
-        uint32_t pbase = 0;
-        if (k < hi) {
-            const uint64_t v = work[k];
-            const uint32_t x = (uint32_t)v;
-            pbase = (uint32_t)(v >> 32);
-            ok = collapse_rec(rec, n, node_count, x, c, cbx, tid, SLOT);
-            if (!ok) atomic_or_agent(flags, kFlagBadIndex);
-        }
-        const uint32_t ic = ok ? (uint32_t)__popc(c.im) : 0u;
-        uint32_t sz[8];
-        if (ok) rec_child_sizes(c, sz);
-        uint32_t total = 0;
-        const uint32_t excl = block_scan_256(ic, scan_tmp, &total);
-        if (tid == 0) sbase = total ? hi + atomic_add_agent(&cnt[level + 1], total) : 0u;
-        __syncthreads();
-        const uint32_t base = sbase;
-        if (ok) {
-            uint32_t ks, kx, kb;
-            emit_node<false>(cbx, tid, c, k, ic ? base + excl : 0u, pbase, c.count - ic, sz, out, prim_idx, n,
-                             capacity, work, flags, ks, kx, kb);
-        }
+        const bool has = k0 + tid < hi && k0 + tid < io.capacity;
+        const uint64_t v = has ? io.work[k0 + tid] : 0ull;
+        collapse_nodes<SLOT>(st, scan_tmp, io, k0, has, (uint32_t)v, (uint32_t)(v >> 32),
+                             IdsFromCounter{&sbase, &cnt[level + 1], hi});
+        lds_barrier();  // sbase and the stage are read before the next nodes
     }
 }
 
-// ---- few launches (single builds up to 2^21 primitives) ----------------------
+// ---- every node expanded first (single builds of small meshes) --------------
 //
-// One lane collapses one node; a block reserves the ids of its nodes' inner
-// children with one atomic add on the node counter and passes the children on
-// to itself, through LDS, while they fit its lanes, else to the next launch
-// through a queue in global memory. Launch l takes the queue positions
-// [cnt[1] + ... + cnt[l-1], +cnt[l]), counts that earlier launches completed,
-// so no lane ever waits on another (no polling, no spin limit); launch 0 is
-// the root.
-//
-// What bounds it is latency: a node costs its lane up to seven dependent record
-// loads (~1,300 cycles each with the choice of the next), then the slots and
-// the quantization, and a mesh has log2(n) levels, since a node's largest child
-// keeps half of its primitives. A level took 15 to 17 us as a launch of its own
-// (counters, queue and a cold L2 first), ~7 us inside a block. Up to
-// kExpandPrims that work is taken out of the levels (k_bvh8_expand).
+// What a BVH8 node looks like depends on its BVH2 node alone, except for the
+// numbers of its children and primitives. So one launch makes the BVH8 node of
+// every internal BVH2 node, side by side: the chain of seven record loads, the
+// slots and the quantization are waited for once instead of once per level. The
+// levels that follow only hand out numbers: a level inside a block is two loads,
+// a count and the writes (~2,500 cycles, 1,300 to 2,700 of them the loads'),
+// where collapsing the nodes took ~17,000. 2,003 primitives: 10 us and 18 us;
+// 300K: 34 us and four launches of 6 to 20 us.
+
+// Primitives up to which a build takes this path, above a launch per level: all
+// internal BVH2 nodes are about five times those that the BVH8 needs, but at
+// once. Collapse stage in us, on a surface, blobs and slivers, this / levels:
+// 32/125, 28/97, 28/97 at 2,003; 53/169, 51/163, 47/144 at 48K; 96/177, 109/205,
+// 102/175 at 300K; 186/210, 211/236, 185/203 at 900K; 213/216, 245/253, 215/224
+// at 1.1M; 347/259, 389/297, 353/267 at 2M.
+constexpr uint32_t kSmallPrims = 1u << 20;
+bool bvh8_small(uint32_t n) { return n <= kSmallPrims; }
+
 // The children of the node each lane collapses, in LDS (child t of lane i at
 // [t][i]): box, id (a leaf is an id below n, its primitive index) and
 // primitive count. Indexed by slot when they are read back, which in
@@ -796,58 +997,6 @@ __device__ __forceinline__ bool collapse_children(const uint4* rec, uint32_t n, 
     return true;
 }
 
-// GreedyAssignment (WideConverter.cu:106-153): each child in push order takes
-// the free slot of the largest cost (GetCost 25-30), the lowest on a tie; with
-// no comparable cost the first free slot. Slots s and 7 - s have opposite
-// costs, bit for bit, so four sums give all eight. Nibble s of the result is
-// the child in slot s, 0xF none.
-__device__ __forceinline__ uint32_t greedy_assign(const Box& pb, const RecChildren& ch, uint32_t tid, uint32_t count) {
-    const float lowest = -3.402823466e+38f;
-    const float pcx = pb.lx + pb.hx, pcy = pb.ly + pb.hy, pcz = pb.lz + pb.hz;
-    uint32_t assign = 0xFFFFFFFFu, free_slots = 0xFFu;
-#pragma unroll
-    for (uint32_t k = 0; k < 8; ++k) {
-        const Box cb = get_child_box(ch, k, tid);
-        const float ox = pcx - (cb.hx + cb.lx), oy = pcy - (cb.hy + cb.ly), oz = pcz - (cb.hz + cb.lz);
-        const float p = ox + oy, m = ox - oy;
-        const float c[4] = {p + oz, p - oz, m + oz, m - oz};
-        // the largest cost of the free slots (a NaN is dropped), then the
-        // lowest slot that has it
-        float cost[8], most = lowest;
-#pragma unroll
-        for (uint32_t s = 0; s < 8; ++s) {
-            cost[s] = (free_slots & (1u << s)) ? (s < 4 ? c[s & 3] : -c[(7 - s) & 3]) : lowest;
-            most = fmaxf(most, cost[s]);
-        }
-        uint32_t best = 8u;
-#pragma unroll
-        for (int s = 7; s >= 0; --s) best = cost[s] == most ? (uint32_t)s : best;
-        if (!(most > lowest)) best = (uint32_t)__builtin_ctz(free_slots | 0x100u);
-        if (k < count) {
-            free_slots &= ~(1u << best);
-            assign = with_nib(assign, best, k);
-        }
-    }
-    return assign;
-}
-
-// Auction slots (auction_assign) of the same children.
-__device__ __forceinline__ uint32_t auction_slots(const Box& pb, const RecChildren& ch, uint32_t tid, uint32_t count) {
-    const float pcx = pb.lx + pb.hx, pcy = pb.ly + pb.hy, pcz = pb.lz + pb.hz;
-    float ox[8], oy[8], oz[8];
-#pragma unroll
-    for (uint32_t k = 0; k < 8; ++k) {
-        ox[k] = oy[k] = oz[k] = 0.0f;
-        if (k < count) {
-            const Box cb = get_child_box(ch, k, tid);
-            ox[k] = pcx - (cb.lx + cb.hx);
-            oy[k] = pcy - (cb.ly + cb.hy);
-            oz[k] = pcz - (cb.lz + cb.hz);
-        }
-    }
-    return auction_assign(pb, ox, oy, oz, count);
-}
-
 // Work items passed on inside a block.
 struct BlockQueue {
     uint32_t x[kBvh8Threads], base[kBvh8Threads], id[kBvh8Threads];
@@ -879,18 +1028,6 @@ struct ChildSink {
         return good;
     }
 };
-
-// Exponents of a node's quantization grid (CreateBVH8Node, WideConverter.cu:156-206).
-__device__ __forceinline__ uint32_t grid_exponents(const Box& pb, float& ix, float& iy, float& iz) {
-    const float qstep = 1.0f / 255.0f;
-    const uint32_t e0 = ceil_log2((pb.hx - pb.lx) * qstep) & 0xFFu;
-    const uint32_t e1 = ceil_log2((pb.hy - pb.ly) * qstep) & 0xFFu;
-    const uint32_t e2 = ceil_log2((pb.hz - pb.lz) * qstep) & 0xFFu;
-    ix = inv_pow2(e0);
-    iy = inv_pow2(e1);
-    iz = inv_pow2(e2);
-    return e0 | (e1 << 8) | (e2 << 16);
-}
 
 // A node's 80 bytes without the child and primitive bases, and its children by
 // slot: id (kInvalid: free) and primitive count (0: a leaf or free).
@@ -935,153 +1072,6 @@ __device__ __forceinline__ PackedNode pack_node(const RecChildren& ch, uint32_t 
     return r;
 }
 
-// Emits the node of one lane: primIdx entries of its leaves, work items of its
-// inner children, the 80 bytes. Primitive ranges are fixed top-down: a node's
-// leaves take the front of its range, then each inner child, in slot order, a
-// range of its primitive count.
-__device__ __forceinline__ bool emit_lane(const RecChildren& ch, uint32_t tid, const Box& pb, uint32_t count,
-                                          uint32_t inner, uint32_t assign, uint32_t base, uint32_t id, uint32_t excl,
-                                          const ChildSink& sink, nxb_bvh8_node* out, uint32_t* prim_idx) {
-    const uint32_t ic = (uint32_t)__popc(inner), leaf_count = count - ic;
-    PackedNode r = pack_node(ch, tid, pb, inner, assign);
-    uint32_t next_base = base + leaf_count, leaves = 0, nth = 0;
-    bool good = true;
-#pragma unroll
-    for (uint32_t s = 0; s < 8; ++s) {
-        if (r.prims[s]) {
-            good &= sink.put(excl + nth, r.kid[s], next_base, r.prims[s]);
-            next_base += r.prims[s];
-            ++nth;
-        } else if (r.kid[s] != kInvalid) {
-            if (base + leaves < sink.n) prim_idx[base + leaves] = r.kid[s];
-            else good = false;
-            ++leaves;
-        }
-    }
-    r.w[1].x = ic ? sink.ids + excl : 0u;
-    r.w[1].y = leaf_count ? base : 0u;
-    uint4* o = reinterpret_cast<uint4*>(out + id);
-#pragma unroll
-    for (uint32_t i = 0; i < 5; ++i) o[i] = r.w[i];
-    return good;
-}
-
-// Primitives up to which a build takes launches that follow subtrees; above, one
-// launch per level (three blocks of 48 KB LDS per CU where k_bvh8_collapse has
-// two). Collapse stage in us, k_bvh8_collapse / a launch per level, on a
-// surface, blobs and slivers: 250/254, 273/300, 259/265 at 1.1M; 276/296,
-// 323/343, 287/307 at 2M; 345/357, 415/388, 325/337 at 3M.
-constexpr uint32_t kSmallPrims = 1u << 21;
-bool bvh8_small(uint32_t n) { return n <= kSmallPrims; }
-
-// Primitives up to which every internal BVH2 node is expanded first: all of them
-// is about five times the nodes that the BVH8 needs, but at once instead of
-// level after level. Collapse stage in us, surface, blobs and slivers,
-// k_bvh8_expand and k_bvh8_place / k_bvh8_collapse: 32/92, 28/72, 28/71 at
-// 2,003; 53/136, 51/132, 47/117 at 48K; 96/148, 109/179, 102/156 at 300K;
-// 211/250, 246/273, 215/259 at 1.1M; 347/276, 389/323, 353/287 at 2M.
-constexpr uint32_t kExpandPrims = 5u << 18;
-bool bvh8_expands(uint32_t n) { return n <= kExpandPrims; }
-
-// Levels that a block follows while the queue grows, by queued nodes: a node's
-// children hold about 1/2, 1/4, 1/8, ... of its primitives (the larger child is
-// expanded each time), so a block that went on alone with a large one would
-// hold up the launch (300K triangles: 181 to 230 us without the limits). 4096
-// and 16384 instead measured within 5%.
-constexpr uint32_t kThreeLevelNodes = 2048, kTwoLevelNodes = 32768;
-__device__ __forceinline__ uint32_t levels_to_follow(uint32_t m) {
-    return m <= kThreeLevelNodes ? 3u : m <= kTwoLevelNodes ? 2u : 1u;
-}
-
-// work[q] = (first primitive << 32 | BVH2 id), work2[q] = (level << 32 | BVH8
-// id) of queue position q. alloc counts the nodes below the root (the root is
-// node 0), zero before launch 0.
-template <uint32_t SLOT>
-__global__ __launch_bounds__(kBvh8Threads) void k_bvh8_collapse(const uint4* __restrict__ rec, uint32_t n,
-                                                                uint32_t node_count, nxb_bvh8_node* __restrict__ out,
-                                                                uint32_t* __restrict__ prim_idx, uint32_t capacity,
-                                                                uint64_t* work, uint64_t* work2, uint32_t* cnt,
-                                                                uint32_t launch, uint32_t* alloc, uint32_t* flags) {
-    __shared__ RecChildren ch;
-    __shared__ BlockQueue bq;
-    __shared__ uint32_t scan_tmp[kBvh8Threads / 64];
-    __shared__ uint32_t sids, squeue, slevel;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t m = launch == 0 ? 1u : min(cnt[launch], capacity);
-    if (m == 0) return;
-    uint32_t lo = 0;
-    for (uint32_t j = 1; j < launch; ++j) lo += cnt[j];
-    const uint32_t hi = launch == 0 ? 0u : lo + m;
-    // one share per block where the grid holds all items (the block then
-    // follows its subtrees), else whole blocks of items, one level of each
-    const bool follow = m <= gridDim.x * kBvh8Threads;
-    // levels before the rest goes to the queue: all in the first launch and
-    // once the queue shrinks, else few enough that no block runs on alone
-    uint32_t left = kMaxLevels;
-    if (launch != 0 && (launch == 1 || m >= cnt[launch - 1])) left = levels_to_follow(m);
-    const uint32_t per = follow ? (m + gridDim.x - 1) / gridDim.x : (uint32_t)kBvh8Threads;
-    for (uint32_t i0 = blockIdx.x * per; i0 < m; i0 += gridDim.x * per) {
-        uint32_t nodes = min(per, m - i0);
-        uint32_t x = node_count - 1, base = 0, id = 0, level = 0;  // the root
-        if (launch != 0) {
-            if (tid == 0) slevel = 0;
-            __syncthreads();
-            const bool has = tid < nodes && lo + i0 + tid < capacity;
-            const uint64_t v = has ? work[lo + i0 + tid] : (uint64_t)kInvalid, v2 = has ? work2[lo + i0 + tid] : 0ull;
-            x = (uint32_t)v;
-            base = (uint32_t)(v >> 32);
-            id = (uint32_t)v2;
-            atomicMax(&slevel, (uint32_t)(v2 >> 32));
-            __syncthreads();
-            level = slevel;  // the deepest of the share: a bound for its levels
-        }
-        for (;;) {
-            const bool has = tid < nodes;
-            Box pb = {0, 0, 0, 0, 0, 0};
-            uint32_t count = 0, inner = 0;
-            const bool ok = has && level < kMaxLevels && id < capacity &&
-                            collapse_children(rec, n, node_count, x, pb, count, inner, ch, tid);
-            bool good = ok || !has;
-            // the ids of the children, reserved while their slots are chosen
-            const uint32_t ic = ok ? (uint32_t)__popc(inner) : 0u;
-            uint32_t total = 0;
-            const uint32_t excl = block_scan_256(ic, scan_tmp, &total);
-            const bool keep = follow && --left != 0 && total <= (uint32_t)kBvh8Threads;
-            if (tid == 0) sids = total ? 1u + atomic_add_agent(alloc, total) : 0u;
-            if (tid == 64) squeue = total && !keep ? hi + atomic_add_agent(&cnt[launch + 1], total) : 0u;
-            uint32_t assign = 0xFFFFFFFFu;
-            if (ok)
-                assign = SLOT == NXB_SLOT_AUCTION ? auction_slots(pb, ch, tid, count)
-                                                  : greedy_assign(pb, ch, tid, count);
-            __syncthreads();
-            const ChildSink sink{&bq, keep, sids, squeue, level + 1, work, work2, capacity, n};
-            if (ok)
-                good &= emit_lane(ch, tid, pb, count, inner, assign, base, id, excl, sink, out, prim_idx);
-            if (!good) atomic_or_agent(flags, kFlagBadIndex);
-            __syncthreads();  // the block's queue is written, sids and squeue are read
-            if (!keep || total == 0) break;
-            nodes = total;
-            ++level;
-            if (tid < nodes) {
-                x = bq.x[tid];
-                base = bq.base[tid];
-                id = bq.id[tid];
-            }
-        }
-    }
-}
-
-// ---- every node expanded first (single builds of small meshes) --------------
-//
-// What a BVH8 node looks like depends on its BVH2 node alone, except for the
-// numbers of its children and primitives. So one launch makes the BVH8 node of
-// every internal BVH2 node, side by side: the chain of seven record loads, the
-// slots and the quantization are waited for once instead of once per level. The
-// levels that follow only hand out numbers: a level inside a block is two loads,
-// a count and the writes (~2,500 cycles, 1,300 to 2,700 of them the loads'),
-// where collapsing the nodes took ~17,000. 2,003 primitives: 10 us and 18 us;
-// 300K: 34 us and four launches of 6 to 20 us.
-
 // Per internal BVH2 node x, at x - n: its BVH8 node.
 //   kids: 8 ids by slot (kInvalid: free), 8 primitive counts (0: a leaf or free)
 //   node: its 80 bytes, without the child and primitive bases
@@ -1107,8 +1097,12 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_expand(const uint4* __res
             ex.kids[4ull * i + 3] = zero;
             continue;
         }
-        const uint32_t assign =
-            SLOT == NXB_SLOT_AUCTION ? auction_slots(pb, ch, tid, count) : greedy_assign(pb, ch, tid, count);
+        uint32_t used, assign = 0xFFFFFFFFu;
+        const auto box = [&](uint32_t k) { return get_child_box(ch, k, tid); };
+        const uint32_t slots = choose_slots<SLOT>(pb, count, used, box);
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k)
+            if (k < count) assign = with_nib(assign, nib(slots, k), k);
         const PackedNode r = pack_node(ch, tid, pb, inner, assign);
         uint4* k = ex.kids + 4ull * i;
         k[0] = make_uint4(r.kid[0], r.kid[1], r.kid[2], r.kid[3]);
@@ -1121,12 +1115,30 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_expand(const uint4* __res
     }
 }
 
-// Numbers the nodes from the root down, launches and queues as in
-// k_bvh8_collapse. Eight lanes take a node, one its slot: a block's pass places
-// 32 nodes, and the node's words go out in three coalesced stores. (One lane per
-// node: 38 us at 2,003 primitives and 105 at 300K for both kernels, now 31 and
-// 96.) At least kPlaceShare nodes per block: each block and level costs two
-// atomic adds on the same two counters (10 ns each).
+// Levels that a block follows while the queue grows, by queued nodes: a node's
+// children hold about 1/2, 1/4, 1/8, ... of its primitives (the larger child is
+// expanded each time), so a block that went on alone with a large one would
+// hold up the launch. One level more for each measured within 5%.
+constexpr uint32_t kThreeLevelNodes = 2048, kTwoLevelNodes = 32768;
+__device__ __forceinline__ uint32_t levels_to_follow(uint32_t m) {
+    return m <= kThreeLevelNodes ? 3u : m <= kTwoLevelNodes ? 2u : 1u;
+}
+
+// Numbers the nodes from the root down. A block reserves the ids of its nodes'
+// inner children with one atomic add on the node counter alloc (the nodes below
+// the root, node 0; zero before launch 0) and passes the children on to itself,
+// through LDS, while they fit its lanes, else to the next launch through a queue
+// in global memory: work[q] = (first primitive << 32 | BVH2 id), work2[q] =
+// (level << 32 | BVH8 id) of queue position q. Launch l takes the positions
+// [cnt[1] + ... + cnt[l-1], +cnt[l]), counts that earlier launches completed, so
+// no lane ever waits on another (no polling, no spin limit); launch 0 is the
+// root.
+//
+// Eight lanes take a node, one its slot: a block's pass places 32 nodes, and a
+// node's words go out in three coalesced stores. (One lane per node: 38 us at
+// 2,003 primitives and 105 at 300K for both kernels, now 31 and 96.) At least
+// kPlaceShare nodes per block: each block and level costs two atomic adds on the
+// same two counters (10 ns each).
 __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_place(Expanded ex, uint32_t n, uint32_t node_count,
                                                              nxb_bvh8_node* __restrict__ out,
                                                              uint32_t* __restrict__ prim_idx, uint32_t capacity,
@@ -1605,42 +1617,32 @@ hipError_t launch_bvh8_collapse(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_
     if (!sc.rec8 || !sc.work2) return hipErrorInvalidValue;
     const bool auction = sc.slot_mode == NXB_SLOT_AUCTION;
     if (bvh8_small(n)) {
+        if (!sc.ex_kids || !sc.ex_node) return hipErrorInvalidValue;
+        const Expanded ex{sc.ex_kids, sc.ex_node};
+        if (from == 0)  // two blocks of 64 KB LDS per CU
+            hipLaunchKernelGGL(auction ? k_bvh8_expand<NXB_SLOT_AUCTION> : k_bvh8_expand<NXB_SLOT_GREEDY>,
+                               dim3(min((n - 2) / kBvh8Threads + 1, device_cu_count() * 2u)), dim3(kBvh8Threads), 0, s,
+                               sc.rec8, n, 2 * n - 1, ex, sc.flags);
+        const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 4u);
         const uint32_t end = min(from + count, kMaxLevels);
-        if (bvh8_expands(n)) {
-            if (!sc.ex_kids || !sc.ex_node) return hipErrorInvalidValue;
-            const Expanded ex{sc.ex_kids, sc.ex_node};
-            if (from == 0)  // two blocks of 64 KB LDS per CU
-                hipLaunchKernelGGL(auction ? k_bvh8_expand<NXB_SLOT_AUCTION> : k_bvh8_expand<NXB_SLOT_GREEDY>,
-                                   dim3(min((n - 2) / kBvh8Threads + 1, device_cu_count() * 2u)), dim3(kBvh8Threads),
-                                   0, s, sc.rec8, n, 2 * n - 1, ex, sc.flags);
-            const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 4u);
-            for (uint32_t l = from; l < end; ++l)
-                hipLaunchKernelGGL(k_bvh8_place, dim3(l == 0 ? 1u : grid), dim3(kBvh8Threads), 0, s, ex, n, 2 * n - 1,
-                                   out, prim_idx, capacity, sc.work, sc.work2, cnt, l, alloc, sc.flags);
-            return hipGetLastError();
-        }
-        auto kernel = auction ? k_bvh8_collapse<NXB_SLOT_AUCTION> : k_bvh8_collapse<NXB_SLOT_GREEDY>;
-        // two blocks of 67 KB LDS per CU
-        const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 2u);
         for (uint32_t l = from; l < end; ++l)
-            hipLaunchKernelGGL(kernel, dim3(l == 0 ? 1u : grid), dim3(kBvh8Threads), 0, s, sc.rec8, n, 2 * n - 1, out,
+            hipLaunchKernelGGL(k_bvh8_place, dim3(l == 0 ? 1u : grid), dim3(kBvh8Threads), 0, s, ex, n, 2 * n - 1, out,
                                prim_idx, capacity, sc.work, sc.work2, cnt, l, alloc, sc.flags);
         return hipGetLastError();
     }
-    // three 48 KB blocks per CU; a level of m nodes uses ceil(m / 256) blocks
-    const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 3u);
+    const LevelIo io{sc.rec8, n, 2 * n - 1, out, prim_idx, capacity, sc.work, sc.flags};
+    // four 36 KB blocks per CU; a level of m nodes uses ceil(m / 256) blocks
+    const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 4u);
     if (from == 0) {
         hipLaunchKernelGGL(auction ? k_bvh8_top<NXB_SLOT_AUCTION> : k_bvh8_top<NXB_SLOT_GREEDY>, dim3(1),
-                           dim3(kBvh8Threads), 0, s, sc.rec8, n, 2 * n - 1, out, prim_idx, capacity, sc.work, cnt,
-                           sc.flags);
+                           dim3(kBvh8Threads), 0, s, io, cnt);
         from = kBvh8TopLevels;
         count = count > kBvh8TopLevels ? count - kBvh8TopLevels : 0u;
     }
     auto level = auction ? k_bvh8_level<NXB_SLOT_AUCTION> : k_bvh8_level<NXB_SLOT_GREEDY>;
     const uint32_t end = min(from + count, kMaxLevels);
     for (uint32_t l = from; l < end; ++l)
-        hipLaunchKernelGGL(level, dim3(grid), dim3(kBvh8Threads), 0, s, sc.rec8, n, 2 * n - 1, out, prim_idx, capacity,
-                           sc.work, cnt, l, sc.flags);
+        hipLaunchKernelGGL(level, dim3(grid), dim3(kBvh8Threads), 0, s, io, cnt, l);
     return hipGetLastError();
 }
 

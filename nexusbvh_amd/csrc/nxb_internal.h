@@ -67,7 +67,7 @@ struct Bvh8Scratch {
                               // node (batches), (level << 32 | BVH8 id) (one mesh)
     uint32_t slot_mode;       // nxb_slot_assignment of the child slots
     const uint4* rec8 = nullptr;  // wide records of the internal nodes (one mesh)
-    // bvh8_expands(n): [n-1] children (64 bytes) and nodes (80 bytes) of all
+    // bvh8_small(n): [n-1] children (64 bytes) and nodes (80 bytes) of all
     // internal nodes' BVH8 nodes
     uint4* ex_kids = nullptr;
     uint4* ex_node = nullptr;
@@ -149,8 +149,7 @@ hipError_t launch_bvh8_run(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_node*
 // tree of more than kBvh8LevelWords - 1 levels sets the bad-index flag.
 constexpr uint32_t kBvh8LevelWords = 97;
 constexpr uint32_t kBvh8TopLevels = 3;  // large meshes: levels 0..2 run in one single-block launch
-bool bvh8_small(uint32_t n);            // few launches that follow subtrees, else one launch per level
-bool bvh8_expands(uint32_t n);          // of the small: every node expanded first (sc.ex_kids, sc.ex_node)
+bool bvh8_small(uint32_t n);            // every node expanded first, then few launches, else one launch per level
 hipError_t launch_bvh8_collapse(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_node* out, uint32_t* prim_idx,
                                 uint32_t capacity, Bvh8Scratch sc, uint32_t* cnt, uint32_t* alloc, uint32_t from,
                                 uint32_t count, hipStream_t s);

@@ -1,7 +1,7 @@
 """GPU tests of the BVH8 of small meshes made from every node's expansion, against
 the oracle, slot for slot: a pass's 32 nodes and a block's 256 queued ones, long
 chains, both slot assignments, few first launches, and either side of the switch
-to collapsing a level at a time (5 * 2^18 primitives).
+to collapsing a level at a time (2^20 primitives).
 """
 import numpy as np
 import pytest
@@ -14,7 +14,7 @@ from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
-SWITCH = 5 << 18
+SWITCH = 1 << 20
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -75,3 +75,11 @@ def test_either_side_of_expansion(n):
     nodes, prim = _build(tris)
     ref = O.build(tris, 1, 32, 32, 8)
     assert O.compare_bvh8(nodes, prim, ref["bvh8"], ref["prim_idx"], n)[0] == 0
+
+
+def test_levels_with_auction_slots():
+    n = SWITCH + 777
+    tris = scenes.slivers(n, seed=84)
+    nodes, prim = _build(tris, slotAssignment=SlotAssignment.AUCTION)
+    a8, ap = O.collapse_bvh8(O.build(tris, 1, 32, 32, 8)["nodes"], n, 1)
+    assert O.compare_bvh8(nodes, prim, a8, ap, n)[0] == 0
