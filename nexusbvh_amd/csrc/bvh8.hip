@@ -583,19 +583,24 @@ struct Kids {
 // the wave's own; record of lane 4i + j at 65 j + 4 i (conflict-free). All lanes
 // of the wave take part.
 template <uint32_t J>
-__device__ __forceinline__ void fetch_quad(const uint4* rec, uint32_t idx, uint4* buf) {
-    const uint32_t of = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)idx, J * 0x55, 0xF, 0xF, true);  // quad's lane J
-    if (of != kInvalid)
-        __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) void*)(rec + 4ull * of + (__lane_id() & 3u)),
-            (__attribute__((address_space(3))) void*)(buf + 65 * J), 16, 0, 0);
+__device__ __forceinline__ uint32_t of_quad(uint32_t v) {  // the value of the four's lane J
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, J * 0x55, 0xF, 0xF, true);
+}
+__device__ __forceinline__ void fetch16(const uint4* from, uint4* buf) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from,
+                                     (__attribute__((address_space(3))) void*)buf, 16, 0, 0);
+}
+template <uint32_t J>
+__device__ __forceinline__ void fetch_rec(const uint4* rec, uint32_t idx, uint4* buf) {
+    const uint32_t of = of_quad<J>(idx);
+    if (of != kInvalid) fetch16(rec + 4ull * of + (__lane_id() & 3u), buf + 65 * J);
 }
 __device__ __forceinline__ void load_rec8_quads(const uint4* rec, uint32_t idx, uint4* buf, Box& l, Box& r,
                                                 uint32_t& li, uint32_t& ri, uint32_t& ls, uint32_t& rs) {
-    fetch_quad<0>(rec, idx, buf);
-    fetch_quad<1>(rec, idx, buf);
-    fetch_quad<2>(rec, idx, buf);
-    fetch_quad<3>(rec, idx, buf);
+    fetch_rec<0>(rec, idx, buf);
+    fetch_rec<1>(rec, idx, buf);
+    fetch_rec<2>(rec, idx, buf);
+    fetch_rec<3>(rec, idx, buf);
     wait_memory_ops();
     wave_lds_sync();
     const uint32_t lane = __lane_id();
@@ -751,13 +756,13 @@ __device__ __forceinline__ uint32_t grid_exponents(const Box& pb, float& ix, flo
     return e0 | (e1 << 8) | (e2 << 16);
 }
 
-// Puts the lane's node into the stage, byte by byte at its slots, without the
-// child and primitive bases, and its children.
-__device__ __forceinline__ void stage_node(NodeStage& st, uint32_t tid, const Box& pb, const Kids& K, uint32_t count,
-                                           uint32_t slots, uint32_t im, uint32_t lm) {
+// Puts the lane's node into the stage's words w, byte by byte at its slots,
+// without the child and primitive bases.
+template <typename KidsOf>
+__device__ __forceinline__ void stage_node(uint4* w, const Box& pb, const KidsOf& K, uint32_t count, uint32_t slots,
+                                           uint32_t im, uint32_t lm) {
     float ix, iy, iz;
     const uint32_t e = grid_exponents(pb, ix, iy, iz);
-    uint4* w = st.w + 5 * tid;
     w[0] = make_uint4(__float_as_uint(pb.lx), __float_as_uint(pb.ly), __float_as_uint(pb.lz), e | (im << 24));
 #pragma unroll
     for (uint32_t i = 1; i < 5; ++i) w[i] = make_uint4(0, 0, 0, 0);
@@ -774,7 +779,6 @@ __device__ __forceinline__ void stage_node(NodeStage& st, uint32_t tid, const Bo
         q[32] = (uint8_t)q_ceil((b.hx - pb.lx) * ix);
         q[40] = (uint8_t)q_ceil((b.hy - pb.ly) * iy);
         q[48] = (uint8_t)q_ceil((b.hz - pb.lz) * iz);
-        st.kid[s][tid] = make_uint2(K.id[k], K.prims[k]);
     }
 }
 
@@ -811,7 +815,10 @@ __device__ __forceinline__ uint32_t collapse_nodes(NodeStage& st, uint32_t* scan
         const uint32_t slots = choose_slots<SLOT>(pb, count, used, [&](uint32_t i) { return K.box[i]; });
 #pragma unroll
         for (uint32_t i = 0; i < 8; ++i) im |= ((inner >> i) & 1u) << nib(slots, i);
-        stage_node(st, tid, pb, K, count, slots, im, used & ~im);
+        stage_node(st.w + 5 * tid, pb, K, count, slots, im, used & ~im);
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i)
+            if (i < count) st.kid[nib(slots, i)][tid] = make_uint2(K.id[i], K.prims[i]);
     }
     lds_barrier();
     const uint32_t base = ids.first() + excl;
@@ -899,7 +906,8 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_top(LevelIo io, uint32_t*
 // (second bound: waves per SIMD, four as the LDS allows; the auction needs the
 // registers of three)
 template <uint32_t SLOT>
-__global__ __launch_bounds__(kBvh8Threads, SLOT == NXB_SLOT_AUCTION ? 3 : 4) void k_bvh8_level(LevelIo io, uint32_t* cnt, uint32_t level) {
+__global__ __launch_bounds__(kBvh8Threads, SLOT == NXB_SLOT_AUCTION ? 3 : 4) void k_bvh8_level(
+    LevelIo io, uint32_t* cnt, uint32_t level) {
     __shared__ NodeStage st;
     __shared__ uint32_t scan_tmp[kBvh8Threads / 64];
     __shared__ uint32_t sbase;
@@ -1319,16 +1327,15 @@ struct TopQueue {
 // region out, children's work items at queue positions qbase.., their node
 // ids nbase.. (tree-local), its leaves at primIdx slots prim_base.. (local to
 // the tree; each node takes its own from the tree's counter, so no subtree
-// sizes are read). The children go to the level queue in work/work2/work3
+// sizes are read). The children go to the level queue in work2/work3
 // (positions below capacity), or with lq to a block's LDS queue (positions
 // below kTopQueue).
 // ti = {first primitive, primitive count, region start, region capacity}.
 __device__ __forceinline__ void emit_tree_node(const ChildBoxes& cbx, uint32_t tid, const Collapsed& c,
                                                uint32_t tree, uint32_t self, uint32_t qbase, uint32_t nbase,
                                                uint32_t prim_base, uint4 ti, nxb_bvh8_node* out,
-                                               uint32_t* prim_idx, uint32_t capacity, uint64_t* work,
-                                               uint64_t* work2, uint64_t* work3, uint32_t* flags,
-                                               TopQueue* lq = nullptr) {
+                                               uint32_t* prim_idx, uint32_t capacity, uint64_t* work2,
+                                               uint64_t* work3, uint32_t* flags, TopQueue* lq = nullptr) {
     const uint32_t ic = (uint32_t)__popc(c.im);
     const uint32_t leaf_count = c.count - ic;
     if (self >= ti.w || (ic != 0 && nbase + ic > ti.w) || (leaf_count != 0 && prim_base + leaf_count > ti.y)) {
@@ -1358,7 +1365,6 @@ __device__ __forceinline__ void emit_tree_node(const ChildBoxes& cbx, uint32_t t
                 lq->self[q] = nbase + rank;
             } else {
                 // read by the next level's kernel
-                work[q] = ch;
                 work2[q] = ((uint64_t)pr << 32) | pl;
                 work3[q] = ((uint64_t)tree << 32) | (nbase + rank);
             }
@@ -1373,22 +1379,114 @@ __device__ __forceinline__ void emit_tree_node(const ChildBoxes& cbx, uint32_t t
                     c.lm);
 }
 
+// As Kids, of BVH2 nodes: an inner child's children, a leaf's kInvalid and
+// primitive index.
+struct TreeKids {
+    Box box[8];
+    uint32_t left[8], right[8];
+};
+
+// Two nodes per lane (c0, c1; kInvalid: none) as load_rec8_quads fetches a
+// record: two lanes each.
+template <uint32_t J>
+__device__ __forceinline__ void fetch_pair(const uint4* nodes, uint32_t c0, uint32_t c1, uint4* buf) {
+    const uint32_t o0 = of_quad<J>(c0), o1 = of_quad<J>(c1), q = __lane_id() & 3u;
+    if (o0 != kInvalid) fetch16(nodes + 2ull * (q & 2u ? o1 : o0) + (q & 1u), buf + 65 * J);
+}
+__device__ __forceinline__ void load_pair_quads(const nxb_bvh2_node* b2, uint32_t c0, uint32_t c1, uint4* buf, Box& b0,
+                                                Box& b1, uint32_t& l0, uint32_t& r0, uint32_t& l1, uint32_t& r1) {
+    const uint4* nodes = reinterpret_cast<const uint4*>(b2);
+    fetch_pair<0>(nodes, c0, c1, buf);
+    fetch_pair<1>(nodes, c0, c1, buf);
+    fetch_pair<2>(nodes, c0, c1, buf);
+    fetch_pair<3>(nodes, c0, c1, buf);
+    wait_memory_ops();
+    wave_lds_sync();
+    const uint32_t lane = __lane_id();
+    const uint4* p = buf + 65 * (lane & 3u) + 4 * (lane >> 2);
+    const uint4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3];
+    wave_lds_sync();
+    b0.lx = __uint_as_float(q0.x); b0.ly = __uint_as_float(q0.y); b0.lz = __uint_as_float(q0.z);
+    b0.hx = __uint_as_float(q0.w); b0.hy = __uint_as_float(q1.x); b0.hz = __uint_as_float(q1.y);
+    b1.lx = __uint_as_float(q2.x); b1.ly = __uint_as_float(q2.y); b1.lz = __uint_as_float(q2.z);
+    b1.hx = __uint_as_float(q2.w); b1.hy = __uint_as_float(q3.x); b1.hz = __uint_as_float(q3.y);
+    l0 = q1.z; r0 = q1.w; l1 = q3.z; r1 = q3.w;
+}
+
+// collapse_kids from BVH2 nodes, of the node with children c0 and c1.
+__device__ __forceinline__ bool collapse_tree_kids(const nxb_bvh2_node* b2, uint32_t node_count, bool has, uint32_t c0,
+                                                   uint32_t c1, TreeKids& K, Box& pb, uint32_t& count, uint32_t& inner,
+                                                   uint4* buf) {
+    count = 0;
+    inner = 0;
+    bool ok = has, live = has;
+    uint32_t msb = 0;
+#pragma unroll
+    for (uint32_t t = 0; t < 7; ++t) {
+        if (live && max(c0, c1) >= node_count) {
+            ok = false;
+            live = false;
+        }
+        if (!ballot(live)) break;
+        Box b0, b1;
+        uint32_t l0, r0, l1, r1;
+        load_pair_quads(b2, live ? c0 : kInvalid, c1, buf, b0, b1, l0, r0, l1, r1);
+        if (!live) continue;
+        if (t == 0) pb = box_union(b0, b1);
+        const bool first_is_1 = !(box_area(b0) < box_area(b1));
+        const uint32_t sl = first_is_1 ? l1 : l0, sr = first_is_1 ? r1 : r0;
+        const Box bs = first_is_1 ? b1 : b0;
+        K.box[t + 1] = first_is_1 ? b0 : b1;
+        K.left[t + 1] = first_is_1 ? l0 : l1;
+        K.right[t + 1] = first_is_1 ? r0 : r1;
+        inner |= (sl != kInvalid ? 1u << msb : 0u) | (K.left[t + 1] != kInvalid ? 2u << t : 0u);
+        const uint32_t top = 31u - (uint32_t)__clz(inner | 1u);
+        c0 = K.left[t + 1];  // of the highest inner child
+        c1 = K.right[t + 1];
+#pragma unroll
+        for (uint32_t j = 0; j <= t; ++j) {
+            const bool here = msb == j;
+            K.box[j].lx = here ? bs.lx : K.box[j].lx;
+            K.box[j].ly = here ? bs.ly : K.box[j].ly;
+            K.box[j].lz = here ? bs.lz : K.box[j].lz;
+            K.box[j].hx = here ? bs.hx : K.box[j].hx;
+            K.box[j].hy = here ? bs.hy : K.box[j].hy;
+            K.box[j].hz = here ? bs.hz : K.box[j].hz;
+            K.left[j] = here ? sl : K.left[j];
+            K.right[j] = here ? sr : K.right[j];
+            c0 = top == j ? K.left[j] : c0;
+            c1 = top == j ? K.right[j] : c1;
+        }
+        count = t + 2;
+        live = inner != 0;
+        if (t < 6 && live) {
+            msb = top;
+            inner &= ~(1u << top);
+        }
+    }
+    return ok;
+}
+
 // A level of a forest whose trees each own an output region (batched
-// builds). Queue position k (level order, as in k_bvh8_level) holds work[k] =
-// its BVH2 node, work2[k] = that node's children and work3[k] = (tree << 32 |
-// tree-local node id); tree t writes its nodes to out + info[t].z and its
+// builds). Queue position k (level order, as in k_bvh8_level) holds work2[k] =
+// its BVH2 node's children and work3[k] = (tree << 32 | tree-local node id);
+// tree t writes its nodes to out + info[t].z and its
 // primitives to prim_idx + info[t].x, so each tree's BVH8 is contiguous with
 // root 0 and needs no compaction afterwards. Node ids come from ids[t] and
-// each node's primIdx slots for its leaves from prims[t].
+// each node's primIdx slots for its leaves from prims[t]. Children, fetches and
+// node words as in collapse_nodes, the children's BVH2 ids not kept at all (162
+// registers, three waves per SIMD; held to 128 it spills and takes 1,400 us):
+// levels 3 and below of 2,048 meshes 1,080 -> 880 us.
 template <uint32_t SLOT>
 __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_tree_level(
-    const nxb_bvh2_node* __restrict__ b2, uint32_t node_count, nxb_bvh8_node* __restrict__ out, uint32_t* prim_idx,
-    uint32_t capacity, uint64_t* work, uint64_t* work2, uint64_t* work3, uint32_t* cnt, uint32_t level,
-    const uint4* __restrict__ info, uint32_t trees, uint32_t* ids, uint32_t* prims, uint32_t* flags) {
-    __shared__ ChildBoxes cbx;
+    const nxb_bvh2_node* __restrict__ b2, uint32_t node_count, nxb_bvh8_node* __restrict__ out,
+    uint32_t* __restrict__ prim_idx, uint32_t capacity, uint64_t* work2, uint64_t* work3, uint32_t* cnt,
+    uint32_t level, const uint4* __restrict__ info, uint32_t trees, uint32_t* ids, uint32_t* prims, uint32_t* flags) {
+    __shared__ uint4 words[5 * kBvh8Threads];
+    __shared__ uint32_t dest[kBvh8Threads];  // node of each lane, from out; kInvalid: none
     __shared__ uint32_t scan_tmp[kBvh8Threads / 64];
     __shared__ uint32_t sbase;
-    const uint32_t tid = threadIdx.x;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, w0 = tid & ~63u;
     const uint32_t m = cnt[level];
     if (m == 0) return;
     uint32_t lo = 0;
@@ -1400,38 +1498,76 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_tree_level(
     }
     for (uint32_t k0 = lo + blockIdx.x * kBvh8Threads; k0 < hi; k0 += gridDim.x * kBvh8Threads) {
         const uint32_t k = k0 + tid;
-        Collapsed c;
-        bool ok = false;
-        uint32_t tree = kInvalid, self = 0;
+        TreeKids K = {};
+        Box pb = {0, 0, 0, 0, 0, 0};
+        uint32_t tree = kInvalid, self = 0, count = 0, inner = 0;
         uint4 ti = make_uint4(0, 0, 0, 0);
-        if (k < hi && k < capacity) {
-            const uint64_t v = work[k], t3 = work3[k];
-            const uint32_t x = (uint32_t)v;
+        uint64_t lr = 0;
+        bool has = k < hi && k < capacity;
+        if (has) {
+            const uint64_t t3 = work3[k];
+            lr = work2[k];
             self = (uint32_t)t3;
-            const uint32_t t = (uint32_t)(t3 >> 32);
-            ti = info[min(t, trees - 1u)];
-            const bool have_lr = level > 0;  // written with work[k] by the level above
-            const uint64_t lr = have_lr ? work2[k] : 0ull;
-            ok = t < trees && x < node_count &&
-                 collapse_node(b2, node_count, x, c, cbx, tid, SLOT, have_lr, (uint32_t)lr, (uint32_t)(lr >> 32));
-            if (ok) tree = t;
+            tree = (uint32_t)(t3 >> 32);
+            ti = info[min(tree, trees - 1u)];
+            has = tree < trees;
         }
-        if (k < hi && !ok) atomic_or_agent(flags, kFlagBadIndex);
-        const uint32_t ic = ok ? (uint32_t)__popc(c.im) : 0u;
-        const uint32_t leaves = ok ? c.count - ic : 0u;
+        const bool ok = collapse_tree_kids(b2, node_count, has, (uint32_t)lr, (uint32_t)(lr >> 32), K, pb, count,
+                                           inner, words + 5 * w0);
+        if (!ok) {
+            tree = kInvalid;
+            if (k < hi) atomic_or_agent(flags, kFlagBadIndex);
+        }
+        const uint32_t ic = ok ? (uint32_t)__popc(inner) : 0u;
+        const uint32_t leaves = ok ? count - ic : 0u;
         uint32_t total = 0;
-        const uint32_t excl = block_scan_256(ic, scan_tmp, &total);
+        const uint32_t excl = block_scan_256<true>(ic, scan_tmp, &total);
         // lanes without inner children or leaves stay in their tree's run
         // (count 0), so a wave whose nodes lie in one tree takes its ids and
         // its primIdx slots with one atomic each
         const uint32_t nbase = alloc_tree_ids(ids, tree, ic);
         const uint32_t pbase = alloc_tree_ids(prims, tree, leaves);
         if (tid == 0) sbase = total ? hi + atomic_add_agent(&cnt[level + 1], total) : 0u;
-        __syncthreads();
-        const uint32_t qbase = sbase + excl;
-        if (ok)
-            emit_tree_node(cbx, tid, c, tree, self, qbase, nbase, pbase, ti, out, prim_idx, capacity, work, work2,
-                           work3, flags);
+        const bool fits = ok && self < ti.w && (ic == 0 || nbase + ic <= ti.w) &&
+                          (leaves == 0 || pbase + leaves <= ti.y);
+        if (ok && !fits) atomic_or_agent(flags, kFlagBadIndex);
+        uint32_t im = 0, used = 0, slots = 0;
+        if (fits) {
+            slots = choose_slots<SLOT>(pb, count, used, [&](uint32_t i) { return K.box[i]; });
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i) im |= ((inner >> i) & 1u) << nib(slots, i);
+            stage_node(words + 5 * tid, pb, K, count, slots, im, used & ~im);
+            *reinterpret_cast<uint2*>(&words[5 * tid + 1]) = make_uint2(ic ? nbase : 0u, leaves ? pbase : 0u);
+        }
+        dest[tid] = fits ? ti.z + self : kInvalid;
+        lds_barrier();
+        if (fits) {
+            const uint32_t qbase = sbase + excl, lm = used & ~im;
+            bool good = qbase + ic <= capacity;
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i) {
+                if (i >= count) break;
+                const uint32_t s = nib(slots, i);
+                if ((inner >> i) & 1u) {
+                    const uint32_t rank = bits_below(im, s), q = qbase + rank;
+                    if (q < capacity) {  // read by the next level's kernel
+                        work2[q] = ((uint64_t)K.right[i] << 32) | K.left[i];
+                        work3[q] = ((uint64_t)tree << 32) | (nbase + rank);
+                    }
+                } else {
+                    prim_idx[ti.x + pbase + bits_below(lm, s)] = K.right[i];
+                }
+            }
+            if (!good) atomic_or_agent(flags, kFlagBadIndex);
+        }
+        // 16 bytes a lane: a tree's nodes are consecutive for the most part
+        uint4* o = reinterpret_cast<uint4*>(out);
+#pragma unroll
+        for (uint32_t i = 0; i < 5; ++i) {
+            const uint32_t c = lane + 64 * i, to = dest[w0 + c / 5u];
+            if (to != kInvalid) o[5ull * to + c % 5u] = words[5 * w0 + c];
+        }
+        lds_barrier();  // sbase, dest and the words are read before the next nodes
     }
 }
 
@@ -1448,7 +1584,7 @@ constexpr uint32_t kTopTrees = 4;
 template <uint32_t SLOT>
 __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_tree_top(
     const nxb_bvh2_node* __restrict__ b2, uint32_t n, uint32_t node_count, nxb_bvh8_node* __restrict__ out,
-    uint32_t* prim_idx, uint32_t capacity, uint64_t* work, uint64_t* work2, uint64_t* work3, uint32_t* cnt,
+    uint32_t* prim_idx, uint32_t capacity, uint64_t* work2, uint64_t* work3, uint32_t* cnt,
     const uint4* __restrict__ info, uint32_t trees, const uint32_t* __restrict__ mesh_lo, uint32_t* ids,
     uint32_t* prims, uint32_t* flags) {
     __shared__ ChildBoxes cbx;
@@ -1506,7 +1642,7 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_tree_top(
         __syncthreads();  // this level's queue is read; sbase and the next count are set
         if (ok)
             emit_tree_node(cbx, tid, c, tree, self, last ? sbase + excl : excl, nbase, pbase, ti, out, prim_idx,
-                           capacity, work, work2, work3, flags, last ? nullptr : &tq[cur ^ 1u]);
+                           capacity, work2, work3, flags, last ? nullptr : &tq[cur ^ 1u]);
         __syncthreads();  // the next level's queue is written
     }
     if (tid < nt) {
@@ -1673,12 +1809,12 @@ hipError_t launch_bvh8_tree_levels(const nxb_bvh2_node* bvh2, uint32_t n, uint32
     hipLaunchKernelGGL(k_bvh8_forest_level_init, dim3(1), dim3(128), 0, s, cnt, 0u);
     auto top = auction ? k_bvh8_tree_top<NXB_SLOT_AUCTION> : k_bvh8_tree_top<NXB_SLOT_GREEDY>;
     hipLaunchKernelGGL(top, dim3((trees + kTopTrees - 1) / kTopTrees), dim3(kBvh8Threads), 0, s, bvh2, n,
-                       2 * n - trees, out, prim_idx, capacity, sc.work, sc.work2, work3, cnt, info, trees, mesh_lo,
+                       2 * n - trees, out, prim_idx, capacity, sc.work2, work3, cnt, info, trees, mesh_lo,
                        ids, prims, sc.flags);
     auto level = auction ? k_bvh8_tree_level<NXB_SLOT_AUCTION> : k_bvh8_tree_level<NXB_SLOT_GREEDY>;
     for (uint32_t l = kTreeTopLevels; l < levels; ++l)
         hipLaunchKernelGGL(level, dim3(grid), dim3(kBvh8Threads), 0, s, bvh2, 2 * n - trees, out, prim_idx,
-                           capacity, sc.work, sc.work2, work3, cnt, l, info, trees, ids, prims, sc.flags);
+                           capacity, sc.work2, work3, cnt, l, info, trees, ids, prims, sc.flags);
     hipLaunchKernelGGL(k_bvh8_level_total, dim3(1), dim3(1), 0, s, cnt, levels, sc.ctr, sc.flags);
     return hipGetLastError();
 }
