@@ -568,7 +568,8 @@ nxb_status nxb_batch_plan_create(const void* d_prims, nxb_prim_type type, uint32
            o_ka = take(N * 8), o_kb = take(N * 8), o_kt = take(sort_n * 8), o_vb = take(N * 4),
            o_vt = take(sort_n * 4), o_hist = take(kHistCopies * kHistCopyWords * 4),
            o_counts = take(p->counts_words * 4), o_parent = take(N * 4), o_recs = take(N * 32),
-           o_csz = take(N * 4), o_nsize = take(N * 4), o_work = take(C8 * 8), o_work2 = take(C8 * 8), o_ctr = take(64), o_grab = take(64), o_lvl = take(kBvh8LevelWords * 4),
+           o_csz = take(N * 4), o_nsize = take(N * 4), o_work = take(CC * 8), o_work2 = take(C8 * 8),
+           o_ctr = take(64), o_grab = take(64), o_lvl = take(kBvh8LevelWords * 4),
            o_tmp8 = take(CC * sizeof(nxb_bvh8_node)), o_nkeys = take(CC * 4), o_nko = take(CC * 4),
            o_nvo = take(CC * 4), o_start = take((M + 1) * 4), o_o2n = take(CC * 4),
            o_work3 = take(compact ? 0 : C8 * 8), o_info = take(M * sizeof(uint4)), o_ids = take(M * 4),

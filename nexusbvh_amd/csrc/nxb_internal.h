@@ -58,7 +58,7 @@ struct HplocScratch {
 constexpr uint32_t kHplocCounterWords = 256;
 
 struct Bvh8Scratch {
-    uint64_t* work;           // [capacity] (prim base << 32 | BVH2 index) per BVH8 node
+    uint64_t* work;           // [capacity] (prim base << 32 | BVH2 index) per BVH8 node; unused by batch levels
     unsigned long long* ctr;  // (finished << 32 | allocated) BVH8 nodes
     uint32_t* grab;           // work grab counter (own cache line)
     uint32_t* flags;

@@ -1,8 +1,7 @@
-"""GPU tests of the BVH8 collapse of small meshes (a launch that follows its
-subtrees inside a block) against the oracle, slot for slot: sizes where a
-level's nodes pass the eight-lanes-per-node limit (96) and the block's lanes
-(256), skewed and nested geometry, few first launches, and either side of the
-switch to a launch per level (2^21 primitives).
+"""GPU tests of the BVH8 collapse of small meshes (launches that follow subtrees
+inside a block) against the oracle, slot for slot: levels of fewer and of more nodes
+than a pass or a block takes, skewed and nested geometry and few first launches; and
+of 2^21 primitives and one more, a launch per level.
 """
 import numpy as np
 import pytest

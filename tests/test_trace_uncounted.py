@@ -1,5 +1,5 @@
-"""GPU tests of the traversal without counts (no d_stats): eight lanes per ray
-up to 2^17 rays, one lane per ray above. Bar as in test_trace.py: the same
+"""GPU tests of the traversal without counts (no d_stats): eight lanes per ray and
+node up to 2^17 rays, one lane per ray above. Bar as in test_trace.py: the same
 triangle and bit-identical t, u and v as the brute force over all triangles.
 """
 import numpy as np
