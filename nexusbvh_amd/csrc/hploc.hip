@@ -543,15 +543,18 @@ __device__ __forceinline__ void ploc_merge(HplocLds<GW, KEEP>& s, bool has_task,
     if constexpr (KEEP != kKeepNodes) sz = s.sz[gbase + gl];
 
     const uint32_t threshold = final ? 1u : C;
-    // One radius for every task (no per-segment table): the unrolled search for
-    // radius 8, a loop for others. With a table the loop runs to the largest
-    // radius of the wave's groups (each group's is uniform over it).
-    const uint32_t fixed_r = rp.table ? 0u : min(rp.radius, (uint32_t)kMaxRadius);
-    uint32_t R = fixed_r, r_wave = fixed_r;
+    // The radius is uniform over a group. The search runs to the larger of the
+    // wave's two, unrolled for 8; only where a table gave two tasks different
+    // ones (plain_r == 0) does each lane mask the distances past its own (two of
+    // 22 instructions a distance). Masked whenever there was a table: learned
+    // radii at 1.9M primitives 508 -> 473 us with the policy's kernels, one task
+    // a wave 560 -> 511.
+    uint32_t R = min(rp.radius, (uint32_t)kMaxRadius), r_wave = R, plain_r = R;
     if (rp.table) {
-        R = has_task ? radius_for(rp, l_start, r_end) : 1u;
-        r_wave = GW == 64 ? __builtin_amdgcn_readfirstlane(R)
-                          : max(__builtin_amdgcn_readlane(R, 0), __builtin_amdgcn_readlane(R, 32));
+        R = has_task ? radius_for(rp, l_start, r_end) : 0u;
+        const uint32_t r0 = __builtin_amdgcn_readfirstlane(R), r1 = GW == 64 ? r0 : __builtin_amdgcn_readlane(R, 32);
+        r_wave = max(r0, r1);
+        plain_r = min(r0, r1) != 0 && r0 != r1 ? 0u : r_wave;
     }
 
     // The group's first num slots hold own/id/sz of its clusters here and after
@@ -563,8 +566,8 @@ __device__ __forceinline__ void ploc_merge(HplocLds<GW, KEEP>& s, bool has_task,
         if (!ballot(run)) break;
         // ---- FindNearestNeighbor (BinaryBuilder.cu:127-163) ----
         uint32_t nn, best;
-        if (fixed_r == 8) nn = nearest<8, false>(s, own, slot, gl, 0, 8u, best);
-        else if (fixed_r) nn = nearest<2, false>(s, own, slot, gl, 0, fixed_r, best);
+        if (plain_r == 8) nn = nearest<8, false>(s, own, slot, gl, 0, 8u, best);
+        else if (plain_r) nn = nearest<2, false>(s, own, slot, gl, 0, plain_r, best);
         else nn = nearest<2, true>(s, own, slot, gl, (int)R + 1, r_wave, best);
         if (ballot(run && best >= kInfBits)) {
             nn = nearest<1, true>(s, own, slot, gl, min((int)num - (int)gl, (int)R + 1), r_wave, best);

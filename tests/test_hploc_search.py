@@ -86,3 +86,22 @@ def test_either_side_of_staged_records(n, mode):
         B.FreeDeviceBVH(bvh)
     ref = O.build(tris, 1, 32, 32 if mode == MergeMode.WAVE32 else 64, 8)
     assert O.compare_bvh8(nodes, prim, ref["bvh8"], ref["prim_idx"], n)[0] == 0
+
+
+@pytest.mark.parametrize("mode", [MergeMode.WAVE32, MergeMode.WAVE64])
+@pytest.mark.parametrize("above", [1, 8, 16])
+@pytest.mark.parametrize("radii,seg_log2", [([8], 6), ([16], 5), ([4, 8], 4), ([2, 8, 16], 6), ([0, 1, 16], 8)])
+def test_radius_tables(radii, seg_log2, above, mode):
+    """Tables that give a wave's two tasks the same radius or different ones."""
+    n = 9_001
+    keys = np.sort(np.random.default_rng(8).integers(0, 1 << 63, n, dtype=np.uint64))
+    nodes0, _, _ = O.scene_bounds(scenes.uniform(n, seed=85), 1)
+    perm = np.random.default_rng(9).permutation(n).astype(np.uint32)
+    table = np.random.default_rng(10).choice(np.array(radii, dtype=np.uint8), (n >> seg_log2) + 1)
+    tbl = native.DeviceBuffer.from_array(table)
+    cfg = BuildConfig(mergeMode=mode, searchRadius=above, radiusPolicy=B.RadiusPolicy.TABLE, radiusTable=tbl,
+                      radiusTableLen=len(table), segmentLog2=seg_log2)
+    ref = O.hploc(keys, perm, nodes0, 32 if mode == MergeMode.WAVE32 else 64, above, table=table, seg_log2=seg_log2)
+    nodes = native.DeviceBuffer.from_array(np.concatenate([nodes0[:n], nodes0[: n - 1]]))
+    stages.hploc(native.DeviceBuffer.from_array(keys), native.DeviceBuffer.from_array(perm), n, 64, nodes, cfg)
+    assert stages.nodes_to_host(nodes, 2 * n - 1).tobytes() == ref[: 2 * n - 1].tobytes()
