@@ -47,9 +47,10 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 STAGE_KEYS = ("bounds", "morton", "sort", "hploc", "bvh8")
 # kernels of each stage, for the counter summary
-STAGE_KERNELS = {"bounds": ("k_scene_bounds",), "morton": ("k_morton_hist",),
-                 "sort": ("k_sort_upsweep", "k_sort_rowscan", "k_sort_downsweep", "k_copy_pairs"),
-                 "hploc": ("k_hploc",), "bvh8": ("k_bvh8_top", "k_bvh8_level")}
+STAGE_KERNELS = {"bounds": ("k_scene_bounds",), "morton": ("k_morton_hist", "k_morton<"),
+                 "sort": ("k_sort_upsweep", "k_sort_rowscan", "k_sort_downsweep", "k_sort_runs", "k_sort_merge",
+                          "k_copy_pairs"),
+                 "hploc": ("k_hploc",), "bvh8": ("k_bvh8_top", "k_bvh8_level", "k_bvh8_expand", "k_bvh8_place")}
 TRAFFIC_PATH = os.path.join(ROOT, "profiles", "pmc_traffic.json")
 
 
