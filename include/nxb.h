@@ -352,6 +352,12 @@ nxb_status nxb_mlp_radius_table(const float* d_params, const float* d_features, 
 nxb_status nxb_mlp_gradients(const float* d_params, const float* d_features, const uint8_t* d_labels,
                              uint32_t count, float* d_grads, float* d_loss, nxb_stream_t stream);
 
+/* The same with both buffers (grads_bytes and loss_bytes long) zeroed first,
+ * in one launch on the stream. */
+nxb_status nxb_mlp_gradients_from_zero(const float* d_params, const float* d_features, const uint8_t* d_labels,
+                                       uint32_t count, float* d_grads, size_t grads_bytes, float* d_loss,
+                                       size_t loss_bytes, nxb_stream_t stream);
+
 /* One Adam step (step >= 1) on d_params with moment buffers d_m, d_v. */
 nxb_status nxb_mlp_adam_step(float* d_params, const float* d_grads, float* d_m, float* d_v, uint32_t step,
                              float lr, float beta1, float beta2, float eps, nxb_stream_t stream);

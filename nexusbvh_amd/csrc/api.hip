@@ -1112,6 +1112,14 @@ nxb_status nxb_mlp_gradients(const float* d_params, const float* d_features, con
     return NXB_SUCCESS;
 }
 
+nxb_status nxb_mlp_gradients_from_zero(const float* d_params, const float* d_features, const uint8_t* d_labels,
+                                       uint32_t count, float* d_grads, size_t grads_bytes, float* d_loss,
+                                       size_t loss_bytes, nxb_stream_t stream) {
+    if ((grads_bytes && !d_grads) || (loss_bytes && !d_loss)) return NXB_ERROR_INVALID_VALUE;
+    NXB_HIP(launch_zero_pair(d_grads, grads_bytes, d_loss, loss_bytes, as_hip(stream)));
+    return nxb_mlp_gradients(d_params, d_features, d_labels, count, d_grads, d_loss, stream);
+}
+
 nxb_status nxb_mlp_adam_step(float* d_params, const float* d_grads, float* d_m, float* d_v, uint32_t step, float lr,
                              float beta1, float beta2, float eps, nxb_stream_t stream) {
     if (!d_params || !d_grads || !d_m || !d_v || step == 0) return NXB_ERROR_INVALID_VALUE;

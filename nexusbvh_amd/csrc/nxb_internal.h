@@ -188,6 +188,7 @@ hipError_t launch_segment_sah(const nxb_bvh2_node* nodes, uint32_t n, uint32_t s
                               double* seg_cost, hipStream_t s);
 hipError_t launch_mlp_table(const float* params, const float* feat, uint32_t count, float min_confidence,
                             uint8_t* table, float* logits, uint32_t* fallbacks, hipStream_t s);
+hipError_t launch_zero_pair(void* a, size_t a_bytes, void* b, size_t b_bytes, hipStream_t s);
 hipError_t launch_mlp_grad(const float* params, const float* feat, const uint8_t* labels, uint32_t count,
                            float* grads, float* loss, hipStream_t s);
 hipError_t launch_adam(float* params, const float* grads, float* m, float* v, uint32_t step, float lr, float beta1,

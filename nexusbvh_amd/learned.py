@@ -65,10 +65,8 @@ def segment_sah(nodes: DeviceBuffer, n: int, scene: DeviceBuffer, seg_log2: int)
 
 def mlp_gradients(params: DeviceBuffer, feats: DeviceBuffer, labels: DeviceBuffer, count: int,
                   grads: DeviceBuffer, loss: DeviceBuffer) -> None:
-    zero(grads)
-    zero(loss)
-    check(lib().nxb_mlp_gradients(params.address, feats.address, labels.address, count, grads.address,
-                                  loss.address, None), "mlp_gradients")
+    check(lib().nxb_mlp_gradients_from_zero(params.address, feats.address, labels.address, count, grads.address,
+                                            grads.nbytes, loss.address, loss.nbytes, None), "mlp_gradients")
 
 
 def mlp_radius_table(params: DeviceBuffer, feats: DeviceBuffer, count: int, min_confidence: float,

@@ -111,6 +111,8 @@ _SIGNATURES = {
     "nxb_mlp_radius_table": (c_int, [c_void_p, c_void_p, c_uint32, c_float, c_void_p, c_void_p, c_void_p,
                                      c_void_p]),
     "nxb_mlp_gradients": (c_int, [c_void_p, c_void_p, c_void_p, c_uint32, c_void_p, c_void_p, c_void_p]),
+    "nxb_mlp_gradients_from_zero": (c_int, [c_void_p, c_void_p, c_void_p, c_uint32, c_void_p, c_size_t, c_void_p,
+                                            c_size_t, c_void_p]),
     "nxb_mlp_adam_step": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_float, c_float, c_float,
                                   c_float, c_void_p]),
     "nxb_last_learned_stats": (None, [POINTER(c_uint32), POINTER(c_uint32)]),

@@ -410,3 +410,19 @@ def test_shipped_network_at_full_size(nx):
     say("learned full size SAH", m8.bvh2Cost, m8.bvh8Cost, "r8", r8.bvh2Cost, r8.bvh8Cost, "fallbacks", fb.value)
     assert m2.bvh2Cost == pytest.approx(m8.bvh2Cost, rel=1e-6)
     assert m8.bvh2Cost < r8.bvh2Cost
+
+
+@gpu
+@pytest.mark.parametrize("grads_bytes,loss_bytes,skip", [(0, 0, 0), (1, 4, 0), (7, 5, 1), (4096, 3, 3), (5508 * 4, 4, 0),
+                                                       (1_000_003, 4099, 2), (4, 9 << 20, 0)])
+def test_gradient_buffers_are_zeroed_whole(nx, grads_bytes, loss_bytes, skip):
+    """No samples: both buffers are zero to their last byte, and nothing around them is."""
+    from nexusbvh_amd.native import DeviceBuffer, check, lib
+    fill = np.full(max(grads_bytes, loss_bytes) + 16, 0xA5, dtype=np.uint8)
+    a, b = DeviceBuffer.from_array(fill), DeviceBuffer.from_array(fill)
+    check(lib().nxb_mlp_gradients_from_zero(None, None, None, 0, a.address + skip, grads_bytes, b.address + skip,
+                                            loss_bytes, None), "gradients_from_zero")
+    for buf, n in ((a, grads_bytes), (b, loss_bytes)):
+        got = buf.to_array(np.uint8, len(fill))
+        assert not got[skip:skip + n].any()
+        assert (got[:skip] == 0xA5).all() and (got[skip + n:] == 0xA5).all()
