@@ -115,6 +115,38 @@ __device__ __forceinline__ float safe_inv(float x) { return 1.0f / (fabsf(x) > 1
 
 __device__ __forceinline__ float exp_scale(uint32_t e) { return __uint_as_float(e << 23); }  // 2^(e-127)
 
+// Slab test from the decoded child box, face by face: a node's origin p and
+// scale s on an axis, the ray's origin o and reciprocal direction i.
+struct FaceSlab {
+    float p, s, o, i;
+    // Distances t0, t1 of the faces at ql and qh, the box widened outward. The
+    // grid bounds the child exactly, but two roundings move a decoded face
+    // inward: the builder's difference fl(c - p), off by up to
+    // |c - p| * 2^-24 <= (|c| + |p|) * 2^-24, which can land
+    // exactly on a grid point, and the decode p + q * s, off by
+    // |l| * 2^-24. (|l| + |p|) * 2^-21 covers both with margin.
+    __device__ __forceinline__ void faces(uint32_t ql, uint32_t qh, float& t0, float& t1) const {
+        float l = p + (float)ql * s, h = p + (float)qh * s;
+        l -= (fabsf(l) + fabsf(p)) * 0x1p-21f;
+        h += (fabsf(h) + fabsf(p)) * 0x1p-21f;
+        t0 = (l - o) * i;
+        t1 = (h - o) * i;
+    }
+};
+__device__ __forceinline__ bool slab_hit_faces(const FaceSlab& x, const FaceSlab& y, const FaceSlab& z, uint32_t qlx,
+                                               uint32_t qly, uint32_t qlz, uint32_t qhx, uint32_t qhy, uint32_t qhz,
+                                               float tmin, float best_t) {
+    float tx0, tx1, ty0, ty1, tz0, tz1;
+    x.faces(qlx, qhx, tx0, tx1);
+    y.faces(qly, qhy, ty0, ty1);
+    z.faces(qlz, qhz, tz0, tz1);
+    const float tn = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), tmin));
+    // the far distance is widened by 2^-20 against the slab test's
+    // own rounding (Ize, "Robust BVH Ray Traversal", 2013)
+    const float tf = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fmaxf(tz0, tz1)) * (1.0f + 0x1p-20f);
+    return tn <= tf && tn <= best_t;
+}
+
 template <bool INDEXED>
 __global__ __launch_bounds__(kTraceThreads) void k_trace(const nxb_bvh8_node* __restrict__ nodes, uint32_t node_count,
                                                          const uint32_t* __restrict__ prim_idx, uint32_t prim_count,
@@ -164,29 +196,11 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace(const nxb_bvh8_node* __
                 const uint32_t h = s >> 2, sh = (s & 3) * 8;
                 const uint32_t meta = ((s < 4 ? meta_lo : meta_hi) >> sh) & 0xFFu;
                 if (meta == 0) continue;
-                // Decoded child box, widened outward. The grid bounds the
-                // child exactly, but two roundings move a decoded face
-                // inward: the builder's difference fl(c - p), off by up to
-                // |c - p| * 2^-24 <= (|c| + |p|) * 2^-24, which can land
-                // exactly on a grid point, and the decode p + q * s, off by
-                // |l| * 2^-24. (|l| + |p|) * 2^-21 covers both with margin.
-                float lx = px + (float)((qlx[h] >> sh) & 0xFFu) * sx;
-                float ly = py + (float)((qly[h] >> sh) & 0xFFu) * sy;
-                float lz = pz + (float)((qlz[h] >> sh) & 0xFFu) * sz;
-                float hx = px + (float)((qhx[h] >> sh) & 0xFFu) * sx;
-                float hy = py + (float)((qhy[h] >> sh) & 0xFFu) * sy;
-                float hz = pz + (float)((qhz[h] >> sh) & 0xFFu) * sz;
-                const float apx = fabsf(px), apy = fabsf(py), apz = fabsf(pz);
-                lx -= (fabsf(lx) + apx) * 0x1p-21f; ly -= (fabsf(ly) + apy) * 0x1p-21f; lz -= (fabsf(lz) + apz) * 0x1p-21f;
-                hx += (fabsf(hx) + apx) * 0x1p-21f; hy += (fabsf(hy) + apy) * 0x1p-21f; hz += (fabsf(hz) + apz) * 0x1p-21f;
-                const float tx0 = (lx - o.x) * ix, tx1 = (hx - o.x) * ix;
-                const float ty0 = (ly - o.y) * iy, ty1 = (hy - o.y) * iy;
-                const float tz0 = (lz - o.z) * iz, tz1 = (hz - o.z) * iz;
-                const float tn = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), tmin));
-                // the far distance is widened by 2^-20 against the slab test's
-                // own rounding (Ize, "Robust BVH Ray Traversal", 2013)
-                const float tf = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fmaxf(tz0, tz1)) * (1.0f + 0x1p-20f);
-                if (!(tn <= tf && tn <= best_t)) continue;
+                if (!slab_hit_faces(FaceSlab{px, sx, o.x, ix}, FaceSlab{py, sy, o.y, iy}, FaceSlab{pz, sz, o.z, iz},
+                                    (qlx[h] >> sh) & 0xFFu, (qly[h] >> sh) & 0xFFu, (qlz[h] >> sh) & 0xFFu,
+                                    (qhx[h] >> sh) & 0xFFu, (qhy[h] >> sh) & 0xFFu, (qhz[h] >> sh) & 0xFFu, tmin,
+                                    best_t))
+                    continue;
                 if (imask & (1u << s)) {
                     inner_hits |= 1u << s;
                 } else {
@@ -225,21 +239,44 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace(const nxb_bvh8_node* __
 // lies at t = (p - o) * i + q * (s * i) on the ray (i: reciprocal direction),
 // one FMA per face once a node's `near`, `far` and `step` are known; the face
 // that the ray meets first is the low one for i > 0, else the high one.
-// With u = 2^-24, the roundings of p - o, its product with i, s * i, i itself
-// and the FMA move t by at most |i| * u * (4 |p - o| + 3 * 255 s); the
-// builder's rounding of the child face puts it up to (2 |p| + 256 s) * u off
-// the grid point that stands for it. `near` and `far` are moved apart by
-// |i| * 2^-21 * (|p - o| + 2 |p| + 256 s), more than both together and not
-// less than k_trace's widening of the faces. An overflow gives a NaN distance
-// or an infinite margin; minimum and maximum drop the former, so both only
-// keep the child.
+// With u = 2^-24, c = (p - o) * i and step = s * i, the roundings of p - o, c, i,
+// the FMA and `near` or `far` move t by at most u * (5 |c| + 510 |step| + 2 e); the
+// builder's rounding of the child face puts it up to (2 |p| + 256 s) * u off the
+// grid point that stands for it. `near` and `far` are moved apart by
+// e = 2^-21 * (|c| + 256 |step| + 2 |p i|), more than both together and not less
+// than slab_hit_faces' widening of the faces.
+// The low and the high face share c, so its overflow would put both on one side of
+// the ray and lose the child (a zero direction component counts as 1e-30, so c
+// overflows from |p - o| = 3.4e8). e, and so near, is infinite or NaN wherever c or
+// step is: such a node is tested by slab_hit_faces, where each face overflows to its
+// own side. Its exponents come through `again`, so that nothing of that test is
+// computed early and kept in registers (one lane per ray: 77 of them instead of 71).
 struct AxisSlab {
     float near, far, step;
 };
 __device__ __forceinline__ AxisSlab axis_slab(float p, float scale, float o, float i) {
-    const float a = p - o, c = a * i;
-    const float e = (fabsf(a) + (2.0f * fabsf(p) + 256.0f * scale)) * (fabsf(i) * 0x1p-21f);
-    return AxisSlab{c - e, c + e, scale * i};
+    const float c = (p - o) * i, step = scale * i;
+    const float e = __builtin_fmaf(fabsf(c), 0x1p-21f,
+                                   __builtin_fmaf(fabsf(step), 0x1p-13f, fabsf(p) * (fabsf(i) * 0x1p-20f)));
+    return AxisSlab{c - e, c + e, step};
+}
+__device__ __forceinline__ uint32_t again(uint32_t em) {
+    asm("" : "+v"(em));
+    return em;
+}
+__device__ __forceinline__ bool in_range(const AxisSlab& x, const AxisSlab& y, const AxisSlab& z) {
+    return fabsf(x.near) + fabsf(y.near) + fabsf(z.near) < INFINITY;
+}
+// Whether (p - o) * i or s * i can overflow for a node below the root with first
+// words w0: the nodes' origins lie in the root's grid, p to p + 255 s, and their
+// scales are at most 2 s. Asked once per ray: in_range at every node took 3% of the
+// traversal of 2^20 primary rays in 2M triangles (502 us; 517 with it, 506 so).
+__device__ __forceinline__ bool may_overflow(float4 w0, Vec3 o, float ix, float iy, float iz) {
+    const uint32_t em = __float_as_uint(w0.w);
+    const float s = exp_scale(max(max(em & 0xFFu, (em >> 8) & 0xFFu), (em >> 16) & 0xFFu));
+    const float d = fmaxf(fmaxf(fabsf(w0.x - o.x), fabsf(w0.y - o.y)), fabsf(w0.z - o.z));
+    const float i = fmaxf(fmaxf(fabsf(ix), fabsf(iy)), fabsf(iz));
+    return !((d + 512.0f * s) * i * 4.0f < INFINITY);
 }
 __device__ __forceinline__ bool slab_hit(const AxisSlab& x, const AxisSlab& y, const AxisSlab& z, float nx, float ny,
                                          float nz, float fx, float fy, float fz, float tmin, float best_t) {
@@ -299,7 +336,11 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_lane(const nxb_bvh8_nod
         const float4* np = reinterpret_cast<const float4*>(nodes + node);
         w0 = np[0]; w1 = np[1]; w2 = np[2]; w3 = np[3]; w4 = np[4];
     };
-    if (more) load(0);
+    bool overflow = false;
+    if (more) {
+        load(0);
+        overflow = may_overflow(w0, o, ix, iy, iz);
+    }
     while (more) {
         ++visited;
         const uint32_t em = __float_as_uint(w0.w), imask = em >> 24;
@@ -321,6 +362,21 @@ __global__ __launch_bounds__(kTraceThreads) void k_trace_lane(const nxb_bvh8_nod
                 auto at = [&](uint32_t q) { return (float)((q >> sh) & 0xFFu); };
                 if (slab_hit(x, y, z, at(nx), at(ny), at(nz), at(fx), at(fy), at(fz), tmin, best_t))
                     hit |= 1u << (4 * h + k);
+            }
+        }
+        if (overflow && !in_range(x, y, z)) {
+            hit = 0;
+            const uint32_t em2 = again(em);
+#pragma unroll 1
+            for (uint32_t s = 0; s < 8; ++s) {
+                const uint32_t sh = 8 * (s & 3);
+                auto at = [&](float lo, float hi) { return (__float_as_uint(s < 4 ? lo : hi) >> sh) & 0xFFu; };
+                if (slab_hit_faces(FaceSlab{w0.x, exp_scale(em2 & 0xFFu), o.x, ix},
+                                   FaceSlab{w0.y, exp_scale((em2 >> 8) & 0xFFu), o.y, iy},
+                                   FaceSlab{w0.z, exp_scale((em2 >> 16) & 0xFFu), o.z, iz}, at(w2.x, w2.y),
+                                   at(w2.z, w2.w), at(w3.x, w3.y), at(w3.z, w3.w), at(w4.x, w4.y), at(w4.z, w4.w),
+                                   tmin, best_t))
+                    hit |= 1u << s;
             }
         }
         // the next node, which the leaves do not change
@@ -442,14 +498,24 @@ __global__ __launch_bounds__(kGroupThreads) void k_trace_group(const nxb_bvh8_no
     NodeSlot cur = {};
     bool more = node_count != 0, have = more && h == 0;  // the root
     if (have) cur = load_slot(0);
+    const bool overflow = more && may_overflow(*reinterpret_cast<const float4*>(nodes), o, ix, iy, iz);
     while (more) {
         const uint32_t em = __float_as_uint(cur.w0.w), imask = em >> 24;
         const AxisSlab x = axis_slab(cur.w0.x, exp_scale(em & 0xFFu), o.x, ix);
         const AxisSlab y = axis_slab(cur.w0.y, exp_scale((em >> 8) & 0xFFu), o.y, iy);
         const AxisSlab z = axis_slab(cur.w0.z, exp_scale((em >> 16) & 0xFFu), o.z, iz);
-        const bool hit = have && cur.meta != 0 &&
-                         slab_hit(x, y, z, (float)cur.nx, (float)cur.ny, (float)cur.nz, (float)cur.fx, (float)cur.fy,
-                                  (float)cur.fz, tmin, best_t);
+        bool hit = slab_hit(x, y, z, (float)cur.nx, (float)cur.ny, (float)cur.nz, (float)cur.fx, (float)cur.fy,
+                            (float)cur.fz, tmin, best_t);
+        if (overflow && !in_range(x, y, z)) {
+            const uint32_t em2 = again(em);
+            const bool fx = ix < 0.0f, fy = iy < 0.0f, fz = iz < 0.0f;  // the far face is the low one
+            hit = slab_hit_faces(FaceSlab{cur.w0.x, exp_scale(em2 & 0xFFu), o.x, ix},
+                                 FaceSlab{cur.w0.y, exp_scale((em2 >> 8) & 0xFFu), o.y, iy},
+                                 FaceSlab{cur.w0.z, exp_scale((em2 >> 16) & 0xFFu), o.z, iz}, fx ? cur.fx : cur.nx,
+                                 fy ? cur.fy : cur.ny, fz ? cur.fz : cur.nz, fx ? cur.nx : cur.fx,
+                                 fy ? cur.ny : cur.fy, fz ? cur.nz : cur.fz, tmin, best_t);
+        }
+        hit = hit && have && cur.meta != 0;
         const bool inner = (imask >> s) & 1u;
         const uint32_t inner_hits = ray_bits(hit && inner);
         uint32_t prim = NXB_INVALID_IDX;
