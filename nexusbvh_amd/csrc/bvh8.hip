@@ -1005,9 +1005,13 @@ __device__ __forceinline__ bool collapse_children(const uint4* rec, uint32_t n, 
     return true;
 }
 
-// Work items passed on inside a block.
+// Work items passed on inside a block. place: the node's BVH8 id, and its level
+// from bit kLevelBit up. (Each node has its own level: a block's share of the
+// queue comes from blocks that followed their subtrees for any number of levels.)
+constexpr uint32_t kLevelBit = 24, kIdMask = (1u << kLevelBit) - 1u;
+static_assert(kSmallPrims <= 1u << kLevelBit && kMaxLevels < 1u << (32 - kLevelBit), "an id and a level in one word");
 struct BlockQueue {
-    uint32_t x[kBvh8Threads], base[kBvh8Threads], id[kBvh8Threads];
+    uint32_t x[kBvh8Threads], base[kBvh8Threads], place[kBvh8Threads];
 };
 
 // Where a level's children go: ids[0..] in the order of the nodes' slots, to
@@ -1015,21 +1019,22 @@ struct BlockQueue {
 struct ChildSink {
     BlockQueue* bq;
     bool keep;
-    uint32_t ids, queue, level;  // level: of the children
+    uint32_t ids, queue;
     uint64_t *work, *work2;
     uint32_t capacity, n;
 
-    __device__ __forceinline__ bool put(uint32_t at, uint32_t x, uint32_t base, uint32_t prims) const {
+    __device__ __forceinline__ bool put(uint32_t at, uint32_t level, uint32_t x, uint32_t base,
+                                        uint32_t prims) const {
         const uint32_t cid = ids + at;
         bool good = cid < capacity && prims >= 2 && base + prims <= n;
         const uint32_t cx = good ? x : kInvalid;  // an invalid item is flagged, not followed
         if (keep) {
             bq->x[at] = cx;
             bq->base[at] = base;
-            bq->id[at] = cid;
+            bq->place[at] = (level << kLevelBit) | (cid & kIdMask);
         } else if (queue + at < capacity) {
             work[queue + at] = ((uint64_t)base << 32) | cx;
-            work2[queue + at] = ((uint64_t)level << 32) | cid;
+            work2[queue + at] = (level << kLevelBit) | (cid & kIdMask);
         } else {
             good = false;
         }
@@ -1136,8 +1141,8 @@ __device__ __forceinline__ uint32_t levels_to_follow(uint32_t m) {
 // inner children with one atomic add on the node counter alloc (the nodes below
 // the root, node 0; zero before launch 0) and passes the children on to itself,
 // through LDS, while they fit its lanes, else to the next launch through a queue
-// in global memory: work[q] = (first primitive << 32 | BVH2 id), work2[q] =
-// (level << 32 | BVH8 id) of queue position q. Launch l takes the positions
+// in global memory: work[q] = (first primitive << 32 | BVH2 id), work2[q] = the
+// place word of queue position q. Launch l takes the positions
 // [cnt[1] + ... + cnt[l-1], +cnt[l]), counts that earlier launches completed, so
 // no lane ever waits on another (no polling, no spin limit); launch 0 is the
 // root.
@@ -1155,7 +1160,7 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_place(Expanded ex, uint32
     constexpr uint32_t kPlaceNodes = kBvh8Threads / 8, kPlacePasses = 8, kPlaceShare = 4;
     __shared__ BlockQueue bq[2];
     __shared__ uint32_t scan_tmp[2][kBvh8Threads / 64];
-    __shared__ uint32_t sids, squeue, slevel;
+    __shared__ uint32_t sids, squeue;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6, s = tid & 7u, g = tid >> 3;
     const uint32_t m = launch == 0 ? 1u : min(cnt[launch], capacity);
     if (m == 0) return;
@@ -1167,29 +1172,24 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_place(Expanded ex, uint32
     if (launch != 0 && (launch == 1 || m >= cnt[launch - 1])) left = levels_to_follow(m);
     const uint32_t per = follow ? max((m + gridDim.x - 1) / gridDim.x, kPlaceShare) : (uint32_t)kBvh8Threads;
     for (uint32_t i0 = blockIdx.x * per; i0 < m; i0 += gridDim.x * per) {
-        uint32_t nodes = min(per, m - i0), level = 0, cur = 0;
+        uint32_t nodes = min(per, m - i0), cur = 0;
         uint32_t below = 1;  // launch 0, one block: ids given out
         if (launch == 0) {
             if (tid == 0) {  // the root
                 bq[0].x[0] = node_count - 1;
                 bq[0].base[0] = 0;
-                bq[0].id[0] = 0;
+                bq[0].place[0] = 0;
             }
         } else {
-            if (tid == 0) slevel = 0;
-            lds_barrier();
             if (tid < nodes) {
                 const bool has = lo + i0 + tid < capacity;
                 const uint64_t v = has ? work[lo + i0 + tid] : (uint64_t)kInvalid;
-                const uint64_t v2 = has ? work2[lo + i0 + tid] : 0ull;
                 bq[0].x[tid] = (uint32_t)v;
                 bq[0].base[tid] = (uint32_t)(v >> 32);
-                bq[0].id[tid] = (uint32_t)v2;
-                atomicMax(&slevel, (uint32_t)(v2 >> 32));
+                bq[0].place[tid] = has ? (uint32_t)work2[lo + i0 + tid] : 0u;
             }
         }
         lds_barrier();
-        if (launch != 0) level = slevel;  // the deepest of the share: a bound for its levels
         for (;;) {
             // what each lane places: slot s of the node of its eight in pass p
             uint32_t kid[kPlacePasses], prims[kPlacePasses], img[kPlacePasses][3], ic = 0;
@@ -1200,8 +1200,9 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_place(Expanded ex, uint32
                 img[p][0] = img[p][1] = img[p][2] = 0;
                 const uint32_t j = p * kPlaceNodes + g;
                 if (p * kPlaceNodes < nodes && j < nodes) {
-                    const uint32_t x = bq[cur].x[j];
-                    if (x >= n && x < node_count && bq[cur].id[j] < capacity && level < kMaxLevels) {
+                    const uint32_t x = bq[cur].x[j], place = bq[cur].place[j];
+                    if (x >= n && x < node_count && (place & kIdMask) < capacity &&
+                        place >> kLevelBit < kMaxLevels) {
                         const uint32_t* k = reinterpret_cast<const uint32_t*>(ex.kids + 4ull * (x - n));
                         const uint32_t* o = reinterpret_cast<const uint32_t*>(ex.node + 5ull * (x - n));
                         prims[p] = k[8 + s];
@@ -1241,13 +1242,14 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_place(Expanded ex, uint32
                 ids = sids;
                 queue = squeue;
             }
-            const ChildSink sink{&bq[cur ^ 1], keep, ids, queue, level + 1, work, work2, capacity, n};
+            const ChildSink sink{&bq[cur ^ 1], keep, ids, queue, work, work2, capacity, n};
             bool good = true;
 #pragma unroll
             for (uint32_t p = 0; p < kPlacePasses; ++p) {
                 if (p * kPlaceNodes >= nodes) break;
                 const uint32_t j = min(p * kPlaceNodes + g, nodes - 1);
-                const uint32_t x = bq[cur].x[j], base = bq[cur].base[j], id = bq[cur].id[j];
+                const uint32_t x = bq[cur].x[j], base = bq[cur].base[j], place = bq[cur].place[j];
+                const uint32_t id = place & kIdMask, level = place >> kLevelBit;
                 const bool ok = p * kPlaceNodes + g < nodes && x >= n && x < node_count && id < capacity &&
                                 level < kMaxLevels;
                 const bool in = prims[p] != 0, leaf = !in && kid[p] != kInvalid;
@@ -1264,7 +1266,8 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_place(Expanded ex, uint32
                 const uint32_t back4 = lane_back<4>(before);
                 before += s >= 4 ? back4 : 0u;
                 if (in)
-                    good &= sink.put(first + bits_below(im, s), kid[p], base + leaves + before - prims[p], prims[p]);
+                    good &= sink.put(first + bits_below(im, s), level + 1, kid[p], base + leaves + before - prims[p],
+                                     prims[p]);
                 if (leaf) {
                     const uint32_t q = base + bits_below(lm, s);
                     if (q < n) prim_idx[q] = kid[p];
@@ -1285,7 +1288,6 @@ __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_place(Expanded ex, uint32
             if (!keep || total == 0) break;
             lds_barrier();  // the next level's queue is written
             nodes = total;
-            ++level;
             cur ^= 1;
         }
         lds_barrier();  // the queue is read before the next share fills it

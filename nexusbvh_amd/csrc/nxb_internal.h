@@ -64,7 +64,7 @@ struct Bvh8Scratch {
     uint32_t* flags;
     const uint32_t* nsize;    // [n-1] primitives under each internal BVH2 node
     uint64_t* work2;          // [capacity] second word of a work item: (right << 32 | left) children of its BVH2
-                              // node (batches), (level << 32 | BVH8 id) (one mesh)
+                              // node (batches), BVH8 id and level (one mesh)
     uint32_t slot_mode;       // nxb_slot_assignment of the child slots
     const uint4* rec8 = nullptr;  // wide records of the internal nodes (one mesh)
     // bvh8_small(n): [n-1] children (64 bytes) and nodes (80 bytes) of all
