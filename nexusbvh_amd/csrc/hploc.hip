@@ -861,13 +861,16 @@ __global__ __launch_bounds__(kHplocThreads) __attribute__((amdgpu_waves_per_eu(6
 // One resident block per slot of the chip (persistent waves): at most
 // kHplocBlocksPerCu per CU and no more than the kernel's occupancy allows (a
 // block that is not resident would start its fixed positions late), fewer
-// when the input gives a wave less than 64 positions.
-template <typename Kernel>
-static uint32_t hploc_grid(Kernel kernel, uint32_t n, uint32_t blocks_per_cu) {
-    static int per_cu = 0;  // per kernel; the same on every gfx950 device
-    if (per_cu < 1 &&
-        (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kHplocThreads, 0) != hipSuccess || per_cu < 1))
-        per_cu = 1;
+// when the input gives a wave less than 64 positions. The kernel is a template
+// argument, so that each has its own occupancy here: kernels of one signature share
+// a type.
+template <auto KERNEL>
+static uint32_t hploc_grid(uint32_t n, uint32_t blocks_per_cu) {
+    static const int per_cu = [] {  // the same on every gfx950 device
+        int blocks = 0;
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, KERNEL, kHplocThreads, 0);
+        return e == hipSuccess && blocks > 0 ? blocks : 1;
+    }();
     const uint32_t want = blocks_per_cu ? min(blocks_per_cu, kHplocBlocksPerCu) : kHplocBlocksPerCu;
     const uint32_t resident = device_cu_count() * min((uint32_t)per_cu, want);
     const uint32_t most = (n + kHplocThreads - 1) / kHplocThreads;
@@ -893,8 +896,8 @@ template <typename K, int GW, bool BATCH, HplocKeep KEEP>
 static hipError_t launch_hploc_kernel(const K* keys, uint32_t* cluster, uint32_t n, const uint32_t* mesh_lo,
                                       uint32_t meshes, const NodeStore& ns, RadiusParams rp, uint32_t blocks_per_cu,
                                       HplocScratch sc, hipStream_t s) {
-    auto kernel = k_hploc<K, GW, BATCH, KEEP>;
-    const uint32_t grid = hploc_grid(kernel, n, blocks_per_cu);
+    const auto kernel = k_hploc<K, GW, BATCH, KEEP>;
+    const uint32_t grid = hploc_grid<k_hploc<K, GW, BATCH, KEEP>>(n, blocks_per_cu);
     const HplocChunks cp = hploc_chunks(n, grid);
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(kHplocThreads), 0, s, keys, cluster, sc.recs, sc.csizes, sc.parent,
                        ns, mesh_lo, meshes, rp, sc.flags, sc.next_chunk, cp.first, cp.chunk);
