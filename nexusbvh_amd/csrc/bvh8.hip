@@ -323,8 +323,7 @@ __device__ __forceinline__ void load_rec8(const uint4* rec, uint32_t i, Box& l, 
 // primIdx as long as its primitive count; the node's own leaves take the
 // front, then each inner child (in slot order) takes a range of its size.
 // Primitive counts of a node's inner children, per output slot (0 for leaf
-// and free slots). The level kernel loads them before the block allocates
-// the child ids, so that their latency overlaps that allocation.
+// and free slots).
 __device__ __forceinline__ void load_child_sizes(const Collapsed& c, const uint32_t* nsize, uint32_t n,
                                                  uint32_t node_count, uint32_t sz[8]) {
 #pragma unroll
@@ -944,9 +943,13 @@ __global__ __launch_bounds__(kBvh8Threads, SLOT == NXB_SLOT_AUCTION ? 3 : 4) voi
 // Primitives up to which a build takes this path, above a launch per level: all
 // internal BVH2 nodes are about five times those that the BVH8 needs, but at
 // once. Collapse stage in us, on a surface, blobs and slivers, this / levels:
-// 32/125, 28/97, 28/97 at 2,003; 53/169, 51/163, 47/144 at 48K; 96/177, 109/205,
-// 102/175 at 300K; 186/210, 211/236, 185/203 at 900K; 213/216, 245/253, 215/224
-// at 1.1M; 347/259, 389/297, 353/267 at 2M.
+// 31/115, 29/95, 28/87 at 2,003; 51/158, 47/153, 46/145 at 48K; 93/165, 105/193,
+// 94/168 at 300K; 178/200, 196/223, 180/200 at 900K; 211/214, 225/239, 195/203
+// at 2^20; 206/205, 240/251, 205/205 at 1.1M; 238/208, 265/258, 246/217 at 1.3M;
+// 337/247, 365/286, 343/252 at 2M: the line lies just below where they meet.
+// With auction slots 108/505, 153/571, 114/420
+// at 2,003; 269/1119, 264/1218, 202/850 at 300K; 616/1314, 600/1424, 455/883 at
+// 2^20; 632/1315, 612/1488, 469/908 at 1.1M; 995/1319, 979/1498, 792/947 at 2M.
 constexpr uint32_t kSmallPrims = 1u << 20;
 bool bvh8_small(uint32_t n) { return n <= kSmallPrims; }
 
@@ -1149,7 +1152,7 @@ __device__ __forceinline__ uint32_t levels_to_follow(uint32_t m) {
 //
 // Eight lanes take a node, one its slot: a block's pass places 32 nodes, and a
 // node's words go out in three coalesced stores. (One lane per node: 38 us at
-// 2,003 primitives and 105 at 300K for both kernels, now 31 and 96.) At least
+// 2,003 primitives and 105 at 300K for both kernels, now 31 and 93.) At least
 // kPlaceShare nodes per block: each block and level costs two atomic adds on the
 // same two counters (10 ns each).
 __global__ __launch_bounds__(kBvh8Threads) void k_bvh8_place(Expanded ex, uint32_t n, uint32_t node_count,
@@ -1784,9 +1787,9 @@ hipError_t launch_bvh8_collapse(const nxb_bvh2_node* bvh2, uint32_t n, nxb_bvh8_
     return hipGetLastError();
 }
 
-// Forest of `trees` BVH2 trees whose roots the caller put in work[0..trees).
-__global__ void k_bvh8_forest_level_init(uint32_t* cnt, uint32_t trees) {
-    for (uint32_t i = threadIdx.x; i <= kMaxLevels; i += blockDim.x) cnt[i] = i == 0 ? trees : 0u;
+// Level counters of a forest: k_bvh8_tree_top counts the first level of the queue.
+__global__ void k_bvh8_forest_level_init(uint32_t* cnt) {
+    for (uint32_t i = threadIdx.x; i <= kMaxLevels; i += blockDim.x) cnt[i] = 0u;
 }
 
 // Node total into the low word of *ctr; a non-empty level past the last one
@@ -1808,7 +1811,7 @@ hipError_t launch_bvh8_tree_levels(const nxb_bvh2_node* bvh2, uint32_t n, uint32
         return hipErrorInvalidValue;
     const uint32_t grid = min((capacity + kBvh8Threads - 1) / kBvh8Threads, device_cu_count() * 3u);
     const bool auction = sc.slot_mode == NXB_SLOT_AUCTION;
-    hipLaunchKernelGGL(k_bvh8_forest_level_init, dim3(1), dim3(128), 0, s, cnt, 0u);
+    hipLaunchKernelGGL(k_bvh8_forest_level_init, dim3(1), dim3(128), 0, s, cnt);
     auto top = auction ? k_bvh8_tree_top<NXB_SLOT_AUCTION> : k_bvh8_tree_top<NXB_SLOT_GREEDY>;
     hipLaunchKernelGGL(top, dim3((trees + kTopTrees - 1) / kTopTrees), dim3(kBvh8Threads), 0, s, bvh2, n,
                        2 * n - trees, out, prim_idx, capacity, sc.work2, work3, cnt, info, trees, mesh_lo,

@@ -81,8 +81,9 @@ constexpr uint32_t kInfBits = 0x7F800000u;  // areas at or above it as bits: inf
 constexpr uint32_t kMoved = 0xFFFFFFFDu;  // temporary id of the node that retired n-1
 constexpr uint32_t kRefill = 32;           // free lanes that make a wave start new positions
 // Resident blocks per CU (6 waves per SIMD): at 28.1M primitives a BVH8 build's
-// H-PLOC takes 2.60 ms with 12, 2.84 with 10, 3.04 with 8; 14 (72 registers)
-// took 3.73.
+// H-PLOC (tasks of 32 lanes, staged records, 80 registers) takes 2.60 ms with 12,
+// 2.84 with 10, 3.04 with 8; 14 (72 registers) took 3.73. Tasks of 64 lanes, with
+// 57 to 71 registers, keep the same limit: they were not measured with more.
 constexpr uint32_t kHplocBlocksPerCu = kHplocMaxBlocksPerCu;
 constexpr uint32_t kHplocMaxChunk = 1024;
 // Primitives from which wide records go through the stage: below, its LDS round

@@ -194,7 +194,7 @@ hipError_t launch_mlp_grad(const float* params, const float* feat, const uint8_t
 hipError_t launch_adam(float* params, const float* grads, float* m, float* v, uint32_t step, float lr, float beta1,
                        float beta2, float eps, hipStream_t s);
 
-// Closest-hit traversal of a BVH8 (one lane per ray).
+// Closest-hit traversal of a BVH8.
 // indices (nullable): tris is then vertex_count vertices of three floats and
 // indices three vertex indices per triangle.
 hipError_t launch_trace(const nxb_bvh8_node* nodes, uint32_t node_count, const uint32_t* prim_idx,

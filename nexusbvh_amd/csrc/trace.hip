@@ -14,8 +14,14 @@
 // (likewise y, bit 1, and z, bit 0), so this order is front to back along
 // the ray's octant.
 //
-// Three kernels give the same hits (a hit is the smallest distance, then the
-// smallest triangle index, whatever the order of the tests):
+// Three kernels, of which each takes the smallest distance, then the smallest
+// triangle index, of the triangles it tests. They visit nodes in different orders
+// and skip those that start beyond the best distance so far, so their hits are the
+// same as long as a triangle's computed distance lies within its box's widened
+// interval. Rounding breaks that only for triangles that are lines at their
+// coordinates' precision (6.6M rays into slivers and needles, many of them along a
+// needle: no difference; 3 of 600,000 rays differ from k_trace's where needles 1e-7
+// wide lie at coordinates of 50,000, whose floats are 4e-3 apart):
 //   k_trace_group  eight lanes per node, one per child slot, and up to four
 //                  nodes of a ray at once: few rays, where a ray's chain of
 //                  dependent steps is what takes the time;
@@ -307,8 +313,10 @@ __device__ __forceinline__ uint32_t next_child(uint32_t base, uint32_t& group, u
 // (20 instead of ~60 instructions a child) 2^20 rays against 2M triangles take
 // 543 instead of 949 us (primary, surface) and 1031 instead of 1764 us
 // (incoherent, uniform). The next node does not depend on the leaves, so its
-// loads go out before their tests: 539 -> 501 and 1030 -> 962 us. Bound by
-// instruction issue, then by the node loads of diverging rays.
+// loads go out before their tests: 539 -> 501 and 1030 -> 962 us. Bound by the issue
+// of vector instructions that few of a wave's rays still need: primary rays fill 71%
+// of the issue slots with 27 of 64 lanes active, incoherent ones 99% with 6 (a wave
+// runs until its longest ray ends); of their L2 requests 6 and 49% miss.
 template <bool INDEXED>
 __global__ __launch_bounds__(kTraceThreads) void k_trace_lane(const nxb_bvh8_node* __restrict__ nodes,
                                                               uint32_t node_count,
@@ -437,8 +445,10 @@ __device__ __forceinline__ uint32_t take_child(uint32_t base, uint32_t& group, u
 // leaves' triangles are fetched and tested.
 //
 // Bound by the latency of a ray's steps (some 1.2 us each where nodes come from
-// memory), so the longest walk decides: two nodes a step nearly halve its steps,
-// for the same instructions per node. 16,384 rays took, with one node a step and
+// memory) with few waves to cover it: on the slivers below 57% of the waves' time is
+// waiting, 2.8 waves per SIMD are in flight, 60% of the issue slots are filled, and
+// 84% of the L2 requests miss (3.2 TB/s). Two nodes a step nearly halve the steps of
+// the longest walk, for the same instructions per node. 16,384 rays took, with one node a step and
 // the next node loaded after the leaves' tests; with it loaded before; with two
 // nodes a step (us, rays a tenth of the scene long from near its surface):
 //   2.9M slivers 955, 740, 497    28.1M blobs 493, 408, 310
@@ -611,7 +621,7 @@ __global__ __launch_bounds__(kGroupThreads) void k_trace_group(const nxb_bvh8_no
 //   four nodes against two    0.61-1.07 at 8,192 rays, 0.76-1.08 at 16,384 (but
 //                             up to 1.17 for short rays near a surface)
 //   two against one           0.69-0.98 at 32,768, 0.83-1.20 at 65,536
-//   one against k_trace_lane  0.48-1.12 at 2^17, 0.73-1.51 at 2^18 (its wave's
+//   one against k_trace_lane  0.54-1.12 at 2^17, 0.69-1.50 at 2^18 (its wave's
 //                             instructions per ray are about twice as many)
 constexpr uint32_t kQuadMaxRays = 1u << 13;
 constexpr uint32_t kPairMaxRays = 1u << 15;

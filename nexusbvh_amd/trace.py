@@ -2,8 +2,9 @@
 reference, which builds BVH8s but does not trace them).
 
 `TraceClosest` runs `nxb_trace_closest` (csrc/trace.hip) through the C ABI:
-one GPU lane per ray, Moller-Trumbore in FP32 without contraction, equal
-distances resolved to the smaller triangle index. There is no CPU fallback.
+one GPU lane per ray, or 8 to 32 where there are few, Moller-Trumbore in FP32
+without contraction, equal distances resolved to the smaller triangle index.
+There is no CPU fallback.
 """
 from __future__ import annotations
 
