@@ -446,13 +446,14 @@ __device__ __forceinline__ uint32_t take_child(uint32_t base, uint32_t& group, u
 //
 // Bound by the latency of a ray's steps (some 1.2 us each where nodes come from
 // memory) with few waves to cover it: on the slivers below 57% of the waves' time is
-// waiting, 2.8 waves per SIMD are in flight, 60% of the issue slots are filled, and
-// 84% of the L2 requests miss (3.2 TB/s). Two nodes a step nearly halve the steps of
-// the longest walk, for the same instructions per node. 16,384 rays took, with one node a step and
-// the next node loaded after the leaves' tests; with it loaded before; with two
-// nodes a step (us, rays a tenth of the scene long from near its surface):
-//   2.9M slivers 955, 740, 497    28.1M blobs 493, 408, 310
-//   1.1M surface  87,  75,  56    1.9M blobs  203, 169, 127
+// waiting, 2.8 waves per SIMD are in flight, 59% of the issue slots are filled, and
+// 84% of the L2 requests miss (3.3 TB/s). Two nodes a step nearly halve the steps of
+// the longest walk, for the same instructions per node. 16,384 rays took, with one
+// node a step and the next node loaded after the leaves' tests; with it loaded
+// before; with two nodes a step (us, rays a tenth of the scene long from near its
+// surface):
+//   2.9M slivers 955, 740, 490    28.1M blobs 493, 408, 309
+//   1.1M surface  87,  75,  55    1.9M blobs  203, 169, 123
 // and 4,096 rays in 48K slivers 45, 43 and with four nodes a step 27. Leaf tests
 // spread over the next two steps, so that every load has a step to arrive, took
 // as long or longer (738 and 481 us of the first two).
